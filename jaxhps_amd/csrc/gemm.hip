@@ -31,7 +31,7 @@ hipError_t gemm(const GemmArgs<T>& a, hipStream_t s) {
     if (a.N <= 2) {
       static const std::string nm = std::string("gemv_conjt<") + tname<T>() + ">";
       prof::Scope ps(s, nm.c_str(), flops, bytes);
-      dim3 grid(ceil_div(a.M, 256), gy);
+      dim3 grid(ceil_div(a.M, 256 / (int)sizeof(T)), gy);  // 256 bytes of A's rows per workgroup
       if (a.N <= 1)
         hipLaunchKernelGGL((gemv_conjt_kernel<T, 1>), grid, dim3(256), 0, s, a);
       else
