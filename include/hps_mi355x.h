@@ -146,12 +146,9 @@ int hps_leaf_solve(hps_handle_t h, int dtype, int kind, int nl, int n, int nb, i
  * without row exchanges.  The merge matrices of the uniform tree eliminate
  * stably in their natural order (pivot growth ~1, multipliers below 4 on the
  * Helmholtz and variable-coefficient workloads), while pivoted panels are
- * latency-bound.  With 0, the register panels (up to 1024 rows, 512 for
- * complex128, in levels of more than 16 matrices) check each matrix's
- * largest multiplier and set info = -1 when it exceeds 64 or is not finite;
- * the other panels are not checked, and a caller that turns pivoting off
- * checks those factors (largest multiplier, finite, nonzero diagonal) and
- * refactors with pivoting when either check fails.  The reference factors
+ * latency-bound.  With 0, the panel kernels check each matrix and set
+ * info = -1 when a multiplier exceeds 64, a pivot is zero or a value is not
+ * finite; the caller refactors with pivoting then.  The reference factors
  * with LAPACK's pivoted LU inside jnp.linalg.inv
  * (merge/_schur_complement.py:107,146). */
 int hps_set_merge_pivoting(hps_handle_t h, int partial_pivoting);

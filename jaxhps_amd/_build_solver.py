@@ -78,7 +78,7 @@ def _merge_levels(pde_problem, T, h, return_top_T, dtypes=None):
         nc = 8
     levels, multi = _levels(T, h, dom.L, kind, nc, table_fn, keep_B=True, root_T=return_top_T, dtypes=dtypes)
     for r in levels:
-        raise_on_info(r.info, "merge stage")
+        raise_on_info(r.info_host, "merge stage")
     return levels, multi
 
 

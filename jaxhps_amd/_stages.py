@@ -217,13 +217,14 @@ class MergeLevel:
     B: Optional[torch.Tensor]
     tables: MergeTables
     Finv: Optional[torch.Tensor] = None  # block inverses for few-column up-pass solves (hps_block_inverses)
+    info_host: Optional[torch.Tensor] = None  # info on the host (set by merge._levels)
 
 
 def merge_level(T_in, h_in, tables: MergeTables, keep_factors=False, want_T=True, pivot=True) -> MergeLevel:
     """One level of 4:1 / 8:1 merges.  T_in (nm*nc, nec, nec), h_in (nm*nc, nec, nsrc) or None.
     keep_factors also keeps B (and D12/D21 for ItI) for the up pass.
-    pivot=False factors the interface matrices without row exchanges (see
-    merge_factors_stable for the check the caller owes)."""
+    pivot=False factors the interface matrices without row exchanges: a matrix
+    that the panel kernels reject has info = -1 and needs pivot=True."""
     lib = load_library()
     hd = _lib.handle()
     dev = T_in.device
@@ -294,7 +295,8 @@ def merge_factors_stable(F_lu, bound=64.0):
     """Device bool: the natural-order (unpivoted) LU factors of a merge level
     are usable -- every entry finite, no zero pivot, every multiplier at most
     `bound` in magnitude (partial pivoting would guarantee 1; the merge
-    matrices of uniform trees give values below 4)."""
+    matrices of uniform trees give values below 4).  The panel kernels report
+    the same through info; this reads factors from anywhere."""
     a = F_lu.abs()
     finite = torch.isfinite(a.amax(dim=(-2, -1)))
     mult = torch.tril(a, -1).amax(dim=(-2, -1))

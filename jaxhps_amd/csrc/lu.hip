@@ -22,10 +22,11 @@
 //   3. trailing update A22 -= L21 U12 with the batched MFMA GEMM.
 // getrs: gather rows by perm; per block X_k = inv(L_kk) X_k, then the MFMA
 //   GEMM update below; backward X_k = inv(U_kk) X_k, GEMM update above.
+#include <limits>
 #include <string>
 #include <utility>
 
-#include "hps_kernels.h"
+#include "gemm_kernels.h"
 #include "hps_prof.h"
 
 namespace hps {
@@ -1133,159 +1134,260 @@ static int rows_panel_max() {
 // Tall panels without pivoting, for matrices whose elimination is stable in
 // the natural order (the merge matrices of the HPS tree: the ItI W = I -
 // D12 D21 and the DtN interface blocks show pivot growth ~1 and multipliers
-// below 4; the caller checks the factors and refactors with pivoting
-// otherwise).  Every workgroup factors the nb x nb diagonal block (one wave,
+// below 4).  Every workgroup factors the nb x nb diagonal block (one wave,
 // rows in registers; redundant work costs less than a second launch) and
-// inverts its U11; its NOPIV_ROWS panel rows below the block then take
-// L21 = A21 inv(U11), four lanes per row, each entry an independent dot product over
-// the row held in the quad's registers.  The last workgroup of the matrix to
-// read the diagonal block (a per-matrix arrival counter) writes the factored
-// block, its packed inverse (dinv) and the identity pivots.  The rows are
-// independent: grid
-// (ceil((n - k - nb) / NOPIV_ROWS), batch).
+// inverts it; its NOPIV_ROWS panel rows below the block then take L21 = A21
+// inv(U11), a workgroup of the block row its 32 columns of U12 = inv(L11)
+// A12, both as MFMA products whose operands were requested before the
+// elimination.  The last workgroup of the matrix to read the diagonal block
+// (a per-matrix arrival counter) writes the factored block, its packed inverse
+// (dinv) and the identity pivots.  The rows are independent: grid
+// (ceil((n - k - nb) / NOPIV_ROWS) + U12 chunks, batch).
+//
+// A matrix with a multiplier above LU_NOPIV_BOUND, a zero pivot or a value
+// that is not finite gets info = -1 (the caller refactors with pivoting).
+//
+// Bound by the serial chain of 32 steps (publish, barrier, read, reciprocal,
+// update: about 0.4 us each in float64).  One wave with its rows in registers
+// and every step unrolled had no barriers, but 110 KB of straight-line code
+// (complex128), fetched once per launch: 52 / 24 / 28 us a panel of complex128 /
+// float64 / complex64 (p = 16, L = 7 and p = 10, L = 3 trees); this sweep, which
+// also leaves no separate inversion and no check of the factors afterwards, 24 / 17 / 19 us.
 // ---------------------------------------------------------------------------
-// lane `lane`'s value of v in every lane of the wave (all lanes active)
-__device__ __forceinline__ float lane_read(float v, int lane) { return __shfl(v, lane, 64); }
-__device__ __forceinline__ double lane_read(double v, int lane) { return __shfl(v, lane, 64); }
-__device__ __forceinline__ c64 lane_read(c64 v, int lane) { return c64{lane_read(v.re, lane), lane_read(v.im, lane)}; }
-__device__ __forceinline__ c128 lane_read(c128 v, int lane) {
-  return c128{lane_read(v.re, lane), lane_read(v.im, lane)};
+// 1 / a from the hardware's reciprocal estimate and Newton steps (to the last
+// bit or the one before; zero, infinite and subnormal a give no usable value,
+// which the panel's check reports).  Complex a is first scaled by the power of
+// two that brings its larger part to [0.5, 1), so |a|^2 neither overflows nor
+// vanishes.  The reciprocal is on the panel's serial chain: half of a division.
+__device__ __forceinline__ double s_inv_fast(double a) {
+  double r = __builtin_amdgcn_rcp(a);
+  r = fma(fma(-a, r, 1.0), r, r);
+  return fma(fma(-a, r, 1.0), r, r);
 }
+__device__ __forceinline__ float s_inv_fast(float a) {
+  const float r = __builtin_amdgcn_rcpf(a);
+  return fmaf(fmaf(-a, r, 1.0f), r, r);
+}
+__device__ __forceinline__ c128 s_inv_fast(c128 a) {
+  const int e = __builtin_amdgcn_frexp_exp(fmax(fabs(a.re), fabs(a.im)));
+  const double re = ldexp(a.re, -e), im = ldexp(a.im, -e);
+  const double d = s_inv_fast(fma(re, re, im * im));
+  return c128{ldexp(re * d, -e), ldexp(-im * d, -e)};
+}
+__device__ __forceinline__ c64 s_inv_fast(c64 a) {
+  const int e = __builtin_amdgcn_frexp_expf(fmaxf(fabsf(a.re), fabsf(a.im)));
+  const float re = ldexpf(a.re, -e), im = ldexpf(a.im, -e);
+  const float d = s_inv_fast(fmaf(re, re, im * im));
+  return c64{ldexpf(re * d, -e), ldexpf(-im * d, -e)};
+}
+
+// c ? a : b by value (a conditional of two array elements is their address,
+// which keeps the arrays in scratch memory)
+__device__ __forceinline__ double s_sel(bool c, double a, double b) { return c ? a : b; }
+__device__ __forceinline__ float s_sel(bool c, float a, float b) { return c ? a : b; }
+__device__ __forceinline__ c128 s_sel(bool c, c128 a, c128 b) { return c128{c ? a.re : b.re, c ? a.im : b.im}; }
+__device__ __forceinline__ c64 s_sel(bool c, c64 a, c64 b) { return c64{c ? a.re : b.re, c ? a.im : b.im}; }
+
+// sum over aligned groups of eight lanes (quad exchanges, then the mirror image within eight)
+__device__ __forceinline__ double oct_sum(double v) {
+  v = quad_sum(v);
+  return v + dpp_move<0x141, 0xf>(0.0, v);
+}
+__device__ __forceinline__ float oct_sum(float v) {
+  v = quad_sum(v);
+  return v + dpp_move<0x141, 0xf>(0.0f, v);
+}
+__device__ __forceinline__ c128 oct_sum(c128 v) { return c128{oct_sum(v.re), oct_sum(v.im)}; }
+__device__ __forceinline__ c64 oct_sum(c64 v) { return c64{oct_sum(v.re), oct_sum(v.im)}; }
+
+__device__ __forceinline__ double s_mod2(double a) { return a * a; }
+__device__ __forceinline__ float s_mod2(float a) { return a * a; }
+__device__ __forceinline__ double s_mod2(c128 a) { return fma(a.re, a.re, a.im * a.im); }
+__device__ __forceinline__ float s_mod2(c64 a) { return fmaf(a.re, a.re, a.im * a.im); }
 
 constexpr int NOPIV_ROWS = 64;  // panel rows per workgroup of the unpivoted panel
 
-// the value of lane CTRL & 3 of each quad (CTRL = 0x55 * lane: quad_perm [l,l,l,l])
-template <int CTRL>
-__device__ __forceinline__ float quad_bcast(float v) { return dpp_move<CTRL, 0xf>(0.0f, v); }
-template <int CTRL>
-__device__ __forceinline__ double quad_bcast(double v) { return dpp_move<CTRL, 0xf>(0.0, v); }
-template <int CTRL>
-__device__ __forceinline__ c64 quad_bcast(c64 v) { return c64{quad_bcast<CTRL>(v.re), quad_bcast<CTRL>(v.im)}; }
-template <int CTRL>
-__device__ __forceinline__ c128 quad_bcast(c128 v) { return c128{quad_bcast<CTRL>(v.re), quad_bcast<CTRL>(v.im)}; }
-
-// x[j] += sum_t a_S[t] W[8 S + t][8 sub + j], a_S = lane S's entries of the quad's row
-template <int S, typename T>
-__device__ __forceinline__ void nopiv_rows_accum(const T (&a)[8], T (&x)[8], const T (*W)[LU_NB + 1], int sub) {
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const T ai = quad_bcast<S * 0x55>(a[t]);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = s_fma(ai, W[8 * S + t][8 * sub + j], x[j]);
+// acc += A B for one 16 x 16 x 4 step of T's MFMA (complex: four real products)
+template <typename T>
+__device__ __forceinline__ void mma_step(T a, T b, typename Mfma<typename real_of<T>::type>::acc_t& re,
+                                         typename Mfma<typename real_of<T>::type>::acc_t& im) {
+  using M = Mfma<typename real_of<T>::type>;
+  re = M::mma(s_re(a), s_re(b), re);
+  if constexpr (is_cplx<T>::value) {
+    re = M::mma(-s_im(a), s_im(b), re);
+    im = M::mma(s_re(a), s_im(b), im);
+    im = M::mma(s_im(a), s_re(b), im);
   }
 }
 
 template <typename T>
 __global__ __launch_bounds__(256) void getrf_panel_nopiv_kernel(int n, T* A, long lda, long sA, int k, int nb,
-                                                                int* ipiv, T* dinv, int* arrivals, int row_wgs,
-                                                                int u12_end) {
+                                                                int* ipiv, T* dinv, int* arrivals, int* info,
+                                                                int row_wgs, int u12_end) {
+  using R = typename real_of<T>::type;
+  using M = Mfma<R>;
+  using acc_t = typename M::acc_t;
+  constexpr R BOUND2 = R(LU_NOPIV_BOUND * LU_NOPIV_BOUND);
   __shared__ T D[LU_NB][LU_NB + 1];
-  __shared__ T W[LU_NB][LU_NB + 1];  // inv(U11)
   __shared__ T P[LU_NB][LU_NB + 1];  // packed inverse
+  __shared__ T prow[2][LU_NB], pcol[2][LU_NB];
   __shared__ int last;
   const int b = blockIdx.y;
   const int tid = threadIdx.x;
+  const int wave = tid >> 6, li = tid & 15, lk = (tid & 63) >> 4;
   T* Ab = A + (long)b * sA;
-  for (int idx = tid; idx < LU_NB * LU_NB; idx += 256) {
-    const int r = idx / LU_NB, c = idx - r * LU_NB;
-    D[r][c] = (r < nb && c < nb) ? Ab[(long)(k + r) * lda + k + c] : (r == c ? s_one<T>() : s_zero<T>());
+  // every load is issued before the first is waited for: the diagonal block's
+  // four entries of this thread, then its operand of the final product -- the
+  // rows of A21 as the MFMA's left operand (wave w: rows 16 w .. 16 w + 15),
+  // or a 32 x 32 chunk of A12 as its right one (waves 2 x 2, 16 columns each).
+  // Entries outside read the block's first one and become zero.
+  T* Akk = Ab + (long)k * lda + k;
+  T dv[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = (tid >> 5) + 8 * i, c = tid & 31;
+    dv[i] = Akk[r < nb && c < nb ? (long)r * lda + c : 0];
+  }
+  const bool is_u12 = (int)blockIdx.x >= row_wgs;
+  const int m0 = k + nb + (int)blockIdx.x * NOPIV_ROWS + 16 * wave;
+  const int c0 = k + nb + ((int)blockIdx.x - row_wgs) * LU_NB + 16 * (wave & 1);
+  const bool edge = is_u12 ? c0 + li < u12_end : m0 + li < n;
+  const long first = is_u12 ? (long)lk * lda + (c0 - k + li) : (long)(m0 - k + li) * lda + lk;
+  const long step = is_u12 ? 4 * lda : 4;
+  T op[LU_NB / 4];
+#pragma unroll
+  for (int q = 0; q < LU_NB / 4; ++q) {
+    const int kk = 4 * q + lk;
+    const bool in = kk < nb && edge;
+    op[q] = Akk[in ? first + q * step : 0];
+    op[q] = s_sel(in, op[q], s_zero<T>());
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = (tid >> 5) + 8 * i, c = tid & 31;
+    D[r][c] = s_sel(r < nb && c < nb, dv[i], s_sel(r == c, s_one<T>(), s_zero<T>()));
   }
   __syncthreads();
   // every workgroup of the matrix has read the original block once the
   // counter reaches gridDim.x: only the last to arrive may overwrite it with
-  // the factors (workgroups of one matrix need not be resident together)
+  // the factors (workgroups of one matrix need not be resident together).  The
+  // answer is needed after the elimination only.
+  // (The offset is hidden from the compiler, which would otherwise combine the
+  // wave's atomics and wait for the result here.)
+  int arrived = 0, zero = 0;
+  asm volatile("" : "+v"(zero));
+  if (tid == 0) arrived = atomicAdd(&arrivals[b + zero], 1);
+  bool ok = true;
+  // One sweep gives the factors and both inverses.  Thread t keeps row t / 8,
+  // columns t % 8 + 8 i of three blocks in registers: x (the block, in the end
+  // its LU), z (inv(L11): the row operations applied to the identity) and y
+  // (inv(U11), one column a step: column j is -inv(U11)[:, <j] u_j / u_jj).
+  // Step j publishes row j (x right of the diagonal, z left of it) and column
+  // j, two buffers and one barrier a step.  The step's column group (j / 8) is
+  // unrolled, its position in the group is a loop: straight-line code for all
+  // 32 steps is larger than the instruction cache.
+  {
+    const int r = tid >> 3, g = tid & 7;
+    T x[4], y[4], z[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      x[i] = D[r][g + 8 * i];
+      y[i] = z[i] = s_zero<T>();
+    }
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq)
+#pragma unroll 1
+      for (int jr = 0; jr < 8; ++jr) {
+        const int j = 8 * jq + jr, par = jr & 1;
+        if (r == j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) prow[par][g + 8 * i] = s_sel(i > jq || (i == jq && g >= jr), x[i], z[i]);
+        if (g == jr) pcol[par][r] = x[jq];
+        __syncthreads();
+        T pr[4], pc[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pr[i] = prow[par][g + 8 * i];
+#pragma unroll
+        for (int i = 0; i <= jq; ++i) pc[i] = pcol[par][g + 8 * i];
+        const T xr = pcol[par][r];
+        const T piv = prow[par][j];
+        const T inv = s_inv_fast(piv);
+        // the entries of y right of column j - 1 are still zero
+        T s = s_mul(y[0], pc[0]);
+#pragma unroll
+        for (int i = 1; i <= jq; ++i) s = s_fma(y[i], pc[i], s);
+        s = oct_sum(s);
+        const R ap = s_abs1(piv);
+        ok = ok && ap > R(0) && ap <= std::numeric_limits<R>::max();
+        if (r > j) {
+          const T l = s_mul(xr, inv);
+          ok = ok && s_mod2(l) <= BOUND2;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (i < jq) z[i] = s_fnms(z[i], l, pr[i]);
+            if (i > jq) x[i] = s_fnms(x[i], l, pr[i]);
+          }
+          const T u = s_fnms(s_sel(g > jr, x[jq], z[jq]), l, pr[jq]);
+          x[jq] = s_sel(g > jr, u, s_sel(g == jr, l, x[jq]));
+          z[jq] = s_sel(g < jr, u, s_sel(g == jr, s_neg(l), z[jq]));
+        }
+        y[jq] = s_sel(g == jr && r <= j, s_sel(r == j, inv, s_neg(s_mul(s, inv))), y[jq]);
+      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = g + 8 * i;
+      const bool in = r < nb && c < nb;
+      D[r][c] = in ? x[i] : s_zero<T>();
+      P[r][c] = in ? (c < r ? z[i] : y[i]) : s_zero<T>();
+    }
+  }
   if (tid == 0) {
-    const int before = atomicAdd(&arrivals[b], 1);
-    last = before == (int)gridDim.x - 1;
+    last = arrived == (int)gridDim.x - 1;
     if (last) atomicExch(&arrivals[b], 0);  // every workgroup has arrived: ready for the next launch
   }
   __syncthreads();
-  // elimination of the diagonal block by wave 0 alone, no barriers: lane r
-  // holds row r in registers; step j reads the pivot row from lane j
-  // (cross-lane shuffles) and the rows below subtract their multiple of it.
-  // The factored block (multipliers below the diagonal) goes back to D, zero
-  // outside nb x nb for the inversion.
-  if (tid < 64) {
-    const int r = tid;
-    T x[LU_NB];
+  acc_t re[2], im[2];
 #pragma unroll
-    for (int c = 0; c < LU_NB; ++c) x[c] = r < LU_NB ? D[r][c] : s_zero<T>();
+  for (int t = 0; t < 2; ++t) re[t] = im[t] = acc_t{0, 0, 0, 0};
+  if (is_u12) {
+    // U12 = inv(L11) A12: the unit-lower part of P on the left, rows 16 t + li
+    const int t = wave >> 1;
 #pragma unroll
-    for (int j = 0; j < LU_NB - 1; ++j) {
-      // rows at or above j (and the idle lanes) take a zero multiplier, so the
-      // step runs without divergence and lane j's row stays as it is; the
-      // shuffles stay outside any branch (lane j must take part for its value
-      // to be read)
-      const bool below = r > j && r < LU_NB;
-      const T inv = s_inv(lane_read(x[j], j));
-      const T l = below ? s_mul(x[j], inv) : s_zero<T>();
-      x[j] = below ? l : x[j];
-#pragma unroll
-      for (int c = j + 1; c < LU_NB; ++c) x[c] = s_fnms(x[c], l, lane_read(x[c], j));
+    for (int q = 0; q < LU_NB / 4; ++q) {
+      const int r = 16 * t + li, kk = 4 * q + lk;
+      const T a = kk < r ? P[r][kk] : (kk == r ? s_one<T>() : s_zero<T>());
+      mma_step<T>(a, op[q], re[0], im[0]);
     }
-    if (r < LU_NB) {
 #pragma unroll
-      for (int c = 0; c < LU_NB; ++c) D[r][c] = (r < nb && c < nb) ? x[c] : s_zero<T>();
-    }
-  }
-  __syncthreads();
-  invert_diag_block<T>(&D[0][0], LU_NB + 1, &P[0][0], LU_NB + 1, nb);
-  __syncthreads();
-  for (int idx = tid; idx < LU_NB * LU_NB; idx += 256) {
-    const int r = idx / LU_NB, c = idx - r * LU_NB;
-    W[r][c] = (r <= c && c < nb) ? P[r][c] : s_zero<T>();  // P holds garbage beyond nb
-  }
-  __syncthreads();
-  if (blockIdx.x >= row_wgs) {
-    // U12 = inv(L11) A12 for 32 columns of the block row right of the panel
-    // (columns up to u12_end): the chunk staged in W (free here), then each
-    // entry a dot product with the unit-lower inv(L11) held in P
-    const int c0 = k + nb + (int)(blockIdx.x - row_wgs) * LU_NB;
-    const int wc = u12_end - c0 < LU_NB ? u12_end - c0 : LU_NB;
-    for (int idx = tid; idx < LU_NB * LU_NB; idx += 256) {
-      const int r = idx / LU_NB, c = idx - r * LU_NB;
-      W[r][c] = (r < nb && c < wc) ? Ab[(long)(k + r) * lda + c0 + c] : s_zero<T>();
-    }
-    __syncthreads();
-    for (int idx = tid; idx < LU_NB * LU_NB; idx += 256) {
-      const int r = idx / LU_NB, c = idx - r * LU_NB;
-      if (r < nb && c < wc) {
-        T acc = W[r][c];
-        for (int q = 0; q < r; ++q) acc = s_fma(P[r][q], W[q][c], acc);
-        Ab[(long)(k + r) * lda + c0 + c] = acc;
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int r = 16 * t + M::out_row(lk, i);
+      if (r < nb && c0 + li < u12_end)
+        Ab[(long)(k + r) * lda + c0 + li] = make_val<T>(re[0][i], is_cplx<T>::value ? im[0][i] : R(0));
     }
   } else {
-    // panel rows below the block: x = a inv(U11), four lanes per row, each
-    // holding eight consecutive entries of the row; entry i comes from lane
-    // i / 8 of the quad by a DPP broadcast, and each lane forms the row's
-    // outputs 8 sub .. 8 sub + 7
-    const int sub = tid & 3;
-    const int rg = k + nb + blockIdx.x * NOPIV_ROWS + (tid >> 2);
-    // a quad's lanes share their row, so whole quads are live or not and the
-    // broadcasts read live lanes only
-    if (rg < n) {
-      T* rowp = Ab + (long)rg * lda + k + 8 * sub;
-      T a[8], x[8];
+    // L21 = A21 inv(U11): the upper part of P on the right
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        a[j] = 8 * sub + j < nb ? rowp[j] : s_zero<T>();
-        x[j] = s_zero<T>();
-      }
-      nopiv_rows_accum<0>(a, x, W, sub);
-      nopiv_rows_accum<1>(a, x, W, sub);
-      nopiv_rows_accum<2>(a, x, W, sub);
-      nopiv_rows_accum<3>(a, x, W, sub);
-      if (nb == LU_NB) {
+    for (int q = 0; q < LU_NB / 4; ++q) {
+      const int kk = 4 * q + lk;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) rowp[j] = x[j];
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (8 * sub + j < nb) rowp[j] = x[j];
+      for (int t = 0; t < 2; ++t) {
+        const int c = 16 * t + li;
+        mma_step<T>(op[q], kk <= c ? P[kk][c] : s_zero<T>(), re[t], im[t]);
       }
     }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = m0 + M::out_row(lk, i), c = 16 * t + li;
+        if (r < n && c < nb) {
+          const T v = make_val<T>(re[t][i], is_cplx<T>::value ? im[t][i] : R(0));
+          ok = ok && s_mod2(v) <= BOUND2;
+          Ab[(long)r * lda + k + c] = v;
+        }
+      }
   }
+  if (!ok) info[b] = -1;  // every writer writes the same value
   if (!last) return;
   for (int idx = tid; idx < nb * nb; idx += 256) {
     const int rr = idx / nb, c = idx - rr * nb;
@@ -1296,7 +1398,7 @@ __global__ __launch_bounds__(256) void getrf_panel_nopiv_kernel(int n, T* A, lon
   T* db = dinv + ((long)b * nblk + k / LU_NB) * LU_NB * LU_NB;
   for (int idx = tid; idx < LU_NB * LU_NB; idx += 256) {
     const int r = idx / LU_NB, c = idx - r * LU_NB;
-    db[idx] = (r < nb && c < nb) ? P[r][c] : s_zero<T>();
+    db[idx] = P[r][c];
   }
 }
 
@@ -1528,8 +1630,8 @@ hipError_t getrf_ws(int n, T* A, long lda, long sA, int* perm, T* dinv, int* scr
           const int bc = batch - b0 < 65535 ? batch - b0 : 65535;
           hipLaunchKernelGGL((getrf_panel_nopiv_kernel<T>), dim3(row_wgs + u12_wgs, bc), dim3(256), 0, s, n,
                              A + (long)b0 * sA, lda, sA, k, nb, ipiv + (long)b0 * n,
-                             dinv + (long)b0 * ((n + LU_NB - 1) / LU_NB) * LU_NB * LU_NB, arrivals + b0, row_wgs,
-                             bend);
+                             dinv + (long)b0 * ((n + LU_NB - 1) / LU_NB) * LU_NB * LU_NB, arrivals + b0, info + b0,
+                             row_wgs, bend);
         }
         e = hipGetLastError();
         swapped = true;  // nothing to swap

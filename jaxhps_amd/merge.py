@@ -12,7 +12,7 @@ from typing import List
 import torch
 
 from ._lib import raise_on_info
-from ._stages import cast, merge_factors_stable, merge_level
+from ._stages import cast, merge_level
 from ._tables import oct_merge_tables, quad_merge_tables
 
 
@@ -25,9 +25,10 @@ def _levels(T_arr, h_arr, l, kind, nc, table_fn, keep_B=False, root_T=True, dtyp
 
     The interface matrices are factored without row exchanges (pivot=False):
     they eliminate stably in their natural order, and pivoted panels are
-    latency-bound.  Every level is checked at the end (one synchronisation);
-    from the first level that fails the check the merges are redone with
-    partial pivoting.  Low-precision levels of fewer than 128 matrices of more
+    latency-bound.  The panel kernels check themselves (info = -1 on a rejected
+    matrix); every level's info is read at the end in one copy (the only
+    synchronisation), and from the first level that holds a rejected matrix
+    the merges are redone with partial pivoting.  Low-precision levels of fewer than 128 matrices of more
     than 256 unknowns keep the inverses of their factors' diagonal blocks for
     the refinement's few-column up passes (MergeLevel.Finv)."""
     from . import profiling
@@ -58,27 +59,25 @@ def _levels(T_arr, h_arr, l, kind, nc, table_fn, keep_B=False, root_T=True, dtyp
             T, h = res.T, res.h
         return out
 
+    def read_info(levels):
+        infos = torch.cat([r.info for r in levels]).cpu().split([r.info.shape[0] for r in levels])
+        for r, i in zip(levels, infos):
+            r.info_host = i
+
     out = run(0, T0, h0, [], pivot)
+    read_info(out)
     if not pivot:
-        # every level was factored without row exchanges: the register-sized
-        # panels check themselves (info = -1 on a rejected matrix); the tall
-        # panels of the levels with panels taller than the register panels
-        # (1024 rows, 512 for complex128) or of at most 16 matrices are
-        # checked here on the factors
-        tall = lambda r: (r.F_lu.shape[-1] > (512 if r.F_lu.dtype == torch.complex128 else 1024)  # noqa: E731
-                          or r.F_lu.shape[0] <= 16)
-        ok = torch.stack([(r.info >= 0).all() & (merge_factors_stable(r.F_lu) if tall(r) else True)
-                          for r in out]).cpu()
-        if not bool(ok.all()):
-            first = int((~ok).nonzero()[0, 0])
+        first = next((i for i, r in enumerate(out) if bool((r.info_host < 0).any())), None)
+        if first is not None:
             T, h = (T0, h0) if first == 0 else (out[first - 1].T, out[first - 1].h)
             out = run(first, T, h, out[:first], True)
+            read_info(out)
     return out, multi
 
 
 def _pack_outputs(levels, multi, return_T, what):
     for r in levels:
-        raise_on_info(r.info, what)
+        raise_on_info(r.info_host, what)
     S_lst = [r.S for r in levels]
     if multi:
         g_lst = [r.gt for r in levels]

@@ -1,5 +1,5 @@
-"""The conjugate-transposed GEMV at the edges of its tiles, against float64 /
-complex128 numpy."""
+"""The unpivoted panel kernel and the conjugate-transposed GEMV at the edges
+of their tiles, against float64 / complex128 numpy."""
 
 import numpy as np
 import pytest
@@ -9,6 +9,64 @@ pytestmark = pytest.mark.gpu
 
 DTYPES = [torch.float64, torch.float32, torch.complex128, torch.complex64]
 EPS = {torch.float64: 2.0**-53, torch.float32: 2.0**-24, torch.complex128: 2.0**-53, torch.complex64: 2.0**-24}
+
+
+def _children(m, nm, dtype, gpu, seed):
+    ne = 4 * m
+    rng = np.random.default_rng(seed)
+    T = 2.0 * np.eye(ne) + 0.3 * rng.standard_normal((4 * nm, ne, ne)) / np.sqrt(ne)
+    if dtype.is_complex:
+        T = T + 0.3j * rng.standard_normal(T.shape) / np.sqrt(ne)
+    return torch.as_tensor(T, device=gpu).to(dtype).contiguous()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,nm", [(2, 1), (8, 3), (9, 2), (25, 16), (49, 1)])
+def test_unpivoted_panel_factors(gpu, dtype, m, nm):
+    """Interface matrices of 8 .. 196 unknowns (whole and partial 32-column
+    panels, partial row and U12 tiles): L U is the gathered matrix.  The error of
+    an LU without exchanges is n eps |L| |U| entrywise."""
+    from jaxhps_amd._stages import merge_level
+    from jaxhps_amd._tables import quad_merge_tables
+
+    print(f"unpivoted panel {dtype} m={m} nm={nm}", flush=True)
+    T = _children(m, nm, dtype, gpu, m)
+    tb = quad_merge_tables(m, "dtn")
+    out = merge_level(T, None, tb, pivot=False)
+    assert (out.info == 0).all()
+    n = 4 * m
+    Th = T.cpu().numpy().reshape(nm, 4, n, n)
+    D = np.zeros((nm, n, n), dtype=complex)
+    for i, re in enumerate(tb.int_rows):
+        for j, ce in enumerate(tb.int_cols):
+            for a in (0, 2):
+                for b in (0, 2):
+                    if re[a] == ce[b]:
+                        D[:, i, j] += Th[:, re[a], re[a + 1], ce[b + 1]]
+    F = out.F_lu.cpu().numpy().astype(complex)
+    Lo, Up = np.tril(F, -1) + np.eye(n), np.triu(F)
+    bound = 4 * (n + 8) * EPS[dtype] * (np.abs(Lo) @ np.abs(Up))  # 4: complex products
+    assert (np.abs(Lo @ Up - D) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.complex64])
+@pytest.mark.parametrize("row", [0, 31, 32, 99])
+def test_unpivoted_panel_rejects(gpu, dtype, row):
+    """A zero row of the interface matrix (first, last of a panel, last of the
+    matrix), or a NaN, marks its matrix alone with info = -1."""
+    from jaxhps_amd._stages import merge_level
+    from jaxhps_amd._tables import quad_merge_tables
+
+    print(f"unpivoted panel rejects {dtype} row {row}", flush=True)
+    m, nm = 25, 4
+    tb = quad_merge_tables(m, "dtn")
+    c0, l0, c1, l1 = (int(v) for v in tb.int_rows[row])
+    for value in (0.0, float("nan")):
+        T = _children(m, nm, dtype, gpu, row)
+        T[4 * 2 + c0, l0, :] = value
+        T[4 * 2 + c1, l1, :] = value
+        info = merge_level(T, None, tb, pivot=False).info.cpu().numpy()
+        assert info[2] == -1 and (np.delete(info, 2) == 0).all(), info
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
