@@ -114,7 +114,8 @@ int hps_leaf_solve(hps_handle_t h, int dtype, int kind, int nl, int n, int nb, i
  *                     merged node's final order (the reference's roll folded in)
  *   cols_final (ni, 4): int_cols in the final unknown order (B's columns);
  *                     NULL = int_cols
- *   final_of_internal (ni): final row of each internal unknown (ItI only)
+ *   final_of_internal (ni): final row of each internal unknown (NULL for DtN
+ *                     merges whose internal order is the final one)
  * The interface system D g_int = -(C g_ext + h_int), D = gather(rows, cols):
  *   DtN: D is dense; F = LU(D), F (nm, ni, ni).
  *   ItI: unknowns in internal order [F-half; G-half] give
@@ -129,8 +130,7 @@ int hps_leaf_solve(hps_handle_t h, int dtype, int kind, int nl, int n, int nb, i
  *   F_inv_out (nm * hps_block_inverses_elems(n), n = ni (DtN) or ni/2 (ItI))
  *   or NULL: for complex64 / float32 levels of fewer than 128 matrices with
  *   hps_block_inverses_elems(n) > 0, the inverses of F's diagonal blocks (as
- *   hps_block_inverses forms them), which the level's few-column source
- *   solve uses too; otherwise not written.
+ *   hps_block_inverses forms them); otherwise not written.
  * upd (host int[4*n_upd]): the nonzero blocks (r0, nr, k0, nk) of B; the
  *   products B S and B gt use only these (n_upd = 0: B dense).
  * d12_blk / d21_blk (host int[4*n], ItI only): the nonzero rectangles of D12
@@ -152,6 +152,20 @@ int hps_leaf_solve(hps_handle_t h, int dtype, int kind, int nl, int n, int nb, i
  * with LAPACK's pivoted LU inside jnp.linalg.inv
  * (merge/_schur_complement.py:107,146). */
 int hps_set_merge_pivoting(hps_handle_t h, int partial_pivoting);
+/* Structure of the elimination in the following hps_merge_level calls on this
+ * handle (DtN; used when merge pivoting is off).  HPS_DISSECT_QUAD: the four
+ * interfaces of a 2D merge in the order a|b, c|d, b|c, d|a in int_rows and
+ * int_cols.  HPS_DISSECT_OCT: the twelve interfaces of a 3D merge in the order
+ * a|b, c|d, e|f, g|h, d|a, b|c, h|e, f|g, a|e, b|f, d|h, c|g.  Interfaces that do
+ * not touch are eliminated independently and zero blocks are left out.
+ * ext_by_child (device, ne int4 entries like `ext`) lists the exterior nodes
+ * child after child, ext_pos (device, ne) their positions in `ext`; both stay
+ * valid until the next call.  HPS_DISSECT_NONE (the default) eliminates
+ * densely.  The row map final_of_internal then also applies to DtN merges
+ * (NULL: the internal order is the final one), here and in hps_up_level.  The
+ * reference inverts the dense matrix (merge/_schur_complement.py:294-774). */
+enum { HPS_DISSECT_NONE = 0, HPS_DISSECT_QUAD = 1, HPS_DISSECT_OCT = 2 };
+int hps_set_merge_dissection(hps_handle_t h, int dissect, const int* ext_by_child, const int* ext_pos);
 /* Pivoting of hps_leaf_solve's factorisation on this handle: 1 (default) =
  * partial pivoting; 0 = natural order, every panel checked in the kernel:
  * a leaf whose largest multiplier exceeds 64 (or is not finite) gets

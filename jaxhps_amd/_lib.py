@@ -16,6 +16,7 @@ LIB_PATH = Path(__file__).resolve().parent / "libhps_mi355x.so"
 
 HPS_OK = 0
 HPS_F64, HPS_F32, HPS_C128, HPS_C64 = 0, 1, 2, 3
+HPS_DISSECT_NONE, HPS_DISSECT_QUAD, HPS_DISSECT_OCT = 0, 1, 2
 HPS_KIND_DTN, HPS_KIND_ITI = 0, 1
 
 DTYPE_CODE = {
@@ -48,6 +49,7 @@ SIGNATURES = {
         [_P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _S],
     ),
     "hps_set_merge_pivoting": (_I, [_P, _I]),
+    "hps_set_merge_dissection": (_I, [_P, _I, _P, _P]),
     "hps_set_leaf_pivoting": (_I, [_P, _I]),
     "hps_merge_workspace": (_S, [_I, _I, _I, _I, _I, _I]),
     "hps_merge_level": (

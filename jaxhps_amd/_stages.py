@@ -15,7 +15,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import HPS_KIND_DTN, HPS_KIND_ITI, check, dtype_code, load_library, ptr, workspace
+from ._lib import HPS_DISSECT_NONE, HPS_KIND_DTN, HPS_KIND_ITI, check, dtype_code, load_library, ptr, workspace
 from ._tables import MergeTables
 
 
@@ -255,8 +255,15 @@ def merge_level(T_in, h_in, tables: MergeTables, keep_factors=False, want_T=True
     upd = np.ascontiguousarray(tables.upd, dtype=np.int32)
     d12 = np.ascontiguousarray(tables.d12_blk, dtype=np.int32)
     d21 = np.ascontiguousarray(tables.d21_blk, dtype=np.int32)
+    # the tables' elimination order serves natural-order factorisation only
+    dissect = getattr(tables, "dissect", HPS_DISSECT_NONE)
+    if kind == HPS_KIND_DTN and not getattr(tables, "reordered", False):
+        final_of_internal = None  # the internal order is the final one
     if not pivot:
         check(lib.hps_set_merge_pivoting(hd, 0), hd, "hps_set_merge_pivoting")
+        if dissect:
+            by_child, pos = tables.by_child_device(dev)
+            check(lib.hps_set_merge_dissection(hd, dissect, ptr(by_child), ptr(pos)), hd, "hps_set_merge_dissection")
     try:
         rc = _merge_level_call(lib, hd, dt, kind, nm, nc, nec, ni, ne, nsrc, T_in, h_in, rows, cols, ext, cols_final,
                                final_of_internal, upd, d12, d21, S, T, ho, gt, F_lu, perm, dinv, info, D12, D21, B,
@@ -264,6 +271,7 @@ def merge_level(T_in, h_in, tables: MergeTables, keep_factors=False, want_T=True
     finally:
         if not pivot:
             lib.hps_set_merge_pivoting(hd, 1)
+            lib.hps_set_merge_dissection(hd, HPS_DISSECT_NONE, None, None)
     check(rc, hd, "hps_merge_level")
     return MergeLevel(S, T, ho, gt, F_lu, perm, dinv, info, D12, D21, B, tables, Finv)
 
@@ -414,6 +422,8 @@ def up_level(h_in, lvl: MergeLevel, inj=None, want_h=True):
     nm = lvl.F_lu.shape[0]
     nsrc = h_in.shape[-1]
     rows, _, ext, _, _, final_of_internal = tb.device(dev)
+    if kind == HPS_KIND_DTN and not getattr(tb, "reordered", False):
+        final_of_internal = None
     gt = torch.empty((nm, tb.ni, nsrc), dtype=dt, device=dev)
     ho = torch.empty((nm, tb.ne, nsrc), dtype=dt, device=dev) if want_h else None
     ws = workspace(lib.hps_up_workspace(dtype_code(dt), kind, nm, tb.ni, nsrc), dev)

@@ -17,7 +17,9 @@ child and which local boundary index it comes from:
 a=SW, b=SE, c=NE, d=NW; interfaces 5=a|b, 6=b|c, 7=c|d, 8=d|a ordered from
 the outer boundary inwards):
 * DtN unknown/equation order [5, 6, 7, 8]
-  (``merge/_uniform_2D_DtN.py:385-437`` index sets, ``:283-307`` blocks);
+  (``merge/_uniform_2D_DtN.py:385-437`` index sets, ``:283-307`` blocks),
+  eliminated in the order [5, 7, 6, 8] (5 and 7 share no child, so they do
+  not couple);
 * ItI unknown order [a5, b5, b6, c6, c7, d7, d8, a8], the reference's order
   after its row permutation r (``merge/_uniform_2D_ItI.py:357-373``); the
   equation for unknown "x_k" is the outgoing data of its neighbour across
@@ -32,6 +34,8 @@ import functools
 
 import numpy as np
 import torch
+
+from ._lib import HPS_DISSECT_OCT, HPS_DISSECT_QUAD
 
 A_, B_, C_, D_ = 0, 1, 2, 3
 
@@ -66,12 +70,12 @@ class MergeTables:
 
     int_rows/int_cols are in the *internal* unknown order the factorisation
     uses; cols_final is int_cols in the final (stored) order and
-    final_of_internal maps internal -> final rows (identity for DtN).  upd
+    final_of_internal maps internal -> final rows.  upd
     lists the nonzero (r0, nr, k0, nk) blocks of B (exterior x unknowns).
     """
 
     def __init__(self, kind, nc, nec, int_rows, int_cols, ext, child_src, cols_final=None, final_of_internal=None,
-                 block=None):
+                 block=None, dissect=0):
         self.kind = kind
         self.nc = nc
         self.nec = nec
@@ -94,7 +98,18 @@ class MergeTables:
             self.d12_blk = _coupling_blocks(int_rows[:nf], int_cols[nf:], block)
             self.d21_blk = _coupling_blocks(int_rows[nf:], int_cols[:nf], block)
         self.adj_src = _adj_src(nc, nec, int_rows, ext)
+        self.reordered = final_of_internal is not None  # internal and final order differ
+        self.dissect = dissect  # HPS_DISSECT_*: the internal order is that elimination's
         self._dev = {}
+
+    def by_child_device(self, dev):
+        """The exterior nodes child after child, and their final positions."""
+        key = ("by_child", str(dev))
+        if key not in self._dev:
+            order = np.argsort(self.ext[:, 0], kind="stable").astype(np.int32)
+            self._dev[key] = tuple(torch.from_numpy(np.ascontiguousarray(x, dtype=np.int32)).to(dev)
+                                   for x in (self.ext[order], order))
+        return self._dev[key]
 
     def adj_device(self, dev):
         """adj_src on the device (the adjoint up pass's child-slot sources)."""
@@ -188,6 +203,11 @@ def _pack(pairs):
     return out
 
 
+def _block_order(blocks, m):
+    """Final index of each internal unknown when the blocks of m come in the given order."""
+    return (np.array(blocks, dtype=np.int32)[:, None] * m + np.arange(m, dtype=np.int32)).reshape(-1)
+
+
 def _adj_src(nc, nec, int_rows, ext):
     """For the adjoint of the up pass: each child slot feeds either one
     merged exterior node (index >= 0) or one interface equation row r of
@@ -225,12 +245,14 @@ def quad_merge_tables(m: int, kind: str) -> MergeTables:
     ext = _ext_2D(m)
     if kind == "dtn":
         nodes = i5 + i6 + i7 + i8
-        rows = _pack(nodes)
-        cols = rows.copy()
+        cols_final = _pack(nodes)
         unknown_slots = [list(p) for p in nodes]
         ext_arr = _pack([[e] for e in ext])
         src = _child_src(4, nec, ext, unknown_slots)
-        return MergeTables("dtn", 4, nec, rows, cols, ext_arr, src, block=m)
+        fin = _block_order((0, 2, 1, 3), m)
+        rows = cols_final[fin]
+        return MergeTables("dtn", 4, nec, rows, rows.copy(), ext_arr, src, cols_final=cols_final,
+                           final_of_internal=fin, block=m, dissect=HPS_DISSECT_QUAD)
     elif kind == "iti":
         # (child, local) of the unknown and of its partner across the interface
         a5 = [(p[0], p[1]) for p in i5]
@@ -271,6 +293,9 @@ _OCT_IFACES = (
     (4, 1, 5, 0), (5, 3, 6, 2), (6, 0, 7, 1), (7, 2, 4, 3),  # 13 e|f, 14 f|g, 15 g|h, 16 h|e
     (0, 4, 4, 5), (1, 4, 5, 5), (2, 4, 6, 5), (3, 4, 7, 5),  # 17 a|e, 18 b|f, 19 c|g, 20 d|h
 )
+# elimination order: the x-interfaces (a|b, c|d, e|f, g|h: no two share a child),
+# the y-interfaces of the upper, then of the lower slab, the z-interfaces at y-, y+
+_OCT_ORDER = (0, 2, 4, 6, 3, 1, 7, 5, 8, 9, 11, 10)
 # merged face k = the children's face-k blocks in this order (the reference's
 # get_rearrange_indices, :443-541): the quad order of the face's two coordinates
 _OCT_EXT = ((4, 7, 3, 0), (5, 6, 2, 1), (4, 5, 1, 0), (7, 6, 2, 3), (4, 5, 6, 7), (0, 1, 2, 3))
@@ -285,8 +310,11 @@ def oct_merge_tables(n: int) -> MergeTables:
     flips in 3D."""
     nec = 6 * n
     nodes = [((c1, f1 * n + j), (c2, f2 * n + j)) for (c1, f1, c2, f2) in _OCT_IFACES for j in range(n)]
-    rows = _pack(nodes)
+    cols_final = _pack(nodes)
     ext = [(c, k * n + j) for k, kids in enumerate(_OCT_EXT) for c in kids for j in range(n)]
     ext_arr = _pack([[e] for e in ext])
     src = _child_src(8, nec, ext, [list(p) for p in nodes])
-    return MergeTables("dtn", 8, nec, rows, rows.copy(), ext_arr, src, block=n)
+    fin = _block_order(_OCT_ORDER, n)
+    rows = cols_final[fin]
+    return MergeTables("dtn", 8, nec, rows, rows.copy(), ext_arr, src, cols_final=cols_final, final_of_internal=fin,
+                       block=n, dissect=HPS_DISSECT_OCT)

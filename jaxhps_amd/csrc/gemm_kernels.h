@@ -91,8 +91,8 @@ __device__ __forceinline__ void gemm_mfma_tile(const GemmArgs<T>& p, int bx, int
   const int li = lane & 15, lk = lane >> 4;
 
   for (int b = by; b < p.batch; b += gridDim.y) {
-    const T* A = p.A + (long)b * p.sA;
-    const T* B = p.B + (long)b * p.sB;
+    const T* A = p.A + batch_offset(b, p.nin, p.sA, p.sA2);
+    const T* B = p.B + batch_offset(b, p.nin, p.sB, p.sB2);
     static_assert(!K3M || CPLX, "three-product form is for complex types");
     acc_t acc_re[TM][TN], acc_im[TM][TN], acc_x[K3M ? TM : 1][K3M ? TN : 1];
 #pragma unroll
@@ -197,8 +197,8 @@ __device__ __forceinline__ void gemm_mfma_tile(const GemmArgs<T>& p, int bx, int
         }
     }
 
-    const T* C = p.C ? p.C + (long)b * p.sC : nullptr;
-    T* D = p.D + (long)b * p.sD;
+    const T* C = p.C ? p.C + batch_offset(b, p.nin, p.sC, p.sC2) : nullptr;
+    T* D = p.D + batch_offset(b, p.nin, p.sD, p.sD2);
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -283,10 +283,10 @@ __global__ __launch_bounds__(256, 2) void gemm_k32_kernel(GemmArgs<T> p, int til
   const int m0 = tm * BM, n0 = tn * BN;
   const int li = lane & 15, lk = lane >> 4;
   for (int b = by; b < p.batch; b += gridDim.y) {
-    const T* A = p.A + (long)b * p.sA;
-    const T* B = p.B + (long)b * p.sB;
-    const T* C = p.C ? p.C + (long)b * p.sC : nullptr;
-    T* D = p.D + (long)b * p.sD;
+    const T* A = p.A + batch_offset(b, p.nin, p.sA, p.sA2);
+    const T* B = p.B + batch_offset(b, p.nin, p.sB, p.sB2);
+    const T* C = p.C ? p.C + batch_offset(b, p.nin, p.sC, p.sC2) : nullptr;
+    T* D = p.D + batch_offset(b, p.nin, p.sD, p.sD2);
     T ra[LA], rb[LB], rc[TM][TN][4];
 #pragma unroll
     for (int i = 0; i < LA; ++i) {
@@ -408,8 +408,8 @@ __global__ __launch_bounds__(256) void gemv_conjt_kernel(GemmArgs<T> p) {
   const int m = blockIdx.x * CW + c;
   const bool live = m < p.M;
   for (int b = blockIdx.y; b < p.batch; b += gridDim.y) {
-    const T* A = p.A + (long)b * p.sA + (live ? m : 0);
-    const T* B = p.B + (long)b * p.sB;
+    const T* A = p.A + batch_offset(b, p.nin, p.sA, p.sA2) + (live ? m : 0);
+    const T* B = p.B + batch_offset(b, p.nin, p.sB, p.sB2);
     T acc[NMAX];
 #pragma unroll
     for (int n = 0; n < NMAX; ++n) acc[n] = s_zero<T>();
@@ -441,8 +441,8 @@ __global__ __launch_bounds__(256) void gemv_conjt_kernel(GemmArgs<T> p) {
 #pragma unroll
       for (int q = 1; q < SL; ++q) v = s_add(v, part[sl][q][c]);
       v = s_scale(v, p.alpha);
-      if (p.beta != 0.0) v = s_add(v, s_scale(p.C[(long)b * p.sC + (long)m * p.ldc + sl], p.beta));
-      p.D[(long)b * p.sD + (long)m * p.ldd + sl] = v;
+      if (p.beta != 0.0) v = s_add(v, s_scale(p.C[batch_offset(b, p.nin, p.sC, p.sC2) + (long)m * p.ldc + sl], p.beta));
+      p.D[batch_offset(b, p.nin, p.sD, p.sD2) + (long)m * p.ldd + sl] = v;
     }
     __syncthreads();  // part is rewritten for the next matrix
   }
@@ -460,8 +460,8 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(GemmArgs<T> p) {
   const int row = blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
   const bool live = row < p.M;  // every lane takes part in the cross-lane sums
   for (int b = blockIdx.y; b < p.batch; b += gridDim.y) {
-    const T* A = p.A + (long)b * p.sA + (long)(live ? row : 0) * p.lda;
-    const T* B = p.B + (long)b * p.sB;
+    const T* A = p.A + batch_offset(b, p.nin, p.sA, p.sA2) + (long)(live ? row : 0) * p.lda;
+    const T* B = p.B + batch_offset(b, p.nin, p.sB, p.sB2);
     R acc_re[NMAX], acc_im[NMAX];
 #pragma unroll
     for (int n = 0; n < NMAX; ++n) {
@@ -512,8 +512,8 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(GemmArgs<T> p) {
       }
     }
     if (!live) continue;
-    T* D = p.D + (long)b * p.sD + (long)row * p.ldd;
-    const T* C = p.C ? p.C + (long)b * p.sC + (long)row * p.ldc : nullptr;
+    T* D = p.D + batch_offset(b, p.nin, p.sD, p.sD2) + (long)row * p.ldd;
+    const T* C = p.C ? p.C + batch_offset(b, p.nin, p.sC, p.sC2) + (long)row * p.ldc : nullptr;
 #pragma unroll
     for (int n = 0; n < NMAX; ++n) {
       if (n < p.N && sub == n) {

@@ -11,6 +11,7 @@
 // comes from) are computed once on the host per tree level; they encode the
 // reference's block index sets, rolls, flips and row permutation, so one
 // merge code path serves 2D DtN, 2D ItI and 3D DtN.
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -282,6 +283,16 @@ int hps_set_leaf_pivoting(hps_handle_t h, int partial_pivoting) {
   return HPS_OK;
 }
 
+int hps_set_merge_dissection(hps_handle_t h, int dissect, const int* ext_by_child, const int* ext_pos) {
+  if (!h) return HPS_ERR_ARG;
+  HPS_ARG(h, dissect >= HPS_DISSECT_NONE && dissect <= HPS_DISSECT_OCT, "bad dissection");
+  HPS_ARG(h, dissect == HPS_DISSECT_NONE || (ext_by_child && ext_pos), "a dissection needs the columns' order");
+  h->dissect = dissect;
+  h->ext_child = ext_by_child;
+  h->ext_pos = ext_pos;
+  return HPS_OK;
+}
+
 int hps_destroy(hps_handle_t h) {
   delete h;
   return HPS_OK;
@@ -456,7 +467,7 @@ static int leaf_t(hps_handle_t h, int kind, int nl, int n, int nb, int nq, int n
 
   // 3. factor and solve
   T* Afac = kind == HPS_KIND_DTN ? lu + nb : lu;
-  HPS_CHECK_HIP(h, getrf_ws<T>(nrows, Afac, ld_lu, s_lu, perm, dinv, scratch, info, nl, s, false, h->leaf_nopiv));
+  HPS_CHECK_HIP(h, getrf_ws<T>(nrows, Afac, ld_lu, s_lu, perm, dinv, scratch, info, nl, s, h->leaf_nopiv));
   if (kind == HPS_KIND_DTN) {
     HPS_CHECK_HIP(h, getrs_perm<T>(nrows, w, Afac, ld_lu, s_lu, perm, dinv, R, w, (long)nrows * w, X, w,
                                    (long)nrows * w, nl, s));
@@ -556,14 +567,25 @@ int hps_leaf_solve(hps_handle_t h, int dtype, int kind, int nl, int n, int nb, i
 //   Zh  nF x nsrc
 //   D12, D21 nF x nF ItI blocks (when the caller does not keep them)
 //   B   ne x ni      (when the caller does not keep it)
-//   getrf scratch
+//   block inverses and panels of the natural-order LU
+//   block inverses for the caller's up passes, their scratch
+//   integer scratch of either factorisation
 // Low-precision merge levels of fewer than 128 matrices of more than 256
-// unknowns get inverses of their factors' diagonal blocks: the merge's own
-// few-column source solve (1 .. 16 columns) goes through them, and a caller
-// that passes F_inv_out keeps them for its up passes.  The workspace holds
-// them (and the forming and solve scratch) whenever the level qualifies.
+// unknowns form inverses of their factors' diagonal blocks for a caller that
+// passes F_inv_out and keeps them for its up passes.
 static bool merge_block_inverses(int dtype, int nfac, int nm) {
   return (dtype == HPS_F32 || dtype == HPS_C64) && nm < 128 && fewinv_eligible(nfac);
+}
+
+// The elimination's structure of a merge: HPS_DISSECT_* (DtN) or dense.  Below
+// MERGE_DISSECT_MIN unknowns an interface the stages' extra launches cost more
+// than the zeros they leave out: the p = 8, L = 3 Poisson tree (6 .. 24 an
+// interface) took 1.08 ms with stages everywhere, 0.87 ms without.
+constexpr int MERGE_DISSECT_MIN = 48;
+static LuPlan merge_plan(int dissect, int nfac, int ne) {
+  if (dissect == HPS_DISSECT_QUAD && nfac / 4 >= MERGE_DISSECT_MIN) return lu_plan_quad(nfac / 4);
+  if (dissect == HPS_DISSECT_OCT && nfac / 12 >= MERGE_DISSECT_MIN) return lu_plan_oct(nfac / 12);
+  return lu_plan_dense(nfac, ne);
 }
 
 size_t hps_merge_workspace(int dtype, int kind, int nm, int ni, int ne, int nsrc) {
@@ -578,12 +600,17 @@ size_t hps_merge_workspace(int dtype, int kind, int nm, int ni, int ne, int nsrc
   tot += kind == HPS_KIND_ITI ? align_up((size_t)nm * nF * ns * es) : 0;
   tot += kind == HPS_KIND_ITI ? 2 * align_up((size_t)nm * nF * nF * es) : 0;
   tot += align_up((size_t)nm * ne * ni * es);
-  tot += align_up(getrf_scratch_bytes(nfac, nm));
-  if ((dtype == HPS_F32 || dtype == HPS_C64) && nm <= BLOCKINV_MAX_BATCH)
-    tot += align_up(blockinv_workspace_elems(nfac, ne) * es);
-  if (merge_block_inverses(dtype, nfac, nm))
-    tot += align_up(nm * fewinv_elems(nfac) * es) + align_up(fewinv_workspace_elems(nfac, nm) * es) +
-           align_up((size_t)nm * nfac * ns * es);
+  // every structure that the sizes allow (the handle's choice is not known here)
+  size_t inv = 0, tmp = 0, ints = getrf_scratch_bytes(nfac, nm);
+  for (int d = HPS_DISSECT_NONE; d <= HPS_DISSECT_OCT; ++d) {
+    if (d != HPS_DISSECT_NONE && (kind == HPS_KIND_ITI || nfac % (d == HPS_DISSECT_QUAD ? 4 : 12))) continue;
+    const LuPlan p = merge_plan(d, nfac, ne);
+    inv = std::max(inv, lub_inv_elems(p, nm));
+    tmp = std::max(tmp, lub_tmp_elems(p, nm));
+    ints = std::max(ints, lub_scratch_bytes(p, nm));
+  }
+  tot += align_up(inv * es) + align_up(tmp * es) + align_up(ints);
+  if (merge_block_inverses(dtype, nfac, nm)) tot += align_up(fewinv_workspace_elems(nfac, nm) * es);
   return tot;
 }
 
@@ -596,15 +623,30 @@ __global__ void add_identity_kernel(T* A, int n, long sA, int nm) {
   if (i < n && m < nm) A[(long)m * sA + (long)i * n + i] = s_add(A[(long)m * sA + (long)i * n + i], s_one<T>());
 }
 
-// dst[m][map[i]][c] = src[m][i][c]  (row scatter from the internal to the final unknown order)
+// dst[m][map[r]][cmap[c]] = src[m][r][c]: the internal order to the final one
+// (a null map keeps its index); src and dst have matrix strides of their own.
+// Bound by one read and one write; 32-bit division is most of what the index
+// costs.
 template <typename T>
-__global__ void row_scatter_kernel(const T* src, T* dst, const int* map, int rows, int cols, int nm) {
-  long total = (long)rows * cols;
-  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
-    int r = (int)(idx / cols), c = (int)(idx - (long)r * cols);
-    for (int m = blockIdx.y; m < nm; m += gridDim.y)
-      dst[((long)m * rows + map[r]) * cols + c] = src[((long)m * rows + r) * cols + c];
+__global__ __launch_bounds__(256) void scatter_kernel(const T* src, long ss, T* dst, long sd, const int* map,
+                                                      const int* cmap, int rows, int cols, int nm) {
+  const unsigned total = (unsigned)rows * (unsigned)cols;
+  for (unsigned idx = blockIdx.x * 256 + threadIdx.x; idx < total; idx += gridDim.x * 256) {
+    const unsigned r = idx / (unsigned)cols, c = idx - r * (unsigned)cols;
+    const long at = (long)(map ? map[r] : (int)r) * cols + (cmap ? cmap[c] : (int)c);
+    for (int m = blockIdx.y; m < nm; m += gridDim.y) dst[(long)m * sd + at] = src[(long)m * ss + idx];
   }
+}
+
+template <typename T>
+static hipError_t scatter_rows(hipStream_t s, const T* src, long ss, T* dst, long sd, const int* map, const int* cmap,
+                               int rows, int cols, int nm) {
+  if ((long)rows * cols >= (1L << 31)) return hipErrorInvalidValue;  // 32-bit indices in one matrix
+  static const std::string nms = std::string("row_scatter<") + tname<T>() + ">";
+  prof::Scope ps(s, nms.c_str(), 0.0, 2.0 * sizeof(T) * (double)rows * cols * nm);
+  hipLaunchKernelGGL((scatter_kernel<T>), grid_for((long)rows * cols, nm), dim3(256), 0, s, src, ss, dst, sd, map,
+                     cmap, rows, cols, nm);
+  return hipGetLastError();
 }
 
 // dst[m][r][c] = src[m][map[r]][c]
@@ -752,18 +794,16 @@ static int merge_t(hps_handle_t h, int kind, int nm, int nc, int nec, int ni, in
   T* Bw = (T*)take((size_t)nm * ne * ni * es);
   constexpr bool lowp = std::is_same<T, float>::value || std::is_same<T, c64>::value;
   const int nfac = iti ? nF : ni;
-  T* binv = lowp && nm <= BLOCKINV_MAX_BATCH && blockinv_workspace_elems(nfac, ne)
-                ? (T*)take(blockinv_workspace_elems(nfac, ne) * es)
-                : nullptr;
-  // block inverses (see merge_block_inverses): into F_inv_out when the caller
-  // keeps them, else into the workspace when the source solve uses them
-  const bool inv_ok = lowp && nm < 128 && fewinv_eligible(nfac);  // merge_block_inverses for this type
-  T* finv_ws = inv_ok ? (T*)take(nm * fewinv_elems(nfac) * es) : nullptr;
-  T* fws = inv_ok ? (T*)take(fewinv_workspace_elems(nfac, nm) * es) : nullptr;
-  T* fsc = inv_ok ? (T*)take((size_t)nm * nfac * ns * es) : nullptr;
-  const bool few = inv_ok && nsrc >= 1 && nsrc <= 16;  // the source solve goes through them
-  const bool form_inv = inv_ok && (few || F_inv_out);
-  T* finv = F_inv_out && inv_ok ? (T*)F_inv_out : finv_ws;
+  // natural order: by blocks, with the handle's dissection for DtN
+  const bool natural = h->merge_nopiv;
+  const int dissect = !iti ? h->dissect : HPS_DISSECT_NONE;
+  const LuPlan plan = merge_plan(dissect, nfac, ne);
+  const bool by_child = natural && plan.nstage > 1;  // columns of C by child
+  T* linv = natural ? (T*)take(lub_inv_elems(plan, nm) * es) : nullptr;
+  T* ltmp = natural ? (T*)take(lub_tmp_elems(plan, nm) * es) : nullptr;
+  // block inverses for the up passes (see merge_block_inverses)
+  const bool form_inv = lowp && nm < 128 && fewinv_eligible(nfac) && F_inv_out;
+  T* fws = form_inv ? (T*)take(fewinv_workspace_elems(nfac, nm) * es) : nullptr;
   int* scratch = (int*)wp;
   T* Fl = (T*)F_lu;
   T* dinv = (T*)F_dinv;
@@ -784,54 +824,59 @@ static int merge_t(hps_handle_t h, int kind, int nm, int nc, int nec, int ni, in
     hipLaunchKernelGGL((add_identity_kernel<T>), dim3(ceil_div(nF, 256), nm), dim3(256), 0, s, Fl, nF, sNF2, nm);
     HPS_CHECK_HIP(h, hipGetLastError());
   }
-  HPS_CHECK_HIP(h, getrf_ws<T>(nF, Fl, nF, sNF2, perm, dinv, scratch, info, nm, s, h->merge_nopiv, h->merge_nopiv));
-  if (form_inv) HPS_CHECK_HIP(h, form_fewinv<T>(nF, Fl, nF, sNF2, dinv, finv, fws, nm, s));
+  if (natural)
+    HPS_CHECK_HIP(h, lu_blocks_factor<T>(plan, Fl, nF, sNF2, perm, dinv, linv, ltmp, scratch, info, nm, s));
+  else
+    HPS_CHECK_HIP(h, getrf_ws<T>(nF, Fl, nF, sNF2, perm, dinv, scratch, info, nm, s));
+  if (form_inv) HPS_CHECK_HIP(h, form_fewinv<T>(nF, Fl, nF, sNF2, dinv, (T*)F_inv_out, fws, nm, s));
 
   // ---- solves: X = -D^{-1} [C | h_int] -------------------------------------
-  // one pass for the C columns (width ne) and one for h (width nsrc)
+  // one pass for the C columns (width ne) and one for h (width nsrc); natural
+  // order solves in place (its scratch is the output), pivoting out of place
   for (int pass = 0; pass < 2; ++pass) {
     const int w = pass == 0 ? ne : nsrc;
     if (w <= 0) continue;
     T* Yp = pass == 0 ? Y : Yh;
     T* Zp = pass == 0 ? Z : Zh;
     T* out = (T*)(pass == 0 ? S_out : gt_out);
+    const long sY = (long)ni * w;
+    // DtN with pivoting: right-hand sides in the output, solutions in Yp
+    T* rhs = iti || natural ? Yp : out;
     if (pass == 0) {
-      HPS_CHECK_HIP(h, gather_launch<T>(s, "C", Tin, nc, nec, rows, ni, ex, ne, -1.0, 0, Yp, ne, (long)ni * ne, nm));
+      HPS_CHECK_HIP(h, gather_launch<T>(s, "C", Tin, nc, nec, rows, ni, by_child ? (const int4*)h->ext_child : ex, ne,
+                                        -1.0, 0, rhs, ne, sY, nm));
     } else {
       static const std::string nmh = std::string("merge_gather_h<") + tname<T>() + ">";
       prof::Scope ps(s, nmh.c_str(), 0.0, 2.0 * es * (double)ni * nsrc * nm);
       hipLaunchKernelGGL((vec_gather_kernel<T>), grid_for((long)ni * nsrc, nm), dim3(256), 0, s, (const T*)h_in, nc,
-                         nec, nsrc, rows, ni, -1.0, Yp, nm);
+                         nec, nsrc, rows, ni, -1.0, rhs, nm);
       HPS_CHECK_HIP(h, hipGetLastError());
     }
-    const long sY = (long)ni * w;
     if (!iti) {
-      if (pass == 1 && few)
-        HPS_CHECK_HIP(h, getrs_perm_fewinv<T>(ni, w, Fl, ni, (long)ni * ni, perm, finv, Yp, w, sY, out, w, sY, fsc,
-                                              nm, s));
+      if (natural)
+        HPS_CHECK_HIP(h, lu_blocks_solve<T>(plan, Fl, ni, sNF2, linv, Yp, w, sY, out, w, sY, w, pass == 0, nm, s));
       else
-        HPS_CHECK_HIP(h, getrs_perm_blockinv<T>(ni, w, Fl, ni, (long)ni * ni, perm, dinv, Yp, w, sY, out, w, sY, nm,
-                                                pass == 0 ? binv : nullptr, s));
+        HPS_CHECK_HIP(h, getrs_perm<T>(ni, w, Fl, ni, sNF2, perm, dinv, rhs, w, sY, Yp, w, sY, nm, s));
+      HPS_CHECK_HIP(h, scatter_rows<T>(s, Yp, sY, out, sY, final_of_internal,
+                                       by_child && pass == 0 ? h->ext_pos : nullptr, ni, w, nm));
     } else {
       const long sZ = (long)nF * w;
       // Z = Y_F - D12 Y_G
       HPS_CHECK_HIP(h, coupling_gemm<T>(s, n_d12, d12_blk, nF, w, -1.0, D12, sNF2, Yp + (long)nF * w, w, sY, Yp, w, sY,
                                         Zp, w, sZ, nm));
-      // X_F = W^{-1} Z  (into Y_F)
-      if (pass == 1 && few)
-        HPS_CHECK_HIP(h, getrs_perm_fewinv<T>(nF, w, Fl, nF, sNF2, perm, finv, Zp, w, sZ, Yp, w, sY, fsc, nm, s));
+      // X_F = W^{-1} Z: in place in Z, or into Y_F
+      const T* XF = natural ? Zp : Yp;
+      const long sXF = natural ? sZ : sY;
+      if (natural)
+        HPS_CHECK_HIP(h, lu_blocks_solve<T>(plan, Fl, nF, sNF2, linv, Zp, w, sZ, Yp, w, sY, w, false, nm, s));
       else
-        HPS_CHECK_HIP(h, getrs_perm_blockinv<T>(nF, w, Fl, nF, sNF2, perm, dinv, Zp, w, sZ, Yp, w, sY, nm,
-                                                pass == 0 ? binv : nullptr, s));
+        HPS_CHECK_HIP(h, getrs_perm<T>(nF, w, Fl, nF, sNF2, perm, dinv, Zp, w, sZ, Yp, w, sY, nm, s));
       // X_G = Y_G - D21 X_F  (in place)
-      HPS_CHECK_HIP(h, coupling_gemm<T>(s, n_d21, d21_blk, nF, w, -1.0, D21, sNF2, Yp, w, sY, Yp + (long)nF * w, w,
+      HPS_CHECK_HIP(h, coupling_gemm<T>(s, n_d21, d21_blk, nF, w, -1.0, D21, sNF2, XF, w, sXF, Yp + (long)nF * w, w,
                                         sY, Yp + (long)nF * w, w, sY, nm));
       // internal -> final unknown order
-      static const std::string nms = std::string("row_scatter<") + tname<T>() + ">";
-      prof::Scope ps(s, nms.c_str(), 0.0, 2.0 * es * (double)ni * w * nm);
-      hipLaunchKernelGGL((row_scatter_kernel<T>), grid_for((long)ni * w, nm), dim3(256), 0, s, Yp, out,
-                         final_of_internal, ni, w, nm);
-      HPS_CHECK_HIP(h, hipGetLastError());
+      HPS_CHECK_HIP(h, scatter_rows<T>(s, XF, sXF, out, sY, final_of_internal, nullptr, nF, w, nm));
+      HPS_CHECK_HIP(h, scatter_rows<T>(s, Yp + (long)nF * w, sY, out, sY, final_of_internal + nF, nullptr, nF, w, nm));
     }
   }
 
@@ -878,6 +923,11 @@ int hps_merge_level(hps_handle_t h, int dtype, int kind, int nm, int nc, int nec
   HPS_ARG(h, kind == HPS_KIND_DTN || ni % 2 == 0, "ItI merges need an even number of interface unknowns");
   HPS_ARG(h, T_in && int_rows && int_cols && ext && S_out && F_lu && perm && F_dinv && info, "null pointer");
   HPS_ARG(h, kind == HPS_KIND_DTN || final_of_internal, "ItI merges need the internal->final row map");
+  if (h->dissect != HPS_DISSECT_NONE) {
+    const int nd = h->dissect == HPS_DISSECT_QUAD ? 4 : 12;
+    HPS_ARG(h, kind == HPS_KIND_DTN && final_of_internal && ni % nd == 0 && ne == 2 * ni,
+            "a dissection needs a DtN merge of 4 (8) children with ne = 2 ni and the internal->final row map");
+  }
   HPS_ARG(h, nsrc == 0 || (h_in && gt_out), "h_in/gt_out required when nsrc > 0");
   HPS_ARG(h, n_upd >= 0 && (n_upd == 0 || upd), "bad update block list");
   for (int u = 0; u < n_upd; ++u)
@@ -962,11 +1012,14 @@ static int up_t(hps_handle_t h, int kind, int nm, int nc, int nec, int ni, int n
   if (inj) HPS_CHECK_HIP(h, add2d<T>(ni, w, -1.0, (const T*)inj, w, sY, Yh, w, sY, nm, s));
   T* out = (T*)gt_out;
   if (!iti) {
+    T* x = final_of_internal ? Zh : out;
     if (fewinv)
-      HPS_CHECK_HIP(h, getrs_perm_fewinv<T>(ni, w, Fl, ni, (long)ni * ni, perm, finv, Yh, w, sY, out, w, sY, Ysc, nm,
+      HPS_CHECK_HIP(h, getrs_perm_fewinv<T>(ni, w, Fl, ni, (long)ni * ni, perm, finv, Yh, w, sY, x, w, sY, Ysc, nm,
                                             s));
     else
-      HPS_CHECK_HIP(h, getrs_perm<T>(ni, w, Fl, ni, (long)ni * ni, perm, dinv, Yh, w, sY, out, w, sY, nm, s));
+      HPS_CHECK_HIP(h, getrs_perm<T>(ni, w, Fl, ni, (long)ni * ni, perm, dinv, Yh, w, sY, x, w, sY, nm, s));
+    if (final_of_internal)
+      HPS_CHECK_HIP(h, scatter_rows<T>(s, x, sY, out, sY, final_of_internal, nullptr, ni, w, nm));
   } else {
     const long sZ = (long)nF * w;
     HPS_CHECK_HIP(h, gemm_call<T>(s, nF, w, nF, -1.0, (const T*)D12v, nF, sNF2, Yh + (long)nF * w, w, sY, 1.0, Yh, w,
@@ -977,9 +1030,7 @@ static int up_t(hps_handle_t h, int kind, int nm, int nc, int nec, int ni, int n
       HPS_CHECK_HIP(h, getrs_perm<T>(nF, w, Fl, nF, sNF2, perm, dinv, Zh, w, sZ, Yh, w, sY, nm, s));
     HPS_CHECK_HIP(h, gemm_call<T>(s, nF, w, nF, -1.0, (const T*)D21v, nF, sNF2, Yh, w, sY, 1.0, Yh + (long)nF * w, w,
                                   sY, Yh + (long)nF * w, w, sY, nm));
-    hipLaunchKernelGGL((row_scatter_kernel<T>), grid_for((long)ni * w, nm), dim3(256), 0, s, Yh, out,
-                       final_of_internal, ni, w, nm);
-    HPS_CHECK_HIP(h, hipGetLastError());
+    HPS_CHECK_HIP(h, scatter_rows<T>(s, Yh, sY, out, sY, final_of_internal, nullptr, ni, w, nm));
   }
   if (h_out) {
     T* ho = (T*)h_out;

@@ -36,6 +36,9 @@ struct hps_handle_s {
   int device = -1;  // the stream's device at creation
   bool merge_nopiv = false;  // hps_merge_level factors without row exchanges
   bool leaf_nopiv = false;   // hps_leaf_solve factors without row exchanges (checked)
+  int dissect = HPS_DISSECT_NONE;         // structure of the DtN merges' elimination
+  const int* ext_child = nullptr;         // with one: exterior table by child, and
+  const int* ext_pos = nullptr;           // its rows' final exterior positions
   std::string err;
 };
 

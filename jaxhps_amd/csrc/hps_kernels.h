@@ -22,11 +22,19 @@ struct GemmArgs {
   T* D = nullptr;
   long ldd = 0, sD = 0;
   int batch = 1;
+  // two-level batches: element b is matrix b / nin, part b % nin of it, and a
+  // part's operands lie s*2 apart inside the matrix
+  int nin = 1;
+  long sA2 = 0, sB2 = 0, sC2 = 0, sD2 = 0;
   int transA = 0;
   // triA: A is a packed 32 x 32 diagonal-block inverse used as its unit-lower
   // part (1) or its upper part (2); needs K <= 32.  D may then alias B.
   int triA = 0;
 };
+
+__host__ __device__ inline long batch_offset(int b, int nin, long s, long s2) {
+  return nin == 1 ? (long)b * s : (long)(b / nin) * s + (long)(b % nin) * s2;
+}
 
 template <typename T>
 hipError_t gemm(const GemmArgs<T>& a, hipStream_t s);
@@ -47,14 +55,12 @@ hipError_t gemm_grouped(const GemmArgs<T>& a, int n_blk, const int* blk, hipStre
 // column j whose pivot candidates are all exactly zero.
 size_t getrf_scratch_bytes(int n, int batch);
 size_t dinv_elems(int n);
-// nopiv: the tall panels (and every panel of at most 16 matrices) without row
-// exchanges; for matrices whose natural-order elimination is stable -- the
-// caller checks the factors.  nopiv_all: every register-sized panel without
-// row exchanges, checked in the kernel: a matrix with a multiplier above 64
-// (or not finite) gets info = -1 and must be refactored with pivoting.
+// natural: register-sized matrices without row exchanges, checked in the kernel:
+// a matrix with a multiplier above 64 (or not finite) gets info = -1 and must be
+// refactored with pivoting.
 template <typename T>
 hipError_t getrf_ws(int n, T* A, long lda, long sA, int* perm, T* dinv, int* scratch, int* info, int batch,
-                    hipStream_t s, bool nopiv = false, bool nopiv_all = false);
+                    hipStream_t s, bool natural = false);
 
 // X = A^{-1} R from getrf_ws's factors.  R (n x nrhs, row stride ldr, batch
 // stride sR) is read only; X must not alias R.
@@ -68,22 +74,8 @@ template <typename T>
 hipError_t getrs_inplace(int n, int nrhs, const T* LU, long lda, long sA, const T* dinv, T* X, long ldx, long sX,
                          int batch, hipStream_t s);
 
-// Many-column solves of large low-precision factors through the inverses of
-// their 512 x 512 diagonal blocks (products with K = 512 instead of 32-row
-// steps).  Eligible: n >= LU_WIDE_MIN, n a multiple of 512, more than 16
-// columns; wsp holds blockinv_workspace_elems(n, nrhs) elements (otherwise,
-// or with wsp == nullptr, this is getrs_perm).
+// few-column block size and the wide column block of large pivoted matrices
 constexpr int LU_WIDE_MIN = 3072;
-constexpr int BLOCKINV_NB = 512;
-constexpr int BLOCKINV_MAX_BATCH = 2;  // the inverses are formed matrix by matrix: top levels only
-inline bool blockinv_eligible(int n, int nrhs) { return n >= LU_WIDE_MIN && n % BLOCKINV_NB == 0 && nrhs > 16; }
-inline size_t blockinv_workspace_elems(int n, int nrhs) {
-  return blockinv_eligible(n, nrhs) ? 2 * (size_t)n * BLOCKINV_NB + (size_t)BLOCKINV_NB * nrhs : 0;
-}
-template <typename T>
-hipError_t getrs_perm_blockinv(int n, int nrhs, const T* LU, long lda, long sA, const int* perm, const T* dinv,
-                               const T* R, long ldr, long sR, T* X, long ldx, long sX, int batch, T* wsp,
-                               hipStream_t s);
 
 // Few-column solves (at most 16 columns) of matrices too large for one
 // workgroup, in fewer than 128 matrices: the refinement's up passes through
@@ -108,6 +100,126 @@ hipError_t form_fewinv(int n, const T* LU, long lda, long sA, const T* dinv, T* 
 template <typename T>
 hipError_t getrs_perm_fewinv(int n, int nrhs, const T* LU, long lda, long sA, const int* perm, const T* inv,
                              const T* R, long ldr, long sR, T* X, long ldx, long sX, T* Y, int batch, hipStream_t s);
+
+// ---------------------------------------------------------------------------
+// Natural-order LU and many-column solves by blocks (lu_blocks.h)
+// ---------------------------------------------------------------------------
+// The elimination's block structure: stages of `cnt` equal diagonal blocks
+// (groups) that do not couple to one another.  Group i of a stage couples,
+// among the later unknowns, to the runs (s[j], ns[j]) only, and its right-hand
+// sides are nonzero in nc columns from c0 + i c_step only.
+constexpr int LUB_NB = 128;       // block of the elimination inside a group
+constexpr int LUB_MAX_CNT = 4;    // groups per stage
+constexpr int LUB_MAX_STAGES = 3;
+constexpr int LUB_MAX_RUNS = 4;
+struct LuGroup {
+  int nrun = 0;
+  int s[LUB_MAX_RUNS] = {}, ns[LUB_MAX_RUNS] = {};
+};
+struct LuStage {
+  int cnt = 1, size = 0, r0 = 0;  // groups, unknowns of a group, first unknown of the stage
+  int c0 = 0, nc = 0, c_step = 0;
+  LuGroup g[LUB_MAX_CNT];
+};
+struct LuPlan {
+  int n = 0, nstage = 0;
+  LuStage st[LUB_MAX_STAGES];
+};
+// one dense group of n unknowns
+inline LuPlan lu_plan_dense(int n, int ncols) {
+  LuPlan p;
+  p.n = n;
+  p.nstage = 1;
+  p.st[0].size = n;
+  p.st[0].nc = ncols;
+  return p;
+}
+// 2D DtN merge, unknowns in the order of the interfaces a|b, c|d, b|c, d|a (m
+// each), columns by child: the first two do not couple
+inline LuPlan lu_plan_quad(int m) {
+  LuPlan p;
+  p.n = 4 * m;
+  p.nstage = 2;
+  p.st[0].cnt = 2;
+  p.st[0].size = m;
+  p.st[0].nc = p.st[0].c_step = 4 * m;
+  for (int i = 0; i < 2; ++i) {
+    p.st[0].g[i].nrun = 1;
+    p.st[0].g[i].s[0] = p.st[0].g[i].ns[0] = 2 * m;
+  }
+  p.st[1].size = p.st[1].r0 = 2 * m;
+  p.st[1].nc = 8 * m;
+  return p;
+}
+// 3D DtN merge (children a .. h, columns by child): the x-interfaces a|b, d|c of
+// the upper slab and e|f, h|g of the lower one (group 2 z + y), the y-interfaces
+// of each slab (two groups), the z-interfaces at y- and at y+
+inline LuPlan lu_plan_oct(int m) {
+  LuPlan p;
+  p.n = 12 * m;
+  p.nstage = 3;
+  p.st[0].cnt = 4;
+  p.st[0].size = m;
+  p.st[0].nc = p.st[0].c_step = 6 * m;
+  for (int i = 0; i < 4; ++i) {
+    LuGroup& g = p.st[0].g[i];
+    g.nrun = 2;
+    g.s[0] = 4 * m + (i / 2) * 2 * m;
+    g.s[1] = 8 * m + (i % 2) * 2 * m;
+    g.ns[0] = g.ns[1] = 2 * m;
+  }
+  p.st[1].cnt = 2;
+  p.st[1].size = 2 * m;
+  p.st[1].r0 = 4 * m;
+  p.st[1].nc = p.st[1].c_step = 12 * m;
+  for (int i = 0; i < 2; ++i) {
+    p.st[1].g[i].nrun = 1;
+    p.st[1].g[i].s[0] = 8 * m;
+    p.st[1].g[i].ns[0] = 4 * m;
+  }
+  p.st[2].size = 4 * m;
+  p.st[2].r0 = 8 * m;
+  p.st[2].nc = 24 * m;
+  return p;
+}
+// groups are cut into equal blocks, a multiple of 32 wide and at most LUB_NB
+inline int lub_block(int size) {
+  const int nb = (size + LUB_NB - 1) / LUB_NB;
+  return ((size + nb - 1) / nb + 31) / 32 * 32;
+}
+inline int lub_blocks(int size) { return (size + lub_block(size) - 1) / lub_block(size); }
+// elements of the block inverses that a solve needs and of the factorisation's
+// scratch, bytes of its integer scratch
+inline size_t lub_inv_elems(const LuPlan& p, int batch) {
+  size_t t = 0;
+  for (int i = 0; i < p.nstage; ++i)
+    t += (size_t)p.st[i].cnt * lub_blocks(p.st[i].size) * 2 * lub_block(p.st[i].size) * lub_block(p.st[i].size);
+  return t * batch;
+}
+inline size_t lub_tmp_elems(const LuPlan& p, int batch) {
+  size_t m = 0;
+  for (int i = 0; i < p.nstage; ++i) {
+    const LuStage& s = p.st[i];
+    const size_t t = (size_t)s.cnt * lub_block(s.size) * ((size_t)(s.size + p.n - s.r0 - s.cnt * s.size) + 32);
+    m = m > t ? m : t;
+  }
+  return m * batch;
+}
+size_t lub_scratch_bytes(const LuPlan& p, int batch);
+
+// A = L U in natural order, in place (batch matrices, row stride lda, batch
+// stride sA); perm becomes the identity, dinv as getrf_ws's, inv the inverses
+// of every block's L and U (lub_inv_elems), tmp lub_tmp_elems elements.
+// info[b] = -1 where a multiplier exceeds 64, a pivot is zero or a value is not
+// finite (the matrix then needs pivoting), else 0.
+template <typename T>
+hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* perm, T* dinv, T* inv, T* tmp,
+                            int* scratch, int* info, int batch, hipStream_t s);
+// B = A^{-1} B; X is scratch of B's shape.  cols: the right-hand sides have the
+// plan's column structure (otherwise they are dense).
+template <typename T>
+hipError_t lu_blocks_solve(const LuPlan& plan, const T* A, long lda, long sA, const T* inv, T* B, long ldb, long sB,
+                           T* X, long ldx, long sX, int nrhs, bool cols, int batch, hipStream_t s);
 
 // X = A^{-H} R from getrf_ws's factors (A^H = U^H L^H P).  W is n x nrhs
 // scratch per batch element (row stride nrhs); X, W and R must not alias.

@@ -42,10 +42,6 @@ namespace hps {
 #endif
 
 constexpr int LU_NB = 32;
-// with row exchanges off, batches this small take the unpivoted panel kernel
-// for every panel: the pivoted register panels then run one workgroup per
-// matrix on an otherwise idle GPU
-constexpr int LU_NOPIV_SMALL_BATCH = 16;
 // largest multiplier an unpivoted register panel accepts (the leaf and merge
 // matrices of the HPS tree stay below 2)
 constexpr double LU_NOPIV_BOUND = 64.0;
@@ -72,7 +68,6 @@ static int lu_outer_block(int n) { return n > LU_BLOCKED_MIN ? LU_NBO : (n >= 25
 // blocks of 512: their trailing updates are single large GEMMs whose K = 512
 // halves the C-tile traffic per flop of K = 256 (the few-column solves keep
 // 256-blocks, which their block kernel holds)
-static_assert(LU_WIDE_MIN == 3072 && BLOCKINV_NB == 2 * LU_NBO, "block sizes");
 static int lu_outer_block_wide(int n) { return n >= LU_WIDE_MIN ? 2 * LU_NBO : lu_outer_block(n); }
 
 static __global__ void fill_int_kernel(int* p, long n, int v) {
@@ -759,14 +754,16 @@ __device__ __forceinline__ void panel_steps(std::integer_sequence<int, J...>, T 
 // the panel's row permutation to the rest of its matrix itself.
 template <typename T, int RPT, int THREADS, bool NOPIV = false>
 __global__ __launch_bounds__(THREADS) void getrf_panel_rows_kernel(int n, T* A, long lda, long sA, int k, int nb,
-                                                                   int* ipiv, int* info, T* dinv, int* swtab) {
+                                                                   int* ipiv, int* info, T* dinv, int* swtab,
+                                                                   int nin, long sA2) {
   using R = typename real_of<T>::type;
   __shared__ PanelLDS<T, THREADS / 64> sh;
   __shared__ T Dblk[LU_NB][LU_NB + 1];
   const int b = blockIdx.x;
   const int t = threadIdx.x;
   const int m = n - k;
-  T* P = A + (long)b * sA + (long)k * lda + k;
+  T* P = A + batch_offset(b, nin, sA, sA2) + (long)k * lda + k;
+  info += b / nin;  // the matrix this part belongs to
   int* ipivb = ipiv + (long)b * n;
   T x[RPT][LU_NB];
   int pos[RPT];
@@ -779,7 +776,7 @@ __global__ __launch_bounds__(THREADS) void getrf_panel_rows_kernel(int n, T* A, 
     for (int c = 0; c < LU_NB; ++c) x[r][c] = (live[r] && c < nb) ? P[(long)pos[r] * lda + c] : s_zero<T>();
   }
   auto on_pivot = [&](int J, int pq, R fv, unsigned) {
-    if (t == 0) record_pivot(k, J, pq, fv == R(0), ipivb, info, b);
+    if (t == 0) record_pivot(k, J, pq, fv == R(0), ipivb, info, 0);
   };
   R lmax = R(0);
   panel_steps<T, RPT, THREADS / 64, NOPIV>(std::make_integer_sequence<int, LU_NB>{}, x, pos, live, sh, nb, on_pivot,
@@ -802,7 +799,7 @@ __global__ __launch_bounds__(THREADS) void getrf_panel_rows_kernel(int n, T* A, 
       for (int w = 1; w < THREADS / 64; ++w) mx = (wmax[w] > mx || wmax[w] != wmax[w]) ? wmax[w] : mx;
       // a zero pivot in the natural order (info > 0) is no verdict on the
       // matrix either: pivoting decides
-      if (!(mx <= R(LU_NOPIV_BOUND)) || info[b] > 0) info[b] = -1;
+      if (!(mx <= R(LU_NOPIV_BOUND)) || info[0] > 0) info[0] = -1;
     }
   }
   // net row permutation of the panel: every row whose position changed
@@ -1223,7 +1220,7 @@ __device__ __forceinline__ void mma_step(T a, T b, typename Mfma<typename real_o
 template <typename T>
 __global__ __launch_bounds__(256) void getrf_panel_nopiv_kernel(int n, T* A, long lda, long sA, int k, int nb,
                                                                 int* ipiv, T* dinv, int* arrivals, int* info,
-                                                                int row_wgs, int u12_end) {
+                                                                int row_wgs, int u12_end, int nin, long sA2) {
   using R = typename real_of<T>::type;
   using M = Mfma<R>;
   using acc_t = typename M::acc_t;
@@ -1235,7 +1232,7 @@ __global__ __launch_bounds__(256) void getrf_panel_nopiv_kernel(int n, T* A, lon
   const int b = blockIdx.y;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, li = tid & 15, lk = (tid & 63) >> 4;
-  T* Ab = A + (long)b * sA;
+  T* Ab = A + batch_offset(b, nin, sA, sA2);
   // every load is issued before the first is waited for: the diagonal block's
   // four entries of this thread, then its operand of the final product -- the
   // rows of A21 as the MFMA's left operand (wave w: rows 16 w .. 16 w + 15),
@@ -1387,7 +1384,7 @@ __global__ __launch_bounds__(256) void getrf_panel_nopiv_kernel(int n, T* A, lon
         }
       }
   }
-  if (!ok) info[b] = -1;  // every writer writes the same value
+  if (!ok) info[b / nin] = -1;  // every writer writes the same value
   if (!last) return;
   for (int idx = tid; idx < nb * nb; idx += 256) {
     const int rr = idx / nb, c = idx - rr * nb;
@@ -1417,16 +1414,16 @@ static hipError_t launch_panel(int n, T* A, long lda, long sA, int k, int nb, in
     prof::Scope ps(s, nm_rows.c_str(), pf, 2.0 * sizeof(T) * (double)m * nb * batch);
     if (m <= 128)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 128, true>), dim3(batch), dim3(128), 0, s, n, A, lda, sA, k,
-                         nb, ipiv, info, dinv, swtab);
+                         nb, ipiv, info, dinv, swtab, 1, 0L);
     else if (m <= 256)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 256, true>), dim3(batch), dim3(256), 0, s, n, A, lda, sA, k,
-                         nb, ipiv, info, dinv, swtab);
+                         nb, ipiv, info, dinv, swtab, 1, 0L);
     else if (m <= 512)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 512, true>), dim3(batch), dim3(512), 0, s, n, A, lda, sA, k,
-                         nb, ipiv, info, dinv, swtab);
+                         nb, ipiv, info, dinv, swtab, 1, 0L);
     else if constexpr (sizeof(T) < 16)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 1024, true>), dim3(batch), dim3(1024), 0, s, n, A, lda, sA,
-                         k, nb, ipiv, info, dinv, swtab);
+                         k, nb, ipiv, info, dinv, swtab, 1, 0L);
     else
       return hipErrorInvalidValue;  // not reached: rows_panel_max<c128>() is 512
     return hipGetLastError();
@@ -1437,16 +1434,16 @@ static hipError_t launch_panel(int n, T* A, long lda, long sA, int k, int nb, in
     // short panels in smaller workgroups: more of them share a CU
     if (m <= 128)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 128>), dim3(batch), dim3(128), 0, s, n, A, lda, sA, k, nb,
-                         ipiv, info, dinv, swtab);
+                         ipiv, info, dinv, swtab, 1, 0L);
     else if (m <= 256)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 256>), dim3(batch), dim3(256), 0, s, n, A, lda, sA, k, nb,
-                         ipiv, info, dinv, swtab);
+                         ipiv, info, dinv, swtab, 1, 0L);
     else if (m <= 512)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 512>), dim3(batch), dim3(512), 0, s, n, A, lda, sA, k, nb,
-                         ipiv, info, dinv, swtab);
+                         ipiv, info, dinv, swtab, 1, 0L);
     else if constexpr (sizeof(T) < 16)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 1024>), dim3(batch), dim3(1024), 0, s, n, A, lda, sA, k, nb,
-                         ipiv, info, dinv, swtab);
+                         ipiv, info, dinv, swtab, 1, 0L);
     else
       return hipErrorInvalidValue;  // not reached: rows_panel_max<c128>() is 512
     return hipGetLastError();
@@ -1492,9 +1489,8 @@ static hipError_t launch_panel(int n, T* A, long lda, long sA, int k, int nb, in
 
 #if HPS_LU_TYPES & 1
 size_t getrf_scratch_bytes(int n, int batch) {
-  // ipiv, swap tables, tournament candidates (two sets), then one arrival
-  // counter per matrix for the unpivoted panel kernel
-  return ((size_t)batch * n + (size_t)batch * SWTAB + 2 * tslu_cand_ints(n, batch) + (size_t)batch) * sizeof(int);
+  // ipiv, swap tables, tournament candidates (two sets)
+  return ((size_t)batch * n + (size_t)batch * SWTAB + 2 * tslu_cand_ints(n, batch)) * sizeof(int);
 }
 #endif
 
@@ -1504,7 +1500,7 @@ size_t getrf_scratch_bytes(int n, int batch) {
 // (the L^H solve).  256 threads = 32 rows x 8 columns per workgroup.
 template <typename T, bool UPPER, bool CT = false>
 __global__ __launch_bounds__(256) void trsm_inv_kernel(int n, int nrhs, const T* dinv, T* X, long ldx, long sX, int k,
-                                                       int nb) {
+                                                       int nb, int nin = 1, long sX2 = 0) {
   __shared__ T Di[LU_NB][LU_NB + 1];
   __shared__ T Xs[LU_NB][8];
   const int b = blockIdx.y;
@@ -1531,7 +1527,7 @@ __global__ __launch_bounds__(256) void trsm_inv_kernel(int n, int nrhs, const T*
     }
     Di[r][q] = v;
   }
-  T* Xb = X + (long)b * sX;
+  T* Xb = X + batch_offset(b, nin, sX, sX2);
   Xs[rr][cc] = (c < nrhs && rr < nb) ? Xb[(long)(k + rr) * ldx + c] : s_zero<T>();
   __syncthreads();
   if (c < nrhs && rr < nb) {
@@ -1546,7 +1542,7 @@ __global__ __launch_bounds__(256) void trsm_inv_kernel(int n, int nrhs, const T*
 // triangle) for wide X, the LDS kernel above for ncols <= 16.
 template <typename T>
 static hipError_t trsm_block(bool upper, int n, int ncols, const T* dinv, T* X, long ldx, long sX, int k, int nb,
-                             int batch, hipStream_t s, const std::string& label) {
+                             int batch, hipStream_t s, const std::string& label, int nin = 1, long sX2 = 0) {
   if (ncols > 16) {
     GemmArgs<T> g;
     g.M = nb;
@@ -1563,28 +1559,32 @@ static hipError_t trsm_block(bool upper, int n, int ncols, const T* dinv, T* X, 
     g.sD = sX;
     g.batch = batch;
     g.triA = upper ? 2 : 1;
+    if (nin > 1) {  // the inverses are stored by part
+      g.nin = nin;
+      g.sA2 = g.sA;
+      g.sA *= nin;
+      g.sB2 = g.sD2 = sX2;
+    }
     return gemm<T>(g, s);
   }
   prof::Scope ps(s, label.c_str(), flop_mult<T>() * batch * (double)nb * nb * ncols,
                  2.0 * sizeof(T) * (double)nb * ncols * batch);
   dim3 tgrid(ceil_div(ncols, 8), batch);
   if (upper)
-    hipLaunchKernelGGL((trsm_inv_kernel<T, true>), tgrid, dim3(256), 0, s, n, ncols, dinv, X, ldx, sX, k, nb);
+    hipLaunchKernelGGL((trsm_inv_kernel<T, true>), tgrid, dim3(256), 0, s, n, ncols, dinv, X, ldx, sX, k, nb, nin, sX2);
   else
-    hipLaunchKernelGGL((trsm_inv_kernel<T, false>), tgrid, dim3(256), 0, s, n, ncols, dinv, X, ldx, sX, k, nb);
+    hipLaunchKernelGGL((trsm_inv_kernel<T, false>), tgrid, dim3(256), 0, s, n, ncols, dinv, X, ldx, sX, k, nb, nin, sX2);
   return hipGetLastError();
 }
 
 template <typename T>
 hipError_t getrf_ws(int n, T* A, long lda, long sA, int* perm, T* dinv, int* scratch, int* info, int batch,
-                    hipStream_t s, bool nopiv, bool nopiv_all) {
+                    hipStream_t s, bool natural) {
   if (n <= 0 || batch <= 0) return hipSuccess;
   int* ipiv = scratch;
   int* swtab = scratch + (long)batch * n;
   int* cand = swtab + (long)batch * SWTAB;
-  int* arrivals = cand + 2 * tslu_cand_ints(n, batch);  // zero between unpivoted panel launches
   hipLaunchKernelGGL(fill_int_kernel, dim3(ceil_div(batch, 256)), dim3(256), 0, s, info, (long)batch, 0);
-  if (nopiv) hipLaunchKernelGGL(fill_int_kernel, dim3(ceil_div(batch, 256)), dim3(256), 0, s, arrivals, (long)batch, 0);
   auto gemm_update = [&](int M, int N, int K, const T* Ap, const T* Bp, T* Cp) -> hipError_t {
     if (M <= 0 || N <= 0 || K <= 0) return hipSuccess;
     GemmArgs<T> g;
@@ -1616,35 +1616,14 @@ hipError_t getrf_ws(int n, T* A, long lda, long sA, int* perm, T* dinv, int* scr
     const int bend = n - k0 < nbo ? n : k0 + nbo;
     for (int k = k0; k < bend; k += LU_NB) {
       const int nb = bend - k < LU_NB ? bend - k : LU_NB;
-      bool swapped = false, u12_done = false;
-      hipError_t e = hipSuccess;
-      if (nopiv && (n - k > rows_panel_max<T>() || batch <= LU_NOPIV_SMALL_BATCH)) {
-        static const std::string nm_np = std::string("getrf_panel_nopiv<") + tname<T>() + ">";
-        const int m = n - k;
-        prof::Scope ps(s, nm_np.c_str(), flop_mult<T>() * batch * ((double)m * nb * nb - (double)nb * nb * nb / 3.0),
-                       2.0 * sizeof(T) * (double)m * nb * batch);
-        // row workgroups, then one workgroup per 32 columns of the block's U12
-        const int row_wgs = ceil_div(m - nb, NOPIV_ROWS) > 0 ? ceil_div(m - nb, NOPIV_ROWS) : 1;
-        const int u12_wgs = bend - k - nb > 0 ? ceil_div(bend - k - nb, LU_NB) : 0;
-        for (int b0 = 0; b0 < batch; b0 += 65535) {
-          const int bc = batch - b0 < 65535 ? batch - b0 : 65535;
-          hipLaunchKernelGGL((getrf_panel_nopiv_kernel<T>), dim3(row_wgs + u12_wgs, bc), dim3(256), 0, s, n,
-                             A + (long)b0 * sA, lda, sA, k, nb, ipiv + (long)b0 * n,
-                             dinv + (long)b0 * ((n + LU_NB - 1) / LU_NB) * LU_NB * LU_NB, arrivals + b0, info + b0,
-                             row_wgs, bend);
-        }
-        e = hipGetLastError();
-        swapped = true;  // nothing to swap
-        u12_done = true;
-      } else {
-        e = launch_panel<T>(n, A, lda, sA, k, nb, ipiv, info, dinv, swtab, cand, batch, s, &swapped, nopiv_all);
-      }
+      bool swapped = false;
+      hipError_t e =
+          launch_panel<T>(n, A, lda, sA, k, nb, ipiv, info, dinv, swtab, cand, batch, s, &swapped, natural);
       if (e != hipSuccess) return e;
       const int others = n - nb;
       if (swapped) {
-        // U12 = inv(L11) A12 for the block's columns right of the panel (the
-        // unpivoted panel kernel forms it itself)
-        if (bend - k - nb > 0 && !u12_done) {
+        // U12 = inv(L11) A12 for the block's columns right of the panel
+        if (bend - k - nb > 0) {
           static const std::string nm = std::string("getrf_u12<") + tname<T>() + ">";
           e = trsm_block<T>(false, n, bend - k - nb, dinv, A + k + nb, lda, sA, k, nb, batch, s, nm);
           if (e != hipSuccess) return e;
@@ -2127,17 +2106,6 @@ hipError_t getrs_inplace(int n, int nrhs, const T* LU, long lda, long sA, const 
   return hipGetLastError();
 }
 
-// ---------------------------------------------------------------------------
-// Many-column solves with large factors in low precision (the S solves of the
-// top merge levels, refined in FP64 afterwards): the inverses of the 512 x 512
-// diagonal blocks of L (unit lower) and U are formed once per solve (all
-// blocks of a matrix as one batched 512-column triangular solve of the
-// identity), after which every block step is a product with K = 512 instead
-// of sixteen 32-row steps whose updates stream the block's columns through
-// HBM.  The products read the explicit block inverses, so the rounding is
-// that of the inverses (cond(L_kk), cond(U_kk): pivot growth ~1 for the merge
-// matrices), corrected by the refinement.
-// ---------------------------------------------------------------------------
 template <typename T>
 __global__ void eye_kernel(T* X, int n, long sX, int batch) {
   const long per = (long)n * n;
@@ -2204,82 +2172,6 @@ static hipError_t form_diag_inverses(int NB, int count, const T* Lb, long lda, l
                       Uinv + (long)k * NB, NB, sBlk, nullptr, 0, 0, Uinv + (long)k * NB, NB, sBlk, count, 2));
     HPS_LU_CHECK(gemm(k, NB, LU_NB, -1.0, 1.0, Lb + k, lda, sDiag, Uinv + (long)k * NB, NB, sBlk, Uinv, NB, sBlk,
                       Uinv, NB, sBlk, count, 0));
-  }
-  return hipGetLastError();
-}
-
-template <typename T>
-hipError_t getrs_perm_blockinv(int n, int nrhs, const T* LU, long lda, long sA, const int* perm, const T* dinv,
-                               const T* R, long ldr, long sR, T* X, long ldx, long sX, int batch, T* wsp,
-                               hipStream_t s) {
-  if (!blockinv_eligible(n, nrhs) || wsp == nullptr)
-    return getrs_perm<T>(n, nrhs, LU, lda, sA, perm, dinv, R, ldr, sR, X, ldx, sX, batch, s);
-  const int NB = BLOCKINV_NB;
-  const int nblk = n / NB;
-  const long sBlk = (long)NB * NB;  // one block inverse
-  T* Linv = wsp;
-  T* Uinv = wsp + (long)nblk * sBlk;
-  T* tmp = Uinv + (long)nblk * sBlk;  // NB x nrhs
-  const long dstride = (long)((n + LU_NB - 1) / LU_NB) * LU_NB * LU_NB;  // dinv per matrix
-  for (int b0 = 0; b0 < batch; b0 += 65535) {
-    static const std::string nm = std::string("getrs_gather<") + tname<T>() + ">";
-    prof::Scope ps(s, nm.c_str(), 0.0, 2.0 * sizeof(T) * (double)n * nrhs * batch);
-    int bc = batch - b0 < 65535 ? batch - b0 : 65535;
-    dim3 grid(ceil_div(nrhs, 64), n, bc);
-    hipLaunchKernelGGL((gather_rows_kernel<T>), grid, dim3(64), 0, s, n, nrhs, perm + (long)b0 * n,
-                       R + (long)b0 * sR, ldr, sR, X + (long)b0 * sX, ldx, sX);
-  }
-  auto gemm = [&](int M, int N, int K, double alpha, double beta, const T* A, long la, long sa, const T* B, long lb,
-                  long sb, const T* C, long lc, long sc, T* D, long ld, long sd, int bt, int tri) -> hipError_t {
-    if (M <= 0 || N <= 0 || K <= 0) return hipSuccess;
-    GemmArgs<T> g;
-    g.M = M;
-    g.N = N;
-    g.K = K;
-    g.alpha = alpha;
-    g.beta = beta;
-    g.A = A;
-    g.lda = la;
-    g.sA = sa;
-    g.B = B;
-    g.ldb = lb;
-    g.sB = sb;
-    g.C = C;
-    g.ldc = lc;
-    g.sC = sc;
-    g.D = D;
-    g.ldd = ld;
-    g.sD = sd;
-    g.batch = bt;
-    g.triA = tri;
-    return hps::gemm<T>(g, s);
-  };
-  for (int b = 0; b < batch; ++b) {
-    const T* Lb = LU + (long)b * sA;
-    const T* db = dinv + (long)b * dstride;
-    T* Xb = X + (long)b * sX;
-    // block inverses: Linv_j = inv(L_jj), Uinv_j = inv(U_jj), all j at once
-    HPS_LU_CHECK(form_diag_inverses<T>(NB, nblk, Lb, lda, (long)NB * (lda + 1), db,
-                                       (long)(NB / LU_NB) * LU_NB * LU_NB, Linv, Uinv, s));
-    // forward: X_j = Linv_j X_j, then the rows below
-    for (int j = 0; j < nblk; ++j) {
-      const int k0 = j * NB;
-      HPS_LU_CHECK(gemm(NB, nrhs, NB, 1.0, 0.0, Linv + (long)j * sBlk, NB, 0, Xb + (long)k0 * ldx, ldx, 0, nullptr,
-                        0, 0, tmp, nrhs, 0, 1, 0));
-      HPS_LU_CHECK(copy2d<T>(NB, nrhs, 1.0, tmp, nrhs, 0, Xb + (long)k0 * ldx, ldx, 0, 1, s));
-      HPS_LU_CHECK(gemm(n - k0 - NB, nrhs, NB, -1.0, 1.0, Lb + (long)(k0 + NB) * lda + k0, lda, 0,
-                        Xb + (long)k0 * ldx, ldx, 0, Xb + (long)(k0 + NB) * ldx, ldx, 0,
-                        Xb + (long)(k0 + NB) * ldx, ldx, 0, 1, 0));
-    }
-    // backward: X_j = Uinv_j X_j, then the rows above
-    for (int j = nblk - 1; j >= 0; --j) {
-      const int k0 = j * NB;
-      HPS_LU_CHECK(gemm(NB, nrhs, NB, 1.0, 0.0, Uinv + (long)j * sBlk, NB, 0, Xb + (long)k0 * ldx, ldx, 0, nullptr,
-                        0, 0, tmp, nrhs, 0, 1, 0));
-      HPS_LU_CHECK(copy2d<T>(NB, nrhs, 1.0, tmp, nrhs, 0, Xb + (long)k0 * ldx, ldx, 0, 1, s));
-      HPS_LU_CHECK(gemm(k0, nrhs, NB, -1.0, 1.0, Lb + k0, lda, 0, Xb + (long)k0 * ldx, ldx, 0, Xb, ldx, 0, Xb, ldx,
-                        0, 1, 0));
-    }
   }
   return hipGetLastError();
 }
@@ -2467,7 +2359,7 @@ hipError_t getrs_conjt(int n, int nrhs, const T* LU, long lda, long sA, const in
         prof::Scope ps(s, nm.c_str(), flop_mult<T>() * batch * (double)nb * nb * nrhs,
                        2.0 * sizeof(T) * (double)nb * nrhs * batch);
         hipLaunchKernelGGL((trsm_inv_kernel<T, false, true>), tgrid, dim3(256), 0, s, n, nrhs, dinv, W, ldw, sW, k,
-                           nb);
+                           nb, 1, 0L);
       }
       HPS_LU_CHECK(gemm_ct(bend - k - nb, nb, LU + (long)k * lda + k + nb, W + (long)k * ldw, W + (long)(k + nb) * ldw));
     }
@@ -2486,7 +2378,7 @@ hipError_t getrs_conjt(int n, int nrhs, const T* LU, long lda, long sA, const in
         prof::Scope ps(s, nm.c_str(), flop_mult<T>() * batch * (double)nb * nb * nrhs,
                        2.0 * sizeof(T) * (double)nb * nrhs * batch);
         hipLaunchKernelGGL((trsm_inv_kernel<T, true, true>), tgrid, dim3(256), 0, s, n, nrhs, dinv, W, ldw, sW, k,
-                           nb);
+                           nb, 1, 0L);
       }
       HPS_LU_CHECK(gemm_ct(k - k0, nb, LU + (long)k * lda + k0, W + (long)k * ldw, W + (long)k0 * ldw));
     }
@@ -2503,19 +2395,25 @@ hipError_t getrs_conjt(int n, int nrhs, const T* LU, long lda, long sA, const in
   return hipGetLastError();
 }
 
+}  // namespace hps
+#include "lu_blocks.h"
+namespace hps {
+
 #if HPS_LU_TYPES & 1
 size_t dinv_elems(int n) { return (size_t)((n + LU_NB - 1) / LU_NB) * LU_NB * LU_NB; }
 #endif
 
 #define HPS_INST_LU(T)                                                                                          \
-  template hipError_t getrf_ws<T>(int, T*, long, long, int*, T*, int*, int*, int, hipStream_t, bool, bool);           \
+  template hipError_t getrf_ws<T>(int, T*, long, long, int*, T*, int*, int*, int, hipStream_t, bool);             \
   template hipError_t getrs_perm<T>(int, int, const T*, long, long, const int*, const T*, const T*, long, long, \
                                     T*, long, long, int, hipStream_t);                                          \
   template hipError_t getrs_inplace<T>(int, int, const T*, long, long, const T*, T*, long, long, int, hipStream_t); \
-  template hipError_t getrs_perm_blockinv<T>(int, int, const T*, long, long, const int*, const T*, const T*, long,     \
-                                             long, T*, long, long, int, T*, hipStream_t);                             \
   template hipError_t getrs_conjt<T>(int, int, const T*, long, long, const int*, const T*, const T*, long, long, \
                                      T*, long, long, T*, int, hipStream_t);                                     \
+  template hipError_t lu_blocks_factor<T>(const LuPlan&, T*, long, long, int*, T*, T*, T*, int*, int*, int,      \
+                                          hipStream_t);                                                          \
+  template hipError_t lu_blocks_solve<T>(const LuPlan&, const T*, long, long, const T*, T*, long, long, T*, long,  \
+                                         long, int, bool, int, hipStream_t);                                      \
   template hipError_t form_fewinv<T>(int, const T*, long, long, const T*, T*, T*, int, hipStream_t);            \
   template hipError_t getrs_perm_fewinv<T>(int, int, const T*, long, long, const int*, const T*, const T*, long,  \
                                            long, T*, long, long, T*, int, hipStream_t);

@@ -69,6 +69,44 @@ def test_unpivoted_panel_rejects(gpu, dtype, row):
         assert info[2] == -1 and (np.delete(info, 2) == 0).all(), info
 
 
+@pytest.mark.parametrize("kind,m,nm,dtype", [
+    ("quad", 47, 2, torch.float64), ("quad", 48, 3, torch.float32), ("quad", 65, 2, torch.complex128),
+    ("quad", 129, 1, torch.float64), ("quad", 20, 40, torch.complex64), ("oct", 47, 1, torch.float64),
+    ("oct", 49, 2, torch.float64), ("oct", 64, 1, torch.float32), ("iti", 65, 3, torch.complex128),
+    ("iti", 20, 30, torch.complex64)])
+def test_block_elimination_matches_pivoted(gpu, kind, m, nm, dtype):
+    """Natural-order block elimination (dense below 48 unknowns an interface,
+    dissected from there; partial blocks, many and few matrices) against the
+    pivoted merge.  The matrices' condition is below 10, so both are within
+    10 n eps of the exact result in the maximum norm."""
+    from jaxhps_amd._stages import merge_level, up_level
+    from jaxhps_amd._tables import oct_merge_tables, quad_merge_tables
+
+    print(f"block elimination {kind} m={m} nm={nm} {dtype}", flush=True)
+    tb = oct_merge_tables(m) if kind == "oct" else quad_merge_tables(m, "iti" if kind == "iti" else "dtn")
+    g = torch.Generator(device=gpu).manual_seed(m)
+    real = torch.float64
+
+    def rand(*shape):
+        x = torch.randn(shape, generator=g, device=gpu, dtype=real)
+        return torch.complex(x, torch.randn(shape, generator=g, device=gpu, dtype=real)) if dtype.is_complex else x
+
+    T = 0.1 * rand(tb.nc * nm, tb.nec, tb.nec) / tb.nec**0.5
+    T = (T + (0.0 if kind == "iti" else 2.0) * torch.eye(tb.nec, device=gpu, dtype=T.dtype)).to(dtype).contiguous()
+    h = rand(tb.nc * nm, tb.nec, 3).to(dtype).contiguous()
+    nat = merge_level(T, h, tb, keep_factors=True, pivot=False)
+    piv = merge_level(T, h, tb, keep_factors=True, pivot=True)
+    assert (nat.info == 0).all()
+    bound = 2 * 10 * tb.ni * EPS[dtype]
+    for name in ("S", "T", "h", "gt"):
+        a, b = getattr(nat, name), getattr(piv, name)
+        assert float((a - b).abs().max() / b.abs().max()) < bound, name
+    # the stored factors serve the up pass: the same data give the same result
+    gt, ho = up_level(h, nat)
+    assert float((gt - piv.gt).abs().max() / piv.gt.abs().max()) < bound
+    assert float((ho - piv.h).abs().max() / piv.h.abs().max()) < bound
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("batch,M,N,K", [(1, 1, 1, 1), (3, 17, 2, 63), (2, 64, 1, 64), (2, 65, 2, 257), (1, 300, 1, 5),
                                          (5, 33, 1, 1000)])
