@@ -1,9 +1,10 @@
 // Batched GEMM for gfx950: D = alpha * A @ B + beta * C.
 //
-// * gemm_mfma_kernel: 64x64x16 block tile, 256 threads = 4 waves of 64 in a
+// * gemm_mfma_kernel: 64x64 block tile, 256 threads = 4 waves of 64 in a
 //   2x2 arrangement, each wave owning a 32x32 sub-tile as 2x2 MFMA 16x16x4
 //   blocks (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32).  Complex types
-//   run 4 real MFMAs per k-step on planar (re/im split) LDS tiles.
+//   run 4 real MFMAs per k-step (complex64: 3) on planar (re/im split) LDS
+//   tiles.
 // * N <= 16 (several right-hand sides): the same kernel with the four waves
 //   stacked along M, one 16-wide MFMA column block.
 // * gemm_skinny_kernel: N <= 2 (down-pass / leaf-apply GEMV shapes).  One
@@ -16,6 +17,25 @@
 
 namespace hps {
 
+// The 64 x 64 tile of a type: K tiles of 8 keep the registers (and LDS) for one
+// workgroup more per CU than tiles of 16 do, except for float32, whose
+// accumulators are small anyway (float64 48 against 46 TFLOP/s, complex128 62 / 60,
+// complex64 138 / 134, float32 72 / 76 on 1024 x 24576 x 128 products).
+template <typename T>
+struct Tile64 {
+  static constexpr int BK = std::is_same<T, float>::value ? 16 : 8;
+  static constexpr int MINB = std::is_same<T, c128>::value ? 4 : 5;
+  static constexpr bool K3M = std::is_same<T, c64>::value;
+};
+
+// every byte offset inside a tile fits 32 bits: 64 rows of A, C or D (TA and B:
+// the rows that one pass of the threads covers, at most 16)
+template <typename T>
+static bool offsets_fit(const GemmArgs<T>& a) {
+  const double lim = 4294967296.0 / sizeof(T) / 65.0;
+  return a.lda < lim && a.ldb < lim && a.ldc < lim && a.ldd < lim;
+}
+
 template <typename T>
 hipError_t gemm(const GemmArgs<T>& a, hipStream_t s) {
   if (a.M <= 0 || a.N <= 0 || a.batch <= 0) return hipSuccess;
@@ -25,6 +45,8 @@ hipError_t gemm(const GemmArgs<T>& a, hipStream_t s) {
   const double flops = 2.0 * a.M * a.N * (double)a.K * a.batch * flop_mult<T>();
   const double bytes = sizeof(T) * ((double)a.M * a.K * (a.sA ? a.batch : 1) + (double)a.K * a.N * (a.sB ? a.batch : 1) +
                                     (double)a.M * a.N * a.batch * (a.beta != 0.0 ? 2 : 1));
+  using TL = Tile64<T>;
+  const bool fit = offsets_fit(a);
   if (a.transA) {
     // op(A) = A^H: the adjoint products (S^H, B^H, Y^H, D12^H ... and the
     // conjugate-transposed triangular updates)
@@ -36,17 +58,21 @@ hipError_t gemm(const GemmArgs<T>& a, hipStream_t s) {
         hipLaunchKernelGGL((gemv_conjt_kernel<T, 1>), grid, dim3(256), 0, s, a);
       else
         hipLaunchKernelGGL((gemv_conjt_kernel<T, 2>), grid, dim3(256), 0, s, a);
-    } else if (a.N <= 16) {
+    } else if (a.N <= 16 && fit) {
       static const std::string nm = std::string("gemm_mfma_64x16_conjt<") + tname<T>() + ">";
       prof::Scope ps(s, nm.c_str(), flops, bytes);
       dim3 grid((unsigned)ceil_div(a.M, 64), gy);
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 1, 1, 4, 4, true>), grid, dim3(256), 0, s, a, 1);
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 1, 1, 4, 16, 4, true>), grid, dim3(256), 0, s, a, 1);
     } else {
       static const std::string nm = std::string("gemm_mfma_64x64_conjt<") + tname<T>() + ">";
       prof::Scope ps(s, nm.c_str(), flops, bytes);
       int tiles_n = ceil_div(a.N, 64), tiles_m = ceil_div(a.M, 64);
       dim3 grid((unsigned)(tiles_m * tiles_n), gy);
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 2, 3, 2, true>), grid, dim3(256), 0, s, a, tiles_n);
+      if (fit)
+        hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 2, TL::MINB, TL::BK, 2, true>), grid, dim3(256), 0, s, a, tiles_n);
+      else
+        hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 2, 2, TL::BK, 2, true, false, size_t>), grid, dim3(256), 0, s, a,
+                           tiles_n);
     }
     return hipGetLastError();
   }
@@ -71,19 +97,19 @@ hipError_t gemm(const GemmArgs<T>& a, hipStream_t s) {
     } else {
       hipLaunchKernelGGL((gemm_skinny_kernel<T, 2>), grid, dim3(256), 0, s, a);
     }
-  } else if (a.N <= 16) {
+  } else if (a.N <= 16 && fit) {
     // one 16-wide MFMA column block; the four waves stack along M (64-row tiles)
     static const std::string nm = std::string("gemm_mfma_64x16<") + tname<T>() + ">";
     prof::Scope ps(s, nm.c_str(), flops, bytes);
     int tiles_m = ceil_div(a.M, 64);
     dim3 grid((unsigned)tiles_m, gy);
-    hipLaunchKernelGGL((gemm_mfma_kernel<T, 1, 1, 4, 4>), grid, dim3(256), 0, s, a, 1);
+    hipLaunchKernelGGL((gemm_mfma_kernel<T, 1, 1, 4, 16, 4>), grid, dim3(256), 0, s, a, 1);
   } else {
     static const std::string nm64 = std::string("gemm_mfma_64x64<") + tname<T>() + ">";
     static const std::string nm32 = std::string("gemm_mfma_64x32<") + tname<T>() + ">";
     static const std::string nmk32 = std::string("gemm_k32<") + tname<T>() + ">";
     static const std::string nmtri = std::string("trsm_k32<") + tname<T>() + ">";
-    if (a.K <= 32) {
+    if (a.K <= 32 && a.N > 16) {
       prof::Scope ps(s, (a.triA ? nmtri : nmk32).c_str(), flops, bytes);
       if (a.M <= 32) {
         // 32 x 64 tiles (the triangular block steps and other 32-row products)
@@ -102,24 +128,23 @@ hipError_t gemm(const GemmArgs<T>& a, hipStream_t s) {
       }
       return hipGetLastError();
     }
-    const bool short_k = a.K <= 64 && a.N <= 256;
+    const bool short_k = a.K <= 64 && a.N <= 256 && fit;
     prof::Scope ps(s, (short_k ? nm32 : nm64).c_str(), flops, bytes);
-    // Tile choice measured on MI355X over the solver's shapes: 64x64 tiles
-    // with 3 workgroups per CU for general shapes (2 for complex128); 64x32
-    // tiles with 2 per CU for the short-K batched updates of the leaf LU and
-    // solves.  128-wide tiles measured slower (one workgroup per CU).
+    // 64x32 tiles for the short-K batched products of small matrices, 64x64
+    // tiles otherwise
     if (short_k) {
       int tiles_n = ceil_div(a.N, 32), tiles_m = ceil_div(a.M, 64);
       dim3 grid((unsigned)(tiles_m * tiles_n), gy);
-      hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 1, 2>), grid, dim3(256), 0, s, a, tiles_n);
+      hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 1, 4, 16>), grid, dim3(256), 0, s, a, tiles_n);
     } else {
       int tiles_n = ceil_div(a.N, 64), tiles_m = ceil_div(a.M, 64);
       dim3 grid((unsigned)(tiles_m * tiles_n), gy);
-      if constexpr (sizeof(T) == 16)  // 3 workgroups per CU would force complex128 to spill registers
-        hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 2, 2>), grid, dim3(256), 0, s, a, tiles_n);
-      else
-        hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 2, 3, 2, false, is_cplx<T>::value>), grid, dim3(256), 0, s, a,
+      if (fit)
+        hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 2, TL::MINB, TL::BK, 2, false, TL::K3M>), grid, dim3(256), 0, s, a,
                            tiles_n);
+      else
+        hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 2, 2, TL::BK, 2, false, TL::K3M, size_t>), grid, dim3(256), 0, s,
+                           a, tiles_n);
     }
   }
   return hipGetLastError();
@@ -131,7 +156,7 @@ hipError_t gemm_grouped(const GemmArgs<T>& a, int n_blk, const int* blk, hipStre
   if (a.transA || a.triA) return hipErrorInvalidValue;
   // one launch when every group takes the 64 x 64 tile path (N > 256, K > 32);
   // otherwise one product per group
-  bool one = a.N > 256;
+  bool one = a.N > 256 && offsets_fit(a);
   for (int u = 0; u < n_blk && one; ++u) one = blk[4 * u + 3] > 32;
   // groups that write the same rows run one after another (each reads the
   // previous one's D as its C)
@@ -178,11 +203,9 @@ hipError_t gemm_grouped(const GemmArgs<T>& a, int n_blk, const int* blk, hipStre
     if (gr.start[gr.n] == 0) continue;  // blocks without rows: nothing to launch
     prof::Scope ps(s, nm.c_str(), flops, bytes);
     dim3 grid((unsigned)gr.start[gr.n], gy);
-    if constexpr (sizeof(T) == 16)
-      hipLaunchKernelGGL((gemm_mfma_grouped_kernel<T, 2, 2, 2, false>), grid, dim3(256), 0, s, a, gr, tiles_n);
-    else
-      hipLaunchKernelGGL((gemm_mfma_grouped_kernel<T, 2, 2, 3, is_cplx<T>::value>), grid, dim3(256), 0, s, a, gr,
-                         tiles_n);
+    using TL = Tile64<T>;
+    hipLaunchKernelGGL((gemm_mfma_grouped_kernel<T, 2, 2, TL::MINB, TL::BK, TL::K3M, unsigned>), grid, dim3(256), 0, s,
+                       a, gr, tiles_n);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

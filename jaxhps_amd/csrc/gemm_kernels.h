@@ -34,13 +34,6 @@ template <> __device__ __forceinline__ float make_val<float>(float re, float) { 
 template <> __device__ __forceinline__ c128 make_val<c128>(double re, double im) { return c128{re, im}; }
 template <> __device__ __forceinline__ c64 make_val<c64>(float re, float im) { return c64{re, im}; }
 
-constexpr int GBK = 16;
-
-// Block tile (WR*TM*16) x (WC*TN*16) x 16 with WC = 4 / WR; 4 waves in a
-// WR x WC arrangement, each owning TM x TN MFMA 16x16 blocks.  WR = 2 is the
-// square layout; WR = 4 stacks the waves along M for N <= 16 (the
-// multi-right-hand-side products).  The next K-tile is fetched from global
-// memory into registers while the current one is multiplied out of LDS.
 // Workgroups are handed to the 8 XCDs round-robin by linear id, and each
 // XCD has its own L2.  For a batch (grid y >= 2) xcd_block gives the
 // workgroup the (x, y) block of the linear id (id % 8) * (W / 8) + id / 8
@@ -61,12 +54,43 @@ template <typename T> __device__ __forceinline__ T s_conj(T x) { return x; }
 template <> __device__ __forceinline__ c128 s_conj<c128>(c128 x) { return c128{x.re, -x.im}; }
 template <> __device__ __forceinline__ c64 s_conj<c64>(c64 x) { return c64{x.re, -x.im}; }
 
+// element at a byte offset from a wave-uniform base: with a 32-bit offset the
+// load takes the base from scalar registers and one vector register an address
+template <typename T, typename O>
+__device__ __forceinline__ T load_at(const T* base, O off) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + off);
+}
+template <typename T, typename O>
+__device__ __forceinline__ void store_at(T* base, O off, T v) {
+  *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + off) = v;
+}
+
+// Block tile (WR*TM*16) x (WC*TN*16) x BK with WC = 4 / WR; 4 waves in a
+// WR x WC arrangement, each owning TM x TN MFMA 16x16 blocks.  WR = 2 is the
+// square layout; WR = 4 stacks the waves along M for N <= 16 (the
+// multi-right-hand-side products).  The next K tile is fetched from global
+// memory into registers while the current one is multiplied out of LDS.
+//
+// Bound by the matrix cores where enough workgroups share a CU to cover each
+// other's loads and epilogues, so registers decide: a thread's addresses are
+// one 32-bit offset for B, C and D each (rows a uniform step apart) and one a
+// row for A; rows and columns past the edge repeat the last one instead of
+// being masked (they only reach results that are not stored); only the
+// last, partial K tile is masked.  With 64-bit indices and masks per element a
+// float64 64 x 64 tile took 149 registers (3 workgroups a CU), now 82 (5, K
+// tiles of 8).  TFLOP/s before / now, products of 4096 x 8192 x 4096 and (K =
+// 128, C added) 1024 x 24576 x 128: float64 51 / 64, 35 / 48; float32 85 / 110,
+// 55 / 76; complex128 65 / 72, 50 / 62; complex64 149 / 165, 101 / 138.  Tiles
+// of 128 x 64 and 128 x 128 gain at most 4 % on the first shape and lose 10 to
+// 40 % on the solver's own K = 128 ones.
+//
 // TA: op(A) = A^H with A stored K x M; the tile load then walks M fastest so
 // the reads stay coalesced.
 // K3M (complex only): three real products per complex one (P1 = Ar Br,
 // P2 = Ai Bi, P3 = (Ar + Ai)(Br + Bi); Re = P1 - P2, Im = P3 - P1 - P2), a
 // quarter fewer MFMAs for one more accumulator per block.
-template <typename T, int TM, int TN, int WR, bool TA, bool K3M>
+// O: type of the byte offsets, unsigned unless a tile's rows span 4 GiB.
+template <typename T, int TM, int TN, int WR, int BK, bool TA, bool K3M, typename O>
 __device__ __forceinline__ void gemm_mfma_tile(const GemmArgs<T>& p, int bx, int by, int tiles_n) {
   using R = typename real_of<T>::type;
   using M = Mfma<R>;
@@ -74,78 +98,90 @@ __device__ __forceinline__ void gemm_mfma_tile(const GemmArgs<T>& p, int bx, int
   constexpr bool CPLX = is_cplx<T>::value;
   constexpr int WC = 4 / WR;
   static_assert(WR * WC == 4, "four waves per block");
+  static_assert(!K3M || CPLX, "three-product form is for complex types");
   constexpr int BM = WR * TM * 16, BN = WC * TN * 16;
-  static_assert((BM * GBK) % 256 == 0 && (GBK * BN) % 256 == 0, "tile loads must cover the block evenly");
-  constexpr int LA = BM * GBK / 256, LB = GBK * BN / 256;
-  __shared__ R As_re[GBK][BM + 1];
-  __shared__ R Bs_re[GBK][BN + 1];
-  __shared__ R As_im[CPLX ? GBK : 1][CPLX ? BM + 1 : 1];
-  __shared__ R Bs_im[CPLX ? GBK : 1][CPLX ? BN + 1 : 1];
+  static_assert((BM * BK) % 256 == 0 && (BK * BN) % 256 == 0 && 256 % BM == 0 && 256 % BN == 0,
+                "tile loads must cover the block evenly");
+  // each thread loads LA elements of A, RA rows (TA: of K) apart, and LB of B
+  constexpr int LA = BM * BK / 256, LB = BK * BN / 256, RA = TA ? 256 / BM : 256 / BK, RB = 256 / BN;
+  __shared__ R As_re[BK][BM + 1];
+  __shared__ R Bs_re[BK][BN + 1];
+  __shared__ R As_im[CPLX ? BK : 1][CPLX ? BM + 1 : 1];
+  __shared__ R Bs_im[CPLX ? BK : 1][CPLX ? BN + 1 : 1];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wr = wave / WC, wc = wave % WC;
-  const int tm = bx / tiles_n, tn = bx % tiles_n;
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = bx / tiles_n * BM, n0 = bx % tiles_n * BN;
   const int li = lane & 15, lk = lane >> 4;
+  const int ar = TA ? tid % BM : tid / BK, ac = TA ? tid / BM : tid % BK;  // row and K index of the first A element
+  const int br = tid / BN, bc = tid % BN;
+  O va[TA ? 1 : LA];
+  if constexpr (TA) {
+    va[0] = ((O)ac * (O)p.lda + (m0 + ar < p.M ? ar : p.M - 1 - m0)) * sizeof(T);
+  } else {
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {
+      const int r = ar + RA * i;
+      va[i] = ((O)(m0 + r < p.M ? r : p.M - 1 - m0) * (O)p.lda + ac) * sizeof(T);
+    }
+  }
+  const O vb = ((O)br * (O)p.ldb + (n0 + bc < p.N ? bc : p.N - 1 - n0)) * sizeof(T);
 
   for (int b = by; b < p.batch; b += gridDim.y) {
-    const T* A = p.A + batch_offset(b, p.nin, p.sA, p.sA2);
-    const T* B = p.B + batch_offset(b, p.nin, p.sB, p.sB2);
-    static_assert(!K3M || CPLX, "three-product form is for complex types");
+    const T* A = p.A + batch_offset(b, p.nin, p.sA, p.sA2) + (TA ? (long)m0 : (long)m0 * p.lda);
+    const T* B = p.B + batch_offset(b, p.nin, p.sB, p.sB2) + n0;
     acc_t acc_re[TM][TN], acc_im[TM][TN], acc_x[K3M ? TM : 1][K3M ? TN : 1];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         acc_re[i][j] = acc_t{0, 0, 0, 0};
-        acc_im[i][j] = acc_t{0, 0, 0, 0};
+        if constexpr (CPLX) acc_im[i][j] = acc_t{0, 0, 0, 0};
         if constexpr (K3M) acc_x[i][j] = acc_t{0, 0, 0, 0};
       }
     T ra[LA], rb[LB];
     auto fetch = [&](int k0) {
+      const T* Ak = A + (TA ? (long)k0 * p.lda : (long)k0);
+      const T* Bk = B + (long)k0 * p.ldb;
+      if (k0 + BK <= p.K) {
 #pragma unroll
-      for (int i = 0; i < LA; ++i) {
-        int e = tid + 256 * i;
-        if constexpr (TA) {
-          int r = e % BM, c = e / BM;
-          int gr = m0 + r, gc = k0 + c;
-          ra[i] = (gr < p.M && gc < p.K) ? s_conj(A[(long)gc * p.lda + gr]) : s_zero<T>();
-        } else {
-          int r = e >> 4, c = e & 15;
-          int gr = m0 + r, gc = k0 + c;
-          ra[i] = (gr < p.M && gc < p.K) ? A[(long)gr * p.lda + gc] : s_zero<T>();
-        }
+        for (int i = 0; i < LA; ++i) ra[i] = TA ? load_at(Ak + (long)(RA * i) * p.lda, va[0]) : load_at(Ak, va[TA ? 0 : i]);
+#pragma unroll
+        for (int i = 0; i < LB; ++i) rb[i] = load_at(Bk + (long)(RB * i) * p.ldb, vb);
+      } else {
+#pragma unroll
+        for (int i = 0; i < LA; ++i)
+          ra[i] = k0 + ac + (TA ? RA * i : 0) >= p.K ? s_zero<T>()
+                  : TA                               ? load_at(Ak + (long)(RA * i) * p.lda, va[0])
+                                                     : load_at(Ak, va[TA ? 0 : i]);
+#pragma unroll
+        for (int i = 0; i < LB; ++i)
+          rb[i] = k0 + br + RB * i < p.K ? load_at(Bk + (long)(RB * i) * p.ldb, vb) : s_zero<T>();
       }
+      if constexpr (TA) {
 #pragma unroll
-      for (int i = 0; i < LB; ++i) {
-        int e = tid + 256 * i;
-        int r = e / BN, c = e % BN;
-        int gr = k0 + r, gc = n0 + c;
-        rb[i] = (gr < p.K && gc < p.N) ? B[(long)gr * p.ldb + gc] : s_zero<T>();
+        for (int i = 0; i < LA; ++i) ra[i] = s_conj(ra[i]);
       }
     };
-    fetch(0);
-    for (int k0 = 0; k0 < p.K; k0 += GBK) {
+    if (p.K > 0) fetch(0);
+    for (int k0 = 0; k0 < p.K; k0 += BK) {
 #pragma unroll
       for (int i = 0; i < LA; ++i) {
-        int e = tid + 256 * i;
-        int r = TA ? e % BM : e >> 4, c = TA ? e / BM : e & 15;
+        const int r = TA ? ar : ar + RA * i, c = TA ? ac + RA * i : ac;
         As_re[c][r] = s_re(ra[i]);
         if constexpr (CPLX) As_im[c][r] = s_im(ra[i]);
       }
 #pragma unroll
       for (int i = 0; i < LB; ++i) {
-        int e = tid + 256 * i;
-        int r = e / BN, c = e % BN;
-        Bs_re[r][c] = s_re(rb[i]);
-        if constexpr (CPLX) Bs_im[r][c] = s_im(rb[i]);
+        Bs_re[br + RB * i][bc] = s_re(rb[i]);
+        if constexpr (CPLX) Bs_im[br + RB * i][bc] = s_im(rb[i]);
       }
       __syncthreads();
-      if (k0 + GBK < p.K) fetch(k0 + GBK);
+      if (k0 + BK < p.K) fetch(k0 + BK);
 #pragma unroll
-      for (int kk = 0; kk < GBK; kk += 4) {
+      for (int kk = 0; kk < BK; kk += 4) {
         R a_re[TM], b_re[TN], a_im[TM], b_im[TN];
 #pragma unroll
         for (int t = 0; t < TM; ++t) {
@@ -197,31 +233,57 @@ __device__ __forceinline__ void gemm_mfma_tile(const GemmArgs<T>& p, int bx, int
         }
     }
 
-    const T* C = p.C ? p.C + batch_offset(b, p.nin, p.sC, p.sC2) : nullptr;
-    T* D = p.D + batch_offset(b, p.nin, p.sD, p.sD2);
+    // the lane's first element of its wave's tile; the others lie uniform steps away
+    const int r0 = wr * (BM / WR) + M::out_row(lk, 0), c0 = wc * (BN / WC) + li;
+    T* D = p.D + batch_offset(b, p.nin, p.sD, p.sD2) + (long)m0 * p.ldd + n0;
+    const O vd = ((O)r0 * (O)p.ldd + c0) * sizeof(T);
+    if (p.beta != 0.0) {
+      const T* C = p.C + batch_offset(b, p.nin, p.sC, p.sC2) + (long)m0 * p.ldc + n0;
+      const O vc = ((O)r0 * (O)p.ldc + c0) * sizeof(T);
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < TM; ++i) {
+        // a row of blocks at a time: its C loads are all in flight together
+        T rc[TN][4];
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          int row = m0 + wr * (BM / WR) + i * 16 + M::out_row(lk, r);
-          int col = n0 + wc * (BN / WC) + j * 16 + li;
-          if (row < p.M && col < p.N) {
-            T v = make_val<T>(acc_re[i][j][r], CPLX ? acc_im[i][j][r] : R(0));
-            v = s_scale(v, p.alpha);
-            if (p.beta != 0.0) v = s_add(v, s_scale(C[(long)row * p.ldc + col], p.beta));
-            D[(long)row * p.ldd + col] = v;
+          for (int r = 0; r < 4; ++r) {
+            const int dr = i * 16 + M::out_row(0, r);
+            rc[j][r] = m0 + r0 + dr < p.M && n0 + c0 + j * 16 < p.N ? load_at(C + (long)dr * p.ldc + j * 16, vc)
+                                                                   : s_zero<T>();
           }
-        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int dr = i * 16 + M::out_row(0, r);
+            const T v = s_scale(make_val<T>(acc_re[i][j][r], CPLX ? acc_im[i][j][r] : R(0)), p.alpha);
+            if (m0 + r0 + dr < p.M && n0 + c0 + j * 16 < p.N)
+              store_at(D + (long)dr * p.ldd + j * 16, vd, s_add(v, s_scale(rc[j][r], p.beta)));
+          }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int dr = i * 16 + M::out_row(0, r);
+            const T v = s_scale(make_val<T>(acc_re[i][j][r], CPLX ? acc_im[i][j][r] : R(0)), p.alpha);
+            if (m0 + r0 + dr < p.M && n0 + c0 + j * 16 < p.N) store_at(D + (long)dr * p.ldd + j * 16, vd, v);
+          }
+    }
   }
 }
 
-template <typename T, int TM, int TN, int MINB = 1, int WR = 2, bool TA = false, bool K3M = false>
+// MINB: workgroups per CU that the register budget is set for
+template <typename T, int TM, int TN, int MINB, int BK, int WR = 2, bool TA = false, bool K3M = false,
+          typename O = unsigned>
 __global__ __launch_bounds__(256, MINB) void gemm_mfma_kernel(GemmArgs<T> p, int tiles_n) {
   int bx, by;
   xcd_block(bx, by);
-  gemm_mfma_tile<T, TM, TN, WR, TA, K3M>(p, bx, by, tiles_n);
+  gemm_mfma_tile<T, TM, TN, WR, BK, TA, K3M, O>(p, bx, by, tiles_n);
 }
 
 // Several products in one launch: group g is the product of rows
@@ -238,7 +300,7 @@ struct GemmGroups {
   int r0[GEMM_MAX_GROUPS] = {}, nr[GEMM_MAX_GROUPS] = {}, k0[GEMM_MAX_GROUPS] = {}, nk[GEMM_MAX_GROUPS] = {};
 };
 
-template <typename T, int TM, int TN, int MINB, bool K3M>
+template <typename T, int TM, int TN, int MINB, int BK, bool K3M, typename O>
 __global__ __launch_bounds__(256, MINB) void gemm_mfma_grouped_kernel(GemmArgs<T> p, GemmGroups g, int tiles_n) {
   int bx, by;
   xcd_block(bx, by);
@@ -251,7 +313,7 @@ __global__ __launch_bounds__(256, MINB) void gemm_mfma_grouped_kernel(GemmArgs<T
   p.B += (long)g.k0[gi] * p.ldb;
   if (p.C) p.C += (long)g.r0[gi] * p.ldc;
   p.D += (long)g.r0[gi] * p.ldd;
-  gemm_mfma_tile<T, TM, TN, 2, false, K3M>(p, bx, by, tiles_n);
+  gemm_mfma_tile<T, TM, TN, 2, BK, false, K3M, O>(p, bx, by, tiles_n);
 }
 
 // Short-K updates (K <= 32: the 32-wide steps of the blocked LU and solves):

@@ -128,3 +128,28 @@ def test_conjt_gemv(gpu, dtype, batch, M, N, K):
     ref = a.conj().transpose(0, 2, 1) @ b + c
     bound = 4 * (K + 2) * EPS[dtype] * (np.abs(a).transpose(0, 2, 1) @ np.abs(b) + np.abs(c))
     assert (np.abs(out.cpu().numpy() - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("conjt", [False, True])
+def test_gemm_wide_rows(gpu, conjt):
+    """Rows so far apart that a tile's byte offsets pass 4 GiB (8.3 M float64
+    elements) take the 64-bit offsets; against the packed product."""
+    from jaxhps_amd import _lib
+
+    print(f"gemm wide rows conjt={conjt}", flush=True)
+    lib, h = _lib.load_library(), _lib.handle()
+    M, N, K, ld = 70, 20, 40, 8_300_000
+    rows, cols = (K, M) if conjt else (M, K)
+    g = torch.Generator(device=gpu).manual_seed(3)
+    A = torch.empty(rows * ld, dtype=torch.float64, device=gpu).as_strided((rows, cols), (ld, 1))
+    A.normal_(generator=g)
+    B = torch.randn(K, N, generator=g, dtype=torch.float64, device=gpu)
+    out = torch.empty(M, N, dtype=torch.float64, device=gpu)
+    fn = lib.hps_gemm_batched_conjt if conjt else lib.hps_gemm_batched
+    rc = fn(h, _lib.dtype_code(A.dtype), M, N, K, 1.0, A.data_ptr(), ld, 0, _lib.ptr(B), N, 0, 0.0, None, N, 0,
+            _lib.ptr(out), N, 0, 1)
+    _lib.check(rc, h, "gemm")
+    a = A.cpu().numpy()
+    ref = (a.T if conjt else a) @ B.cpu().numpy()
+    bound = 2 * K * 2.0**-53 * (np.abs(a.T if conjt else a) @ np.abs(B.cpu().numpy()))
+    assert (np.abs(out.cpu().numpy() - ref) <= bound).all()
