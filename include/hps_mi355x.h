@@ -103,6 +103,29 @@ int hps_leaf_solve(hps_handle_t h, int dtype, int kind, int nl, int n, int nb, i
                    const void* G, const void* source, void* Y, void* T, void* v, void* hvec, void* lu, int* perm,
                    void* dinv, int* info, void* ws, size_t ws_bytes);
 
+/* ItI leaf stage for real coefficients by static condensation: the interior
+ * block A_ii is factored in real arithmetic, the boundary system
+ * S = G_b - G_i A_ii^{-1} A_ib in complex.  dtype is the complex type; e is its
+ * real type.
+ *   coeffs (ncoef, nl, n), diffops (nops, n, n): e
+ *   GQ (nb + nq, n - nb): e, the interior columns of G and QH (real)
+ *   Gb (nb, nb), Qb (nq, nb): complex, their boundary columns;  P (nb, nq)
+ *   source (nl, n, nsrc) or NULL
+ * Outputs Y, T, v, h as hps_leaf_solve;  alu (nl, n-nb, n): e, [A_ib | LU(A_ii)]
+ *   with aperm, adinv;  X (nl, n-nb, nb + 2 nsrc): e, A_ii^{-1} [A_ib | f_i]
+ *   (the sources' columns as (re, im) pairs);  slu (nl, nb, nb) = LU(S) with
+ *   sperm, sdinv;  info[l] = -1 where the condensation is not to be used (a
+ *   rejected factorisation, or an entry of X_b above 16: A_ii close to a
+ *   Dirichlet eigenvalue), and the caller takes hps_leaf_solve instead.
+ * Replaces local_solve_stage_uniform_2D_ItI + get_ItI
+ *   (local_solve/_uniform_2D_ItI.py:10-193), which inverts B. */
+size_t hps_leaf_condensed_workspace(int dtype, int nl, int n, int nb, int nq, int nsrc);
+int hps_leaf_condensed(hps_handle_t h, int dtype, int nl, int n, int nb, int nq, int nsrc, int ncoef,
+                       const int* coef_ops, const void* coeffs, const void* diffops, const void* GQ, const void* Gb,
+                       const void* Qb, const void* P, const void* source, void* Y, void* T, void* v, void* hvec,
+                       void* alu, int* aperm, void* adinv, void* X, void* slu, int* sperm, void* sdinv, int* info,
+                       void* ws, size_t ws_bytes);
+
 /* ---- merge stage (one tree level) ------------------------------------------
  * nm merges of nc children each (4 in 2D, 8 in 3D); children's maps
  * T_in (nm*nc, nec, nec) and data h_in (nm*nc, nec, nsrc).

@@ -242,3 +242,28 @@ class PDEProblem:
                 d["Q"] = dev(self.Q)
             self._dev_cache[key] = d
         return self._dev_cache[key]
+
+    def condensed_ops(self, device, dtype):
+        """The ItI leaf operators split at the boundary for hps_leaf_condensed
+        (dtype complex): real differentiation operators and interior columns of
+        G and QH, complex boundary columns.  None where the interior columns
+        are not real."""
+        key = ("condensed", str(device), dtype)
+        if key not in self._dev_cache:
+            G, QH = np.asarray(self.G), np.asarray(self.QH)
+            nb = self.P.shape[0]
+            GQ = np.concatenate([G[:, nb:], QH[:, nb:]])
+            if np.any(GQ.imag):
+                self._dev_cache[key] = None
+            else:
+                real = torch.float64 if dtype == torch.complex128 else torch.float32
+
+                def dev(x, dt):
+                    return torch.as_tensor(np.ascontiguousarray(x)).to(device=device, dtype=dt)
+
+                self._dev_cache[key] = {
+                    "diffops": dev(np.stack([getattr(self, n) for n in self.operator_names()]), real),
+                    "GQ": dev(GQ.real, real), "Gb": dev(G[:, :nb], dtype), "Qb": dev(QH[:, :nb], dtype),
+                    "P": dev(self.P, dtype),
+                }
+        return self._dev_cache[key]

@@ -72,6 +72,18 @@ class LeafResult:
     # iti_row_scale; 1 for DtN.
     row_scale: Optional[torch.Tensor] = None
     nb: int = 0
+    condensed: Optional[Condensed] = None
+
+
+@dataclass
+class Condensed:
+    """Interior factors of condensed ItI leaves (hps_leaf_condensed); the
+    leaf's lu, perm and dinv then factor the boundary system."""
+    alu: torch.Tensor   # (nl, ni, n) real: [A_ib | LU(A_ii)]
+    perm: torch.Tensor
+    dinv: torch.Tensor
+    X: torch.Tensor     # (nl, ni, nb + 2 nsrc) real: A_ii^{-1} [A_ib | f_i]
+    Gi: torch.Tensor    # (nb, ni) real: interior columns of G
 
 
 def iti_row_scale(pde, coeffs, clist, device):
@@ -139,15 +151,6 @@ def leaf_solve(pde, kind: int, dtype, device, source=None, nsrc_zero=False, leaf
     if not clist:
         raise ValueError("PDEProblem has no coefficients")
     coef_ops = np.array([-1 if nm == "I" else names.index(nm) for nm, _ in clist], dtype=np.int32)
-    coeffs = torch.stack([to_device(a, device, dtype) for _, a in clist]).contiguous()
-    if leaf_half_sides is not None:
-        hs = np.asarray(leaf_half_sides, dtype=np.float64)
-        inv = torch.as_tensor(1.0 / hs).to(device)
-        inv2 = torch.as_tensor(1.0 / (hs * hs)).to(device)
-        for k, (nm, _) in enumerate(clist):
-            order = 0 if nm == "I" else len(nm) - 2
-            if order:
-                scale_batched(coeffs[k], inv if order == 1 else inv2)
     if nsrc_zero:
         nsrc = 0
         src = None
@@ -158,6 +161,19 @@ def leaf_solve(pde, kind: int, dtype, device, source=None, nsrc_zero=False, leaf
         else:
             nsrc = source.shape[-1]
             src = source
+    if kind == HPS_KIND_ITI and not is_complex_input(*[a for _, a in clist]):
+        res = _leaf_condensed(pde, dtype, device, clist, coef_ops, src, nsrc)
+        if res is not None:
+            return res
+    coeffs = torch.stack([to_device(a, device, dtype) for _, a in clist]).contiguous()
+    if leaf_half_sides is not None:
+        hs = np.asarray(leaf_half_sides, dtype=np.float64)
+        inv = torch.as_tensor(1.0 / hs).to(device)
+        inv2 = torch.as_tensor(1.0 / (hs * hs)).to(device)
+        for k, (nm, _) in enumerate(clist):
+            order = 0 if nm == "I" else len(nm) - 2
+            if order:
+                scale_batched(coeffs[k], inv if order == 1 else inv2)
     nrows = n - nb if kind == HPS_KIND_DTN else n
     Y = torch.empty((nl, n, nq), dtype=dtype, device=device)
     T = torch.empty((nl, nq, nq), dtype=dtype, device=device)
@@ -200,6 +216,45 @@ def leaf_solve(pde, kind: int, dtype, device, source=None, nsrc_zero=False, leaf
         if hv is not None:
             scale_batched(hv, inv)
     return LeafResult(Y, T, v, hv, lu, perm, dinv, info, kind, row_scale, nb)
+
+
+def _leaf_condensed(pde, dtype, device, clist, coef_ops, src, nsrc) -> Optional[LeafResult]:
+    """ItI leaf stage with real coefficients by static condensation; None
+    where a leaf rejects it (its interior problem is close to singular)."""
+    ops = pde.condensed_ops(device, dtype)
+    if ops is None:
+        return None
+    lib = load_library()
+    h = _lib.handle()
+    nl = pde.domain.n_leaves
+    nb, nq = ops["P"].shape
+    n = pde.domain.p**2
+    ni = n - nb
+    rdt = real_dtype(dtype)
+    coeffs = torch.stack([to_device(a, device, rdt) for _, a in clist]).contiguous()
+
+    def empty(*shape, dt=dtype):
+        return torch.empty(shape, dtype=dt, device=device)
+
+    Y, T = empty(nl, n, nq), empty(nl, nq, nq)
+    v = empty(nl, n, nsrc) if nsrc else None
+    hv = empty(nl, nq, nsrc) if nsrc else None
+    alu, aperm = empty(nl, ni, n, dt=rdt), empty(nl, ni, dt=torch.int32)
+    adinv, X = empty(nl, _lib.dinv_size(ni), dt=rdt), empty(nl, ni, nb + 2 * nsrc, dt=rdt)
+    slu, sperm, sdinv = empty(nl, nb, nb), empty(nl, nb, dt=torch.int32), empty(nl, _lib.dinv_size(nb))
+    info = empty(nl, dt=torch.int32)
+    ws = workspace(lib.hps_leaf_condensed_workspace(dtype_code(dtype), nl, n, nb, nq, nsrc), device)
+    rc = lib.hps_leaf_condensed(
+        h, dtype_code(dtype), nl, n, nb, nq, nsrc, len(clist), coef_ops.ctypes.data_as(ctypes.c_void_p), ptr(coeffs),
+        ptr(ops["diffops"]), ptr(ops["GQ"]), ptr(ops["Gb"]), ptr(ops["Qb"]), ptr(ops["P"]), ptr(src), ptr(Y), ptr(T),
+        ptr(v), ptr(hv), ptr(alu), ptr(aperm), ptr(adinv), ptr(X), ptr(slu), ptr(sperm), ptr(sdinv), ptr(info), ptr(ws),
+        ws.numel(),
+    )
+    check(rc, h, "hps_leaf_condensed")
+    if bool((info < 0).any()):
+        return None
+    return LeafResult(Y, T, v, hv, slu, sperm, sdinv, info, HPS_KIND_ITI, None, nb,
+                      Condensed(alu, aperm, adinv, X, ops["GQ"][:nb]))
 
 
 @dataclass
@@ -395,6 +450,8 @@ def leaf_apply_inverse(leaf: LeafResult, rhs):
     """v = (leaf operator)^{-1} rhs for a full collocation right-hand side
     rhs (n_leaves, n, nsrc): DtN solves the interior rows with A_ii (v is zero
     on the boundary); ItI solves with B = [G; A_int]."""
+    if leaf.condensed is not None:
+        return _apply_inverse_condensed(leaf, rhs)
     nl, nrows, n = leaf.lu.shape
     nsrc = rhs.shape[-1]
     if leaf.kind == HPS_KIND_DTN:
@@ -409,6 +466,47 @@ def leaf_apply_inverse(leaf: LeafResult, rhs):
     X = torch.empty_like(R)
     getrs_into(n, leaf.lu, 0, n, n * n, leaf.perm, leaf.dinv, R, X)
     return X
+
+
+def at(t, offset=0):
+    """Device address of a tensor's element `offset` (in its own elements)."""
+    return ctypes.c_void_p(t.data_ptr() + offset * t.element_size())
+
+
+def gemm_at(dtype, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, batch, conjt=False):
+    """hps_gemm_batched (conjt: op(A) = A^H, A stored K x M) on device addresses."""
+    lib = load_library()
+    hd = _lib.handle()
+    fn = lib.hps_gemm_batched_conjt if conjt else lib.hps_gemm_batched
+    check(fn(hd, dtype_code(dtype), M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, D, ldd, sD, batch), hd,
+          "hps_gemm_batched")
+
+
+def _apply_inverse_condensed(leaf: LeafResult, rhs):
+    """B^{-1} rhs through the condensed factors: w = A_ii^{-1} r_i,
+    u_b = S^{-1}(r_b - G_i w), u_i = w - X_b u_b.  The real factors take a
+    complex right-hand side as twice as many real columns."""
+    lib = load_library()
+    hd = _lib.handle()
+    c = leaf.condensed
+    rhs = rhs.contiguous()
+    nl, n, w = rhs.shape
+    nb, ni = c.Gi.shape
+    dt, rdt = rhs.dtype, c.alu.dtype
+    w2, wr = 2 * w, c.X.shape[2]
+    out = torch.empty_like(rhs)
+    t = torch.empty((nl, nb, w), dtype=dt, device=rhs.device)
+    rc = lib.hps_getrs_batched(hd, dtype_code(rdt), ni, w2, at(c.alu, nb), n, ni * n, ptr(c.perm), ptr(c.dinv),
+                               at(rhs, nb * w), w2, n * w2, at(out, nb * w), w2, n * w2, nl)
+    check(rc, hd, "hps_getrs_batched")
+    gemm_at(rdt, nb, w2, ni, -1.0, ptr(c.Gi), ni, 0, at(out, nb * w), w2, n * w2, 1.0, at(rhs), w2, n * w2, at(t), w2,
+            nb * w2, nl)
+    rc = lib.hps_getrs_batched(hd, dtype_code(dt), nb, w, ptr(leaf.lu), nb, nb * nb, ptr(leaf.perm), ptr(leaf.dinv),
+                               ptr(t), w, nb * w, at(out), w, n * w, nl)
+    check(rc, hd, "hps_getrs_batched")
+    gemm_at(rdt, ni, w2, nb, -1.0, ptr(c.X), wr, ni * wr, at(out), w2, n * w2, 1.0, at(out, nb * w), w2, n * w2,
+            at(out, nb * w), w2, n * w2, nl)
+    return out
 
 
 def up_level(h_in, lvl: MergeLevel, inj=None, want_h=True):

@@ -40,7 +40,7 @@ import torch
 
 from . import _lib
 from ._lib import HPS_KIND_DTN, HPS_KIND_ITI, check, dtype_code, load_library, ptr, workspace
-from ._stages import to_device
+from ._stages import at, gemm_at, to_device
 
 
 def _gemm_conjt(A, lda, sA, M, K, B, ldb, sB, N, batch, C=None, beta=0.0, out=None):
@@ -68,6 +68,25 @@ def getrs_conjt(n, lu, lu_offset, lda, sA, perm, dinv, R):
                                      ptr(ws), ws.numel())
     check(rc, hd, "hps_getrs_batched_conjt")
     return X
+
+
+def _condensed_inverse_conjt(leaf, v):
+    """B^{-H} v through the condensed leaf factors (hps_leaf_condensed):
+    x_b = S^{-H}(v_b - X_b^T v_i), x_i = A_ii^{-T}(v_i - G_i^T x_b)."""
+    c = leaf.condensed
+    nl, n, w = v.shape
+    nb, ni = c.Gi.shape
+    rdt = c.alu.dtype
+    w2, wr = 2 * w, c.X.shape[2]
+    b = torch.empty((nl, nb, w), dtype=v.dtype, device=v.device)
+    gemm_at(rdt, nb, w2, ni, -1.0, ptr(c.X), wr, ni * wr, at(v, nb * w), w2, n * w2, 1.0, at(v), w2, n * w2, at(b), w2,
+            nb * w2, nl, conjt=True)
+    xb = getrs_conjt(nb, leaf.lu, 0, nb, nb * nb, leaf.perm, leaf.dinv, b)
+    y = torch.empty((nl, ni, w2), dtype=rdt, device=v.device)
+    gemm_at(rdt, ni, w2, nb, -1.0, ptr(c.Gi), ni, 0, at(xb), w2, nb * w2, 1.0, at(v, nb * w), w2, n * w2, at(y), w2,
+            ni * w2, nl, conjt=True)
+    xi = getrs_conjt(ni, c.alu, nb, n, ni * n, c.perm, c.dinv, y)
+    return torch.cat([xb, torch.view_as_complex(xi.view(nl, ni, w, 2))], dim=1)
 
 
 def _adjoint_down_level(gbar_children, S, tables):
@@ -139,7 +158,9 @@ def adjoint_lambda(pde_problem, G):
     Q = pde_problem.device_ops(dev, dt)["Q"]
     vbar = _gemm_conjt(Q, n, 0, n, nq, hbar.contiguous(), w, nq * w, w, nl, C=Gd, beta=1.0)
     _, nrows, _ = leaf.lu.shape
-    if leaf.kind == HPS_KIND_ITI:
+    if leaf.condensed is not None:
+        lam = _condensed_inverse_conjt(leaf, vbar)
+    elif leaf.kind == HPS_KIND_ITI:
         # the factors are of B' = diag(s, 1) B, so B^{-H} = diag(s, 1) B'^{-H}
         lam = getrs_conjt(n, leaf.lu, 0, n, n * n, leaf.perm, leaf.dinv, vbar)
         if leaf.row_scale is not None:

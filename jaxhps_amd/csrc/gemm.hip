@@ -128,17 +128,23 @@ hipError_t gemm(const GemmArgs<T>& a, hipStream_t s) {
       }
       return hipGetLastError();
     }
-    const bool short_k = a.K <= 64 && a.N <= 256 && fit;
-    prof::Scope ps(s, (short_k ? nm32 : nm64).c_str(), flops, bytes);
-    // 64x32 tiles for the short-K batched products of small matrices, 64x64
-    // tiles otherwise
-    if (short_k) {
+    const bool narrow = a.N <= 32 && fit;
+    prof::Scope ps(s, (narrow ? nm32 : nm64).c_str(), flops, bytes);
+    // 64x32 tiles where one covers all columns, 64x64 tiles otherwise
+    if (narrow) {
       int tiles_n = ceil_div(a.N, 32), tiles_m = ceil_div(a.M, 64);
       dim3 grid((unsigned)(tiles_m * tiles_n), gy);
       hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 1, 4, 16>), grid, dim3(256), 0, s, a, tiles_n);
     } else {
       int tiles_n = ceil_div(a.N, 64), tiles_m = ceil_div(a.M, 64);
       dim3 grid((unsigned)(tiles_m * tiles_n), gy);
+      if constexpr (!is_cplx<T>::value) {
+        if (a.sum2 && fit) {
+          hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 2, 4, TL::BK, 2, false, false, unsigned, true>), grid, dim3(256), 0,
+                             s, a, tiles_n);
+          return hipGetLastError();
+        }
+      }
       if (fit)
         hipLaunchKernelGGL((gemm_mfma_kernel<T, 2, 2, TL::MINB, TL::BK, 2, false, TL::K3M>), grid, dim3(256), 0, s, a,
                            tiles_n);

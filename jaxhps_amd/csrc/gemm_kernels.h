@@ -90,7 +90,8 @@ __device__ __forceinline__ void store_at(T* base, O off, T v) {
 // P2 = Ai Bi, P3 = (Ar + Ai)(Br + Bi); Re = P1 - P2, Im = P3 - P1 - P2), a
 // quarter fewer MFMAs for one more accumulator per block.
 // O: type of the byte offsets, unsigned unless a tile's rows span 4 GiB.
-template <typename T, int TM, int TN, int WR, int BK, bool TA, bool K3M, typename O>
+// SUM2: sums over 32 k at a time, added up at the end (GemmArgs::sum2).
+template <typename T, int TM, int TN, int WR, int BK, bool TA, bool K3M, typename O, bool SUM2 = false>
 __device__ __forceinline__ void gemm_mfma_tile(const GemmArgs<T>& p, int bx, int by, int tiles_n) {
   using R = typename real_of<T>::type;
   using M = Mfma<R>;
@@ -132,7 +133,8 @@ __device__ __forceinline__ void gemm_mfma_tile(const GemmArgs<T>& p, int bx, int
   for (int b = by; b < p.batch; b += gridDim.y) {
     const T* A = p.A + batch_offset(b, p.nin, p.sA, p.sA2) + (TA ? (long)m0 : (long)m0 * p.lda);
     const T* B = p.B + batch_offset(b, p.nin, p.sB, p.sB2) + n0;
-    acc_t acc_re[TM][TN], acc_im[TM][TN], acc_x[K3M ? TM : 1][K3M ? TN : 1];
+    static_assert(!SUM2 || (!CPLX && 32 % BK == 0), "two-level sums are for real types");
+    acc_t acc_re[TM][TN], acc_im[TM][TN], acc_x[K3M ? TM : 1][K3M ? TN : 1], sum[SUM2 ? TM : 1][SUM2 ? TN : 1];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -140,6 +142,7 @@ __device__ __forceinline__ void gemm_mfma_tile(const GemmArgs<T>& p, int bx, int
         acc_re[i][j] = acc_t{0, 0, 0, 0};
         if constexpr (CPLX) acc_im[i][j] = acc_t{0, 0, 0, 0};
         if constexpr (K3M) acc_x[i][j] = acc_t{0, 0, 0, 0};
+        if constexpr (SUM2) sum[i][j] = acc_t{0, 0, 0, 0};
       }
     T ra[LA], rb[LB];
     auto fetch = [&](int k0) {
@@ -222,6 +225,23 @@ __device__ __forceinline__ void gemm_mfma_tile(const GemmArgs<T>& p, int bx, int
         }
       }
       __syncthreads();
+      if constexpr (SUM2) {
+        if ((k0 + BK) % 32 == 0 || k0 + BK >= p.K) {
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+              sum[i][j] += acc_re[i][j];
+              acc_re[i][j] = acc_t{0, 0, 0, 0};
+            }
+        }
+      }
+    }
+    if constexpr (SUM2) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc_re[i][j] = sum[i][j];
     }
     if constexpr (K3M) {
 #pragma unroll
@@ -279,11 +299,11 @@ __device__ __forceinline__ void gemm_mfma_tile(const GemmArgs<T>& p, int bx, int
 
 // MINB: workgroups per CU that the register budget is set for
 template <typename T, int TM, int TN, int MINB, int BK, int WR = 2, bool TA = false, bool K3M = false,
-          typename O = unsigned>
+          typename O = unsigned, bool SUM2 = false>
 __global__ __launch_bounds__(256, MINB) void gemm_mfma_kernel(GemmArgs<T> p, int tiles_n) {
   int bx, by;
   xcd_block(bx, by);
-  gemm_mfma_tile<T, TM, TN, WR, BK, TA, K3M, O>(p, bx, by, tiles_n);
+  gemm_mfma_tile<T, TM, TN, WR, BK, TA, K3M, O, SUM2>(p, bx, by, tiles_n);
 }
 
 // Several products in one launch: group g is the product of rows

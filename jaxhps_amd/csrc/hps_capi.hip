@@ -391,11 +391,20 @@ int hps_getrs_batched(hps_handle_t h, int dtype, int n, int nrhs, const void* LU
 // ---------------------------------------------------------------------------
 // leaf solve
 // ---------------------------------------------------------------------------
+constexpr int LEAF_CHUNK = 8192;  // leaves whose block inverses are held at once
+
 size_t hps_leaf_workspace(int dtype, int kind, int nl, int n, int nb, int nq, int nsrc) {
   size_t es = dtype_size(dtype);
   int nrows = kind == HPS_KIND_DTN ? n - nb : n;
   size_t rhs = align_up((size_t)nl * nrows * (nq + nsrc) * es);
-  return 2 * rhs + align_up(getrf_scratch_bytes(nrows, nl));
+  size_t tot = 2 * rhs + align_up(getrf_scratch_bytes(nrows, nl));
+  if (kind == HPS_KIND_DTN) {
+    // the natural-order factorisation's block inverses, panels and integers
+    const int m = nl < LEAF_CHUNK ? nl : LEAF_CHUNK;
+    const LuPlan p = lu_plan_dense(nrows, nq + nsrc, m);
+    tot += align_up(lub_inv_elems(p, m) * es) + align_up(lub_tmp_elems(p, m) * es) + align_up(lub_scratch_bytes(p, m));
+  }
+  return tot;
 }
 
 template <typename T>
@@ -467,11 +476,34 @@ static int leaf_t(hps_handle_t h, int kind, int nl, int n, int nb, int nq, int n
 
   // 3. factor and solve
   T* Afac = kind == HPS_KIND_DTN ? lu + nb : lu;
-  HPS_CHECK_HIP(h, getrf_ws<T>(nrows, Afac, ld_lu, s_lu, perm, dinv, scratch, info, nl, s, h->leaf_nopiv));
-  if (kind == HPS_KIND_DTN) {
+  T* sol = X;
+  if (kind == HPS_KIND_DTN && h->leaf_nopiv) {
+    // natural order by blocks, the right-hand sides solved in place (X is
+    // scratch), LEAF_CHUNK leaves at a time
+    const int m = nl < LEAF_CHUNK ? nl : LEAF_CHUNK;
+    const LuPlan p = lu_plan_dense(nrows, w, m);
+    char* q = wp + align_up(getrf_scratch_bytes(nrows, nl));
+    T* inv = (T*)q;
+    q += align_up(lub_inv_elems(p, m) * es);
+    T* tmp = (T*)q;
+    q += align_up(lub_tmp_elems(p, m) * es);
+    const long sR = (long)nrows * w;
+    for (int l0 = 0; l0 < nl; l0 += LEAF_CHUNK) {
+      const int c = nl - l0 < LEAF_CHUNK ? nl - l0 : LEAF_CHUNK;
+      T* Al = Afac + (long)l0 * s_lu;
+      HPS_CHECK_HIP(h, lu_blocks_factor<T>(p, Al, ld_lu, s_lu, perm + (long)l0 * nrows,
+                                           dinv + (long)l0 * dinv_elems(nrows), inv, tmp, (int*)q, info + l0, c, s));
+      HPS_CHECK_HIP(h, lu_blocks_solve<T>(p, Al, ld_lu, s_lu, inv, R + l0 * sR, w, sR, X + l0 * sR, w, sR, w, false, c,
+                                          s));
+    }
+    sol = R;
+  } else {
+    HPS_CHECK_HIP(h, getrf_ws<T>(nrows, Afac, ld_lu, s_lu, perm, dinv, scratch, info, nl, s, h->leaf_nopiv));
+  }
+  if (kind == HPS_KIND_DTN && !h->leaf_nopiv) {
     HPS_CHECK_HIP(h, getrs_perm<T>(nrows, w, Afac, ld_lu, s_lu, perm, dinv, R, w, (long)nrows * w, X, w,
                                    (long)nrows * w, nl, s));
-  } else {
+  } else if (kind == HPS_KIND_ITI) {
     // ItI: the right-hand sides [P 0; 0 f_int] go straight to X in the
     // factors' row order (no R), then the solves run in place
     {
@@ -488,10 +520,10 @@ static int leaf_t(hps_handle_t h, int kind, int nl, int n, int nb, int nq, int n
   // 4. unpack Y and v
   if (kind == HPS_KIND_DTN) {
     HPS_CHECK_HIP(h, copy2d<T>(nb, nq, 1.0, P, nq, 0, Y, nq, (long)n * nq, nl, s));
-    HPS_CHECK_HIP(h, copy2d<T>(ni, nq, -1.0, X, w, (long)ni * w, Y + (long)nb * nq, nq, (long)n * nq, nl, s));
+    HPS_CHECK_HIP(h, copy2d<T>(ni, nq, -1.0, sol, w, (long)ni * w, Y + (long)nb * nq, nq, (long)n * nq, nl, s));
     if (nsrc > 0) {
       HPS_CHECK_HIP(h, copy2d<T>(nb, nsrc, 1.0, nullptr, 0, 0, (T*)vv, nsrc, (long)n * nsrc, nl, s));
-      HPS_CHECK_HIP(h, copy2d<T>(ni, nsrc, 1.0, X + nq, w, (long)ni * w, (T*)vv + (long)nb * nsrc, nsrc,
+      HPS_CHECK_HIP(h, copy2d<T>(ni, nsrc, 1.0, sol + nq, w, (long)ni * w, (T*)vv + (long)nb * nsrc, nsrc,
                                  (long)n * nsrc, nl, s));
     }
   } else {
@@ -582,10 +614,10 @@ static bool merge_block_inverses(int dtype, int nfac, int nm) {
 // than the zeros they leave out: the p = 8, L = 3 Poisson tree (6 .. 24 an
 // interface) took 1.08 ms with stages everywhere, 0.87 ms without.
 constexpr int MERGE_DISSECT_MIN = 48;
-static LuPlan merge_plan(int dissect, int nfac, int ne) {
+static LuPlan merge_plan(int dissect, int nfac, int ne, int nm) {
   if (dissect == HPS_DISSECT_QUAD && nfac / 4 >= MERGE_DISSECT_MIN) return lu_plan_quad(nfac / 4);
   if (dissect == HPS_DISSECT_OCT && nfac / 12 >= MERGE_DISSECT_MIN) return lu_plan_oct(nfac / 12);
-  return lu_plan_dense(nfac, ne);
+  return lu_plan_dense(nfac, ne, nm);
 }
 
 size_t hps_merge_workspace(int dtype, int kind, int nm, int ni, int ne, int nsrc) {
@@ -604,7 +636,7 @@ size_t hps_merge_workspace(int dtype, int kind, int nm, int ni, int ne, int nsrc
   size_t inv = 0, tmp = 0, ints = getrf_scratch_bytes(nfac, nm);
   for (int d = HPS_DISSECT_NONE; d <= HPS_DISSECT_OCT; ++d) {
     if (d != HPS_DISSECT_NONE && (kind == HPS_KIND_ITI || nfac % (d == HPS_DISSECT_QUAD ? 4 : 12))) continue;
-    const LuPlan p = merge_plan(d, nfac, ne);
+    const LuPlan p = merge_plan(d, nfac, ne, nm);
     inv = std::max(inv, lub_inv_elems(p, nm));
     tmp = std::max(tmp, lub_tmp_elems(p, nm));
     ints = std::max(ints, lub_scratch_bytes(p, nm));
@@ -762,6 +794,8 @@ static hipError_t coupling_gemm(hipStream_t s, int n_blk, const int* blk, int nF
   return block_gemm<T>(s, n_blk, blk, w, alpha, Dxy, nF, sD, X, ldx, sX, C ? 1.0 : 0.0, C, ldc, sC, Out, ldo, sO, nm);
 }
 
+#include "leaf_condensed.h"
+
 template <typename T>
 static int merge_t(hps_handle_t h, int kind, int nm, int nc, int nec, int ni, int ne, int nsrc, const void* T_in,
                    const void* h_in, const int* int_rows, const int* int_cols, const int* ext,
@@ -797,7 +831,7 @@ static int merge_t(hps_handle_t h, int kind, int nm, int nc, int nec, int ni, in
   // natural order: by blocks, with the handle's dissection for DtN
   const bool natural = h->merge_nopiv;
   const int dissect = !iti ? h->dissect : HPS_DISSECT_NONE;
-  const LuPlan plan = merge_plan(dissect, nfac, ne);
+  const LuPlan plan = merge_plan(dissect, nfac, ne, nm);
   const bool by_child = natural && plan.nstage > 1;  // columns of C by child
   T* linv = natural ? (T*)take(lub_inv_elems(plan, nm) * es) : nullptr;
   T* ltmp = natural ? (T*)take(lub_tmp_elems(plan, nm) * es) : nullptr;

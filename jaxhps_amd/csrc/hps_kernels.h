@@ -27,6 +27,10 @@ struct GemmArgs {
   int nin = 1;
   long sA2 = 0, sB2 = 0, sC2 = 0, sD2 = 0;
   int transA = 0;
+  // sum2 (real types, not transA): sum over 32 k at a time and add the sums up,
+  // for products with much cancellation -- the rounding of a long chain grows
+  // with its length.  A hint: shapes without that kernel sum in one chain.
+  int sum2 = 0;
   // triA: A is a packed 32 x 32 diagonal-block inverse used as its unit-lower
   // part (1) or its upper part (2); needs K <= 32.  D may then alias B.
   int triA = 0;
@@ -123,12 +127,17 @@ struct LuStage {
 };
 struct LuPlan {
   int n = 0, nstage = 0;
+  int nbmax = LUB_NB;  // widest block
   LuStage st[LUB_MAX_STAGES];
 };
-// one dense group of n unknowns
-inline LuPlan lu_plan_dense(int n, int ncols) {
+// One dense group of n unknowns.  Many matrices (LUB_MANY) take blocks of 64:
+// their launches are full either way, and a block's inverse, half of it zero,
+// costs operations and traffic in proportion to its width.  LUB_MANY_NOTE
+constexpr int LUB_MANY = 1024;
+inline LuPlan lu_plan_dense(int n, int ncols, int batch) {
   LuPlan p;
   p.n = n;
+  if (batch >= LUB_MANY) p.nbmax = 64;
   p.nstage = 1;
   p.st[0].size = n;
   p.st[0].nc = ncols;
@@ -182,25 +191,25 @@ inline LuPlan lu_plan_oct(int m) {
   p.st[2].nc = 24 * m;
   return p;
 }
-// groups are cut into equal blocks, a multiple of 32 wide and at most LUB_NB
-inline int lub_block(int size) {
-  const int nb = (size + LUB_NB - 1) / LUB_NB;
+// groups are cut into equal blocks, a multiple of 32 wide and at most nbmax
+inline int lub_block(const LuPlan& p, int size) {
+  const int nb = (size + p.nbmax - 1) / p.nbmax;
   return ((size + nb - 1) / nb + 31) / 32 * 32;
 }
-inline int lub_blocks(int size) { return (size + lub_block(size) - 1) / lub_block(size); }
+inline int lub_blocks(const LuPlan& p, int size) { return (size + lub_block(p, size) - 1) / lub_block(p, size); }
 // elements of the block inverses that a solve needs and of the factorisation's
 // scratch, bytes of its integer scratch
 inline size_t lub_inv_elems(const LuPlan& p, int batch) {
   size_t t = 0;
   for (int i = 0; i < p.nstage; ++i)
-    t += (size_t)p.st[i].cnt * lub_blocks(p.st[i].size) * 2 * lub_block(p.st[i].size) * lub_block(p.st[i].size);
+    t += (size_t)p.st[i].cnt * lub_blocks(p, p.st[i].size) * 2 * lub_block(p, p.st[i].size) * lub_block(p, p.st[i].size);
   return t * batch;
 }
 inline size_t lub_tmp_elems(const LuPlan& p, int batch) {
   size_t m = 0;
   for (int i = 0; i < p.nstage; ++i) {
     const LuStage& s = p.st[i];
-    const size_t t = (size_t)s.cnt * lub_block(s.size) * ((size_t)(s.size + p.n - s.r0 - s.cnt * s.size) + 32);
+    const size_t t = (size_t)s.cnt * lub_block(p, s.size) * ((size_t)(s.size + p.n - s.r0 - s.cnt * s.size) + 32);
     m = m > t ? m : t;
   }
   return m * batch;

@@ -34,13 +34,13 @@ constexpr int LUB_SPREAD_PARTS = 96;
 // cores, one 16 x 16 tile a wave.  db: the packed 32 x 32 inverses (part
 // stride nq blocks).  Writes whole columns, zeros included; ldi x ldi storage,
 // inv(U) after inv(L).
-template <typename T>
+template <typename T, int NBMAX>
 __global__ __launch_bounds__(256) void block_inverse_kernel(int nb, const T* A, long lda, long sA, int nin, long sA2,
                                                             const T* db, T* inv, int ldi, long sI, long sI2, int batch) {
   using R = typename real_of<T>::type;
   using M = Mfma<R>;
   using acc_t = typename M::acc_t;
-  __shared__ T X[LUB_NB][LU_NB + 1];
+  __shared__ T X[NBMAX][LU_NB + 1];
   __shared__ T W[LU_NB][LU_NB + 1];
   const int nq = (nb + LU_NB - 1) / LU_NB;
   const bool upper = (int)blockIdx.x >= nq;
@@ -63,26 +63,38 @@ __global__ __launch_bounds__(256) void block_inverse_kernel(int nb, const T* A, 
       X[s * LU_NB + r][c] = tri(s, r, c);
     }
     __syncthreads();
+    // the pairs (i, q) of the strip in one sequence: the next pair's factor
+    // entries (and, with a block row's first pair, its diagonal inverse) are
+    // requested before the current pair's product
     const int steps = upper ? s : nq - 1 - s;
+    auto load = [&](int i, int q, T (&a)[LU_NB / 4]) {
+      const int row = i * LU_NB + tr;
+#pragma unroll
+      for (int k = 0; k < LU_NB / 4; ++k) {
+        const int col = q * LU_NB + 4 * k + lk;
+        const bool in = row < nb && col < nb;
+        a[k] = Ab[in ? (long)row * lda + col : 0];
+        a[k] = s_sel(in, a[k], s_zero<T>());
+      }
+    };
+    T a[LU_NB / 4], an[LU_NB / 4], di[LU_NB / 4];
+    if (steps > 0) load(upper ? s - 1 : s + 1, s, a);
     for (int t = 1; t <= steps; ++t) {
       const int i = upper ? s - t : s + t;
       const int q0 = upper ? i + 1 : s, q1 = upper ? s + 1 : i;
-      T di[LU_NB / 4];  // this block row's diagonal inverse, requested with the first operands
 #pragma unroll
       for (int k = 0; k < LU_NB / 4; ++k) di[k] = tri(i, tr, 4 * k + lk);
       acc_t re = acc_t{0, 0, 0, 0}, im = acc_t{0, 0, 0, 0};
-      const int row = i * LU_NB + tr;
       for (int q = q0; q < q1; ++q) {
-        T a[LU_NB / 4];
-#pragma unroll
-        for (int k = 0; k < LU_NB / 4; ++k) {
-          const int col = q * LU_NB + 4 * k + lk;
-          const bool in = row < nb && col < nb;
-          a[k] = Ab[in ? (long)row * lda + col : 0];
-          a[k] = s_sel(in, a[k], s_zero<T>());
-        }
+        const int i2 = upper ? i - 1 : i + 1;
+        if (q + 1 < q1)
+          load(i, q + 1, an);
+        else if (t < steps)
+          load(i2, upper ? i2 + 1 : s, an);
 #pragma unroll
         for (int k = 0; k < LU_NB / 4; ++k) mma_step<T>(a[k], X[q * LU_NB + 4 * k + lk][tc], re, im);
+#pragma unroll
+        for (int k = 0; k < LU_NB / 4; ++k) a[k] = an[k];
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -278,13 +290,13 @@ hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* pe
   hipLaunchKernelGGL(lu_blocks_init_kernel, dim3(igrid < 4096 ? igrid : 4096), dim3(256), 0, s, n, batch, batch * cnt,
                      perm, info, arrivals);
   HPS_LU_CHECK(hipGetLastError());
-  const bool single = plan.nstage == 1 && plan.st[0].cnt == 1 && lub_blocks(n) == 1;
+  const bool single = plan.nstage == 1 && plan.st[0].cnt == 1 && lub_blocks(plan, n) == 1;
   const long sI = lub_inv_elems(plan, 1);
   T* ginv = inv;
   for (int is = 0; is < plan.nstage; ++is) {
     const LuStage& st = plan.st[is];
     const int nin = st.cnt, parts = nin * batch, size = st.size;
-    const int nb0 = lub_block(size);
+    const int nb0 = lub_block(plan, size);
     const int end = st.r0 + nin * size;  // first unknown after the stage
     const int rest = n - end;
     // 32 x 32 inverses of the current block (a single block's are dinv itself), then the panels
@@ -292,7 +304,7 @@ hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* pe
     T* pan = tmp + (long)parts * nb0 * LU_NB;
     const long gs = (long)size * (lda + 1);               // diagonal step from group to group
     const long gr = (long)size * lda, gc = (long)size;    // row and column step
-    const long sI2 = (long)lub_blocks(size) * 2 * nb0 * nb0;
+    const long sI2 = (long)lub_blocks(plan, size) * 2 * nb0 * nb0;
     T* a0 = A + (long)st.r0 * (lda + 1);
     for (int k = 0, blk = 0; k < size; k += nb0, ++blk) {
       const int nb = size - k < nb0 ? size - k : nb0;
@@ -306,8 +318,13 @@ hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* pe
         static const std::string nm = std::string("block_inverse<") + tname<T>() + ">";
         prof::Scope ps(s, nm.c_str(), flop_mult<T>() * parts * 2.0 / 3.0 * (double)nb * nb * nb,
                        sizeof(T) * 3.0 * (double)nb * nb * parts);
-        hipLaunchKernelGGL((block_inverse_kernel<T>), dim3(2 * ceil_div(nb, LU_NB), parts < 65535 ? parts : 65535),
-                           dim3(256), 0, s, nb, akk, lda, sA, nin, gs, db, li, nb0, sI, sI2, parts);
+        const dim3 igrid(2 * ceil_div(nb, LU_NB), parts < 65535 ? parts : 65535);
+        if (nb <= 64)  // less LDS: more workgroups a CU
+          hipLaunchKernelGGL((block_inverse_kernel<T, 64>), igrid, dim3(256), 0, s, nb, akk, lda, sA, nin, gs, db, li,
+                             nb0, sI, sI2, parts);
+        else
+          hipLaunchKernelGGL((block_inverse_kernel<T, LUB_NB>), igrid, dim3(256), 0, s, nb, akk, lda, sA, nin, gs, db,
+                             li, nb0, sI, sI2, parts);
         HPS_LU_CHECK(hipGetLastError());
       }
       if (m == 0) continue;
@@ -400,8 +417,8 @@ hipError_t lu_blocks_solve(const LuPlan& plan, const T* A, long lda, long sA, co
   // forward: X = inv(L) B, group by group in the columns where B is not zero
   for (int is = 0; is < plan.nstage; ++is) {
     const LuStage& st = plan.st[is];
-    const int nin = st.cnt, size = st.size, nb0 = lub_block(size);
-    const long sI2 = (long)lub_blocks(size) * 2 * nb0 * nb0;
+    const int nin = st.cnt, size = st.size, nb0 = lub_block(plan, size);
+    const long sI2 = (long)lub_blocks(plan, size) * 2 * nb0 * nb0;
     ginv[is] = off;
     off += nin * sI2;
     const int c0 = cols ? st.c0 : 0, nc = cols ? st.nc : nrhs, cs = cols ? st.c_step : 0;
@@ -436,8 +453,8 @@ hipError_t lu_blocks_solve(const LuPlan& plan, const T* A, long lda, long sA, co
   // backward: B = inv(U) X, all columns
   for (int is = plan.nstage - 1; is >= 0; --is) {
     const LuStage& st = plan.st[is];
-    const int nin = st.cnt, size = st.size, nb0 = lub_block(size);
-    const long sI2 = (long)lub_blocks(size) * 2 * nb0 * nb0;
+    const int nin = st.cnt, size = st.size, nb0 = lub_block(plan, size);
+    const long sI2 = (long)lub_blocks(plan, size) * 2 * nb0 * nb0;
     for (int i = 0; i < nin; ++i)
       for (int t = 0; t < st.g[i].nrun; ++t) {
         const long k0 = st.r0 + (long)i * size;
@@ -446,7 +463,7 @@ hipError_t lu_blocks_solve(const LuPlan& plan, const T* A, long lda, long sA, co
                             {B + (long)r * ldb, ldb, sB, 0}, 1.0, {X + k0 * ldx, ldx, sX, 0}, 1, batch, s));
       }
     const T* a0 = A + (long)st.r0 * (lda + 1);
-    for (int blk = lub_blocks(size) - 1; blk >= 0; --blk) {
+    for (int blk = lub_blocks(plan, size) - 1; blk >= 0; --blk) {
       const int k = blk * nb0, nb = size - k < nb0 ? size - k : nb0;
       const Parts<T> b{B + (long)(st.r0 + k) * ldb, ldb, sB, (long)size * ldb};
       HPS_LU_CHECK(mul<T>(nb, nrhs, nb, 1.0,
