@@ -191,25 +191,35 @@ inline LuPlan lu_plan_oct(int m) {
   p.st[2].nc = 24 * m;
   return p;
 }
-// groups are cut into equal blocks, a multiple of 32 wide and at most nbmax
-inline int lub_block(const LuPlan& p, int size) {
-  const int nb = (size + p.nbmax - 1) / p.nbmax;
-  return ((size + nb - 1) / nb + 31) / 32 * 32;
+// A group is cut into blocks of nbmax from its end, so that the trailing
+// products of every step are whole tiles; the first block takes the remainder
+// (with 64-wide blocks one of up to 16 joins the first whole block: 196 unknowns
+// are 68 + 64 + 64, where 64 + 64 + 64 + 4 left 132 and 68 unknowns to nine and
+// four 64 x 64 tiles).
+inline int lub_first(const LuPlan& p, int size) {
+  if (size <= p.nbmax) return size;
+  const int r = size % p.nbmax;
+  return r == 0 ? p.nbmax : (p.nbmax < LUB_NB && r <= 16 ? p.nbmax + r : r);
 }
-inline int lub_blocks(const LuPlan& p, int size) { return (size + lub_block(p, size) - 1) / lub_block(p, size); }
+inline int lub_blocks(const LuPlan& p, int size) { return 1 + (size - lub_first(p, size)) / p.nbmax; }
+// row stride (and rows) of a stored block inverse
+inline int lub_ld(const LuPlan& p, int size) {
+  const int f = lub_first(p, size), m = size > p.nbmax && f < p.nbmax ? p.nbmax : f;
+  return (m + 31) / 32 * 32;
+}
 // elements of the block inverses that a solve needs and of the factorisation's
 // scratch, bytes of its integer scratch
 inline size_t lub_inv_elems(const LuPlan& p, int batch) {
   size_t t = 0;
   for (int i = 0; i < p.nstage; ++i)
-    t += (size_t)p.st[i].cnt * lub_blocks(p, p.st[i].size) * 2 * lub_block(p, p.st[i].size) * lub_block(p, p.st[i].size);
+    t += (size_t)p.st[i].cnt * lub_blocks(p, p.st[i].size) * 2 * lub_ld(p, p.st[i].size) * lub_ld(p, p.st[i].size);
   return t * batch;
 }
 inline size_t lub_tmp_elems(const LuPlan& p, int batch) {
   size_t m = 0;
   for (int i = 0; i < p.nstage; ++i) {
     const LuStage& s = p.st[i];
-    const size_t t = (size_t)s.cnt * lub_block(p, s.size) * ((size_t)(s.size + p.n - s.r0 - s.cnt * s.size) + 32);
+    const size_t t = (size_t)s.cnt * lub_ld(p, s.size) * ((size_t)(s.size + p.n - s.r0 - s.cnt * s.size) + 32);
     m = m > t ? m : t;
   }
   return m * batch;

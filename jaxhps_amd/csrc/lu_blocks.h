@@ -27,6 +27,9 @@ namespace hps {
 // parts up to which the unpivoted panel kernel takes the diagonal blocks
 constexpr int LUB_SPREAD_PARTS = 96;
 
+// widest block whose products with its inverses run in place: the GEMM's tile
+constexpr int LUB_INPLACE = 64;
+
 // Inverses of L (unit lower, blockIdx.x < nq) and U of nb x nb diagonal
 // blocks, nb <= 128: one workgroup per 32-column strip of one inverse, the strip
 // in LDS.  Block row i of inv(L)'s strip s is -inv(L_ii) sum_{s <= q < i}
@@ -171,6 +174,23 @@ __global__ __launch_bounds__(256) void panel_back_kernel(int rows, int cols, con
   }
 }
 
+// info of the matrices whose multipliers (rows x cols at A) pass the bound
+template <typename T>
+__global__ __launch_bounds__(256) void panel_check_kernel(int rows, int cols, const T* A, long lda, long sA, int nin,
+                                                          long sA2, int* info, int batch) {
+  constexpr auto BOUND2 = typename real_of<T>::type(LU_NOPIV_BOUND * LU_NOPIV_BOUND);
+  const int total = rows * cols;
+  for (int b = blockIdx.y; b < batch; b += gridDim.y) {
+    const T* a = A + batch_offset(b, nin, sA, sA2);
+    bool ok = true;
+    for (int idx = blockIdx.x * 256 + threadIdx.x; idx < total; idx += gridDim.x * 256) {
+      const int r = idx / cols, c = idx - r * cols;
+      ok = ok && s_mod2(a[(long)r * lda + c]) <= BOUND2;
+    }
+    if (!ok) info[b / nin] = -1;
+  }
+}
+
 // X[:, c] = 0 for the columns outside [c0, c0 + nc)
 template <typename T>
 __global__ __launch_bounds__(256) void zero_outside_kernel(int rows, int cols, int c0, int c_step, int nc, T* X,
@@ -296,7 +316,7 @@ hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* pe
   for (int is = 0; is < plan.nstage; ++is) {
     const LuStage& st = plan.st[is];
     const int nin = st.cnt, parts = nin * batch, size = st.size;
-    const int nb0 = lub_block(plan, size);
+    const int nb0 = lub_ld(plan, size);
     const int end = st.r0 + nin * size;  // first unknown after the stage
     const int rest = n - end;
     // 32 x 32 inverses of the current block (a single block's are dinv itself), then the panels
@@ -306,8 +326,8 @@ hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* pe
     const long gr = (long)size * lda, gc = (long)size;    // row and column step
     const long sI2 = (long)lub_blocks(plan, size) * 2 * nb0 * nb0;
     T* a0 = A + (long)st.r0 * (lda + 1);
-    for (int k = 0, blk = 0; k < size; k += nb0, ++blk) {
-      const int nb = size - k < nb0 ? size - k : nb0;
+    const int first = lub_first(plan, size);
+    for (int k = 0, blk = 0, nb = first; k < size; k += nb, nb = plan.nbmax, ++blk) {
       const int below = size - k - nb;   // rows (columns) of the group after the block
       const int m = below + rest;
       T* akk = a0 + (long)k * (lda + 1);
@@ -332,45 +352,58 @@ hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* pe
       const dim3 bgrid(ceil_div((long)m * nb, 1024) < 1024 ? ceil_div((long)m * nb, 1024) : 1024,
                        parts < 65535 ? parts : 65535);
       const long sP = (long)m * nb;
-      // L21 = A21 inv(U11): the group's rows, then the later unknowns' rows
-      const Parts<T> u{ui, nb0, sI, sI2}, l{li, nb0, sI, sI2};
-      HPS_LU_CHECK(mul<T>(below, nb, nb, 1.0, {akk + (long)nb * lda, lda, sA, gs}, u, 0.0,
-                          {pan, nb, sP * nin, sP}, nin, batch, s));
-      HPS_LU_CHECK(mul<T>(rest, nb, nb, 1.0, {A + (long)end * lda + st.r0 + k, lda, sA, gc}, u, 0.0,
-                          {pan + (long)below * nb, nb, sP * nin, sP}, nin, batch, s));
-      // (with one group the two segments are neighbours and go back together)
-      auto back = [&](bool rows, int first, int count, T* dst, long step) -> hipError_t {
-        if (count <= 0) return hipSuccess;
-        prof::Scope ps(s, nmc.c_str(), 0.0, 2.0 * sizeof(T) * (double)count * nb * parts);
-        if (rows)
-          hipLaunchKernelGGL((panel_back_kernel<T, true>), bgrid, dim3(256), 0, s, count, nb, pan + (long)first * nb,
-                             (long)nb, sP, dst, lda, sA, nin, step, info, parts);
-        else
-          hipLaunchKernelGGL((panel_back_kernel<T, false>), bgrid, dim3(256), 0, s, nb, count, pan + first, (long)m,
-                             sP, dst, lda, sA, nin, step, info, parts);
-        return hipGetLastError();
-      };
-      if (nin == 1) {
-        HPS_LU_CHECK(back(true, 0, m, akk + (long)nb * lda, gs));
-      } else {
-        HPS_LU_CHECK(back(true, 0, below, akk + (long)nb * lda, gs));
-        HPS_LU_CHECK(back(true, below, rest, A + (long)end * lda + st.r0 + k, gc));
-      }
+      // L21 = A21 inv(U11): the group's rows, then the later unknowns' rows;
       // U12 = inv(L11) A12, the same way by columns
-      HPS_LU_CHECK(mul<T>(nb, below, nb, 1.0, l, {akk + nb, lda, sA, gs}, 0.0, {pan, m, sP * nin, sP}, nin, batch, s));
-      HPS_LU_CHECK(mul<T>(nb, rest, nb, 1.0, l, {A + (long)(st.r0 + k) * lda + end, lda, sA, gr}, 0.0,
-                          {pan + below, m, sP * nin, sP}, nin, batch, s));
-      if (nin == 1) {
-        HPS_LU_CHECK(back(false, 0, m, akk + nb, gs));
+      const Parts<T> u{ui, nb0, sI, sI2}, l{li, nb0, sI, sI2};
+      T* arc = A + (long)end * lda + st.r0 + k;    // later rows, the block's columns
+      T* acr = A + (long)(st.r0 + k) * lda + end;  // the block's rows, later columns
+      if (nb <= LUB_INPLACE && (below == 0 || below > 2) && (rest == 0 || rest > 2)) {
+        // one tile holds the block's width, so every workgroup has read all that
+        // it overwrites (its rows of A21, its columns of A12) before it writes
+        // (one or two columns of A12 take the GEMV kernel, which is not so)
+        HPS_LU_CHECK(mul<T>(below, nb, nb, 1.0, {akk + (long)nb * lda, lda, sA, gs}, u, 0.0,
+                            {akk + (long)nb * lda, lda, sA, gs}, nin, batch, s));
+        HPS_LU_CHECK(mul<T>(rest, nb, nb, 1.0, {arc, lda, sA, gc}, u, 0.0, {arc, lda, sA, gc}, nin, batch, s));
+        HPS_LU_CHECK(mul<T>(nb, below, nb, 1.0, l, {akk + nb, lda, sA, gs}, 0.0, {akk + nb, lda, sA, gs}, nin, batch, s));
+        HPS_LU_CHECK(mul<T>(nb, rest, nb, 1.0, l, {acr, lda, sA, gr}, 0.0, {acr, lda, sA, gr}, nin, batch, s));
+        for (int seg = 0; seg < 2; ++seg) {
+          const int rows = seg == 0 ? below : rest;
+          if (rows <= 0) continue;
+          static const std::string nmk = std::string("panel_check<") + tname<T>() + ">";
+          prof::Scope ps(s, nmk.c_str(), 0.0, sizeof(T) * (double)rows * nb * parts);
+          hipLaunchKernelGGL((panel_check_kernel<T>), bgrid, dim3(256), 0, s, rows, nb,
+                             seg == 0 ? akk + (long)nb * lda : arc, lda, sA, nin, seg == 0 ? gs : gc, info, parts);
+          HPS_LU_CHECK(hipGetLastError());
+        }
       } else {
-        HPS_LU_CHECK(back(false, 0, below, akk + nb, gs));
-        HPS_LU_CHECK(back(false, below, rest, A + (long)(st.r0 + k) * lda + end, gr));
+        HPS_LU_CHECK(mul<T>(below, nb, nb, 1.0, {akk + (long)nb * lda, lda, sA, gs}, u, 0.0,
+                            {pan, nb, sP * nin, sP}, nin, batch, s));
+        HPS_LU_CHECK(mul<T>(rest, nb, nb, 1.0, {arc, lda, sA, gc}, u, 0.0, {pan + (long)below * nb, nb, sP * nin, sP},
+                            nin, batch, s));
+        // (with one group the two segments are neighbours and go back together)
+        auto back = [&](bool rows, int first_, int count, T* dst, long step) -> hipError_t {
+          if (count <= 0) return hipSuccess;
+          prof::Scope ps(s, nmc.c_str(), 0.0, 2.0 * sizeof(T) * (double)count * nb * parts);
+          if (rows)
+            hipLaunchKernelGGL((panel_back_kernel<T, true>), bgrid, dim3(256), 0, s, count, nb,
+                               pan + (long)first_ * nb, (long)nb, sP, dst, lda, sA, nin, step, info, parts);
+          else
+            hipLaunchKernelGGL((panel_back_kernel<T, false>), bgrid, dim3(256), 0, s, nb, count, pan + first_, (long)m,
+                               sP, dst, lda, sA, nin, step, info, parts);
+          return hipGetLastError();
+        };
+        HPS_LU_CHECK(back(true, 0, nin == 1 ? m : below, akk + (long)nb * lda, gs));
+        if (nin > 1) HPS_LU_CHECK(back(true, below, rest, arc, gc));
+        HPS_LU_CHECK(mul<T>(nb, below, nb, 1.0, l, {akk + nb, lda, sA, gs}, 0.0, {pan, m, sP * nin, sP}, nin, batch, s));
+        HPS_LU_CHECK(mul<T>(nb, rest, nb, 1.0, l, {acr, lda, sA, gr}, 0.0, {pan + below, m, sP * nin, sP}, nin, batch, s));
+        HPS_LU_CHECK(back(false, 0, nin == 1 ? m : below, akk + nb, gs));
+        if (nin > 1) HPS_LU_CHECK(back(false, below, rest, acr, gr));
       }
       // the group's trailing block, the later rows in its columns and its rows
       // in the later columns; the later unknowns' own block waits for the whole
       // group (one product with K = size)
       const Parts<T> lg{akk + (long)nb * lda, lda, sA, gs}, ug{akk + nb, lda, sA, gs};
-      const Parts<T> lr{A + (long)end * lda + st.r0 + k, lda, sA, gc}, ur{A + (long)(st.r0 + k) * lda + end, lda, sA, gr};
+      const Parts<T> lr{arc, lda, sA, gc}, ur{acr, lda, sA, gr};
       HPS_LU_CHECK(mul<T>(below, below, nb, -1.0, lg, ug, 1.0, {akk + (long)nb * (lda + 1), lda, sA, gs}, nin, batch, s));
       HPS_LU_CHECK(mul<T>(rest, below, nb, -1.0, lr, ug, 1.0, {lr.p + nb, lda, sA, gc}, nin, batch, s));
       HPS_LU_CHECK(mul<T>(below, rest, nb, -1.0, lg, ur, 1.0, {ur.p + (long)nb * lda, lda, sA, gr}, nin, batch, s));
@@ -417,7 +450,7 @@ hipError_t lu_blocks_solve(const LuPlan& plan, const T* A, long lda, long sA, co
   // forward: X = inv(L) B, group by group in the columns where B is not zero
   for (int is = 0; is < plan.nstage; ++is) {
     const LuStage& st = plan.st[is];
-    const int nin = st.cnt, size = st.size, nb0 = lub_block(plan, size);
+    const int nin = st.cnt, size = st.size, nb0 = lub_ld(plan, size);
     const long sI2 = (long)lub_blocks(plan, size) * 2 * nb0 * nb0;
     ginv[is] = off;
     off += nin * sI2;
@@ -426,8 +459,7 @@ hipError_t lu_blocks_solve(const LuPlan& plan, const T* A, long lda, long sA, co
     T* b0 = B + (long)st.r0 * ldb + c0;
     T* x0 = X + (long)st.r0 * ldx + c0;
     const T* a0 = A + (long)st.r0 * (lda + 1);
-    for (int k = 0, blk = 0; k < size; k += nb0, ++blk) {
-      const int nb = size - k < nb0 ? size - k : nb0;
+    for (int k = 0, blk = 0, nb = lub_first(plan, size); k < size; k += nb, nb = plan.nbmax, ++blk) {
       const Parts<T> x{x0 + (long)k * ldx, ldx, sX, gx};
       HPS_LU_CHECK(mul<T>(nb, nc, nb, 1.0, {inv + ginv[is] + (long)blk * 2 * nb0 * nb0, nb0, sI, sI2},
                           {b0 + (long)k * ldb, ldb, sB, gb}, 0.0, x, nin, batch, s));
@@ -453,7 +485,7 @@ hipError_t lu_blocks_solve(const LuPlan& plan, const T* A, long lda, long sA, co
   // backward: B = inv(U) X, all columns
   for (int is = plan.nstage - 1; is >= 0; --is) {
     const LuStage& st = plan.st[is];
-    const int nin = st.cnt, size = st.size, nb0 = lub_block(plan, size);
+    const int nin = st.cnt, size = st.size, nb0 = lub_ld(plan, size);
     const long sI2 = (long)lub_blocks(plan, size) * 2 * nb0 * nb0;
     for (int i = 0; i < nin; ++i)
       for (int t = 0; t < st.g[i].nrun; ++t) {
@@ -464,7 +496,8 @@ hipError_t lu_blocks_solve(const LuPlan& plan, const T* A, long lda, long sA, co
       }
     const T* a0 = A + (long)st.r0 * (lda + 1);
     for (int blk = lub_blocks(plan, size) - 1; blk >= 0; --blk) {
-      const int k = blk * nb0, nb = size - k < nb0 ? size - k : nb0;
+      const int first = lub_first(plan, size);
+      const int k = blk == 0 ? 0 : first + (blk - 1) * plan.nbmax, nb = blk == 0 ? first : plan.nbmax;
       const Parts<T> b{B + (long)(st.r0 + k) * ldb, ldb, sB, (long)size * ldb};
       HPS_LU_CHECK(mul<T>(nb, nrhs, nb, 1.0,
                           {inv + ginv[is] + (long)(2 * blk + 1) * nb0 * nb0, nb0, sI, sI2},
