@@ -73,11 +73,12 @@ def test_unpivoted_panel_rejects(gpu, dtype, row):
     ("quad", 47, 2, torch.float64), ("quad", 48, 3, torch.float32), ("quad", 65, 2, torch.complex128),
     ("quad", 129, 1, torch.float64), ("quad", 20, 40, torch.complex64), ("oct", 47, 1, torch.float64),
     ("oct", 49, 2, torch.float64), ("oct", 64, 1, torch.float32), ("iti", 65, 3, torch.complex128),
-    ("iti", 20, 30, torch.complex64)])
+    ("iti", 20, 30, torch.complex64), ("quad", 17, 1024, torch.float64), ("quad", 36, 1024, torch.float32),
+    ("iti", 21, 1024, torch.complex64)])
 def test_block_elimination_matches_pivoted(gpu, kind, m, nm, dtype):
     """Natural-order block elimination (dense below 48 unknowns an interface,
-    dissected from there; partial blocks, many and few matrices) against the
-    pivoted merge.  The matrices' condition is below 10, so both are within
+    dissected from there; partial blocks, many and few matrices, first blocks of
+    1, 2, 20, 68 and 80 unknowns) against the pivoted merge.  The matrices' condition is below 10, so both are within
     10 n eps of the exact result in the maximum norm."""
     from jaxhps_amd._stages import merge_level, up_level
     from jaxhps_amd._tables import oct_merge_tables, quad_merge_tables
@@ -105,6 +106,98 @@ def test_block_elimination_matches_pivoted(gpu, kind, m, nm, dtype):
     gt, ho = up_level(h, nat)
     assert float((gt - piv.gt).abs().max() / piv.gt.abs().max()) < bound
     assert float((ho - piv.h).abs().max() / piv.h.abs().max()) < bound
+
+
+def _iti_leaves(gpu, p, L, k2, imag=0.0):
+    """An ItI problem with smooth coefficients on 4^L leaves, and its leaf
+    matrices B = [G; A_int] (complex128, numpy) for chosen leaves."""
+    import jaxhps_amd as jh
+
+    dom = jh.Domain(p=p, q=p - 2, root=jh.DiscretizationNode2D(-1.0, 1.0, -1.0, 1.0), L=L)
+    x = dom.interior_points
+    cf = {"D_xx": 1.0 + 0.2 * np.sin(x[..., 0]), "D_yy": 1.0 + 0.1 * x[..., 1], "D_x": 0.3 * x[..., 1],
+          "I": k2 * (1.0 + 0.3 * np.cos(x[..., 0] + x[..., 1])) + 1j * imag}
+    if imag == 0.0:
+        cf["I"] = cf["I"].real
+    pde = jh.PDEProblem(dom, use_ItI=True, eta=3.0, **{f"{n}_coefficients": a for n, a in cf.items()})
+    nb = np.asarray(pde.P).shape[0]
+
+    def matrix(leaf):
+        A = sum(cf[nm][leaf][:, None]
+                * (np.eye(p * p) if nm == "I" else np.asarray(getattr(pde, nm))) for nm, _ in pde.coefficient_list())
+        return np.concatenate([np.asarray(pde.G), A[nb:]]).astype(complex)
+
+    return pde, nb, matrix
+
+
+@pytest.mark.parametrize("p,L,nsrc,dtype", [
+    (5, 1, 0, torch.complex128), (8, 2, 1, torch.complex128), (16, 1, 3, torch.complex128), (9, 2, 2, torch.complex64),
+    (10, 5, 1, torch.complex64), (11, 5, 3, torch.complex128), (14, 5, 1, torch.complex128)])
+def test_condensed_leaves(gpu, p, L, nsrc, dtype):
+    """Y, T, v, h and the kept factors' B^{-1} and B^{-H} of condensed leaves
+    (one and several blocks, few and many leaves) against numpy solves with B.
+    An eliminated system's error is within n eps cond, the impedance rows
+    brought to the others' size first (a power of ten below B's condition)."""
+    from jaxhps_amd._stages import HPS_KIND_ITI, leaf_apply_inverse, leaf_solve
+    from jaxhps_amd.adjoint import _condensed_inverse_conjt
+
+    print(f"condensed leaves p={p} L={L} nsrc={nsrc} {dtype}", flush=True)
+    pde, nb, matrix = _iti_leaves(gpu, p, L, 4.0)
+    nl, n = 4**L, p * p
+    g = torch.Generator(device=gpu).manual_seed(p)
+    f = torch.randn(nl, n, max(nsrc, 1), generator=g, device=gpu, dtype=dtype)
+    res = leaf_solve(pde, HPS_KIND_ITI, dtype, gpu, source=f if nsrc else None, nsrc_zero=nsrc == 0)
+    assert res.condensed is not None
+    inv, invh = leaf_apply_inverse(res, f), _condensed_inverse_conjt(res, f)
+    P, QH = np.asarray(pde.P), np.asarray(pde.QH)
+    for leaf in {0, nl // 2 + 1, nl - 1}:
+        B = matrix(leaf)
+        scale = np.ones(n)
+        scale[:nb] = np.abs(B[nb:]).max() / np.abs(B[:nb]).max()
+        bound = n * EPS[dtype] * np.linalg.cond(scale[:, None] * B)
+        fl = f[leaf].cpu().numpy().astype(complex)
+        fi = fl.copy()
+        fi[:nb] = 0.0
+        rhs = np.zeros((n, P.shape[1]), dtype=complex)
+        rhs[:nb] = P
+        ref = {"Y": np.linalg.solve(B, rhs), "inv": np.linalg.solve(B, fl),
+               "invh": np.linalg.solve(B.conj().T, fl)}
+        ref["T"] = QH @ ref["Y"]
+        got = {"Y": res.Y, "T": res.T, "inv": inv, "invh": invh}
+        if nsrc:
+            ref["v"] = np.linalg.solve(B, fi)
+            ref["h"] = QH @ ref["v"]
+            got.update(v=res.v, h=res.h)
+        for nm, r in ref.items():
+            # T and h: the error of Y and v through QH
+            size = {"T": np.abs(QH).sum(1).max() * np.abs(ref["Y"]).max(),
+                    "h": np.abs(QH).sum(1).max() * np.abs(ref.get("v", 0.0)).max()}.get(nm, np.abs(r).max())
+            err = np.abs(got[nm][leaf].cpu().numpy() - r).max() / size
+            assert err <= bound, (nm, leaf, err, bound)
+
+
+def test_condensed_leaves_give_way(gpu):
+    """Complex coefficients, and a leaf at an eigenvalue of its Dirichlet
+    problem, take the factorisation of B; the results stay right."""
+    from jaxhps_amd._stages import HPS_KIND_ITI, leaf_solve
+
+    print("condensed leaves give way", flush=True)
+    for imag, k2 in ((0.5, 4.0), (0.0, None)):
+        if k2 is None:  # the constant part nearest an eigenvalue of leaf 0
+            pde, nb, matrix = _iti_leaves(gpu, 8, 1, 0.0)
+            x = pde.domain.interior_points[0, nb:]
+            A, W = matrix(0)[nb:, nb:].real, 1.0 + 0.3 * np.cos(x[:, 0] + x[:, 1])
+            w = np.linalg.eigvals(-A / W[:, None])
+            k2 = float(w[np.abs(w.imag) < 1e-9].real.min())
+        pde, nb, matrix = _iti_leaves(gpu, 8, 1, k2, imag)
+        res = leaf_solve(pde, HPS_KIND_ITI, torch.complex128, gpu, nsrc_zero=True)
+        assert res.condensed is None
+        B = matrix(0)
+        rhs = np.zeros((64, pde.P.shape[1]), dtype=complex)
+        rhs[:nb] = np.asarray(pde.P)
+        ref = np.linalg.solve(B, rhs)
+        err = np.abs(res.Y[0].cpu().numpy() - ref).max() / np.abs(ref).max()
+        assert err <= 64 * 2.0**-53 * np.linalg.cond(B), err
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
