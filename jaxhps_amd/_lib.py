@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from pathlib import Path
 
 import torch
@@ -144,23 +145,39 @@ def _require_gpu():
         raise HPSLibraryError("jaxhps_amd needs a ROCm GPU; torch.cuda.is_available() is False")
 
 
-_handles: dict = {}
+class _Handle(ctypes.c_void_p):
+    """A library handle, given back with the last reference to it."""
+
+    def __del__(self):
+        if self.value and _lib is not None:
+            _lib.hps_destroy(self)
+
+
+class _ThreadHandles(threading.local):
+    """This thread's handles by (device, stream).  A handle carries the
+    factorisations' switches from a set call to the stage call that reads them
+    (and the last error), so no two threads share one, also on one stream."""
+
+    def __init__(self):
+        self.by_stream: dict = {}
+
+
+_handles = _ThreadHandles()
 
 
 def handle():
-    """Library handle bound to torch's current stream on the current device."""
+    """This thread's library handle bound to torch's current stream on the current device."""
     _require_gpu()
     lib = load_library()
     stream = torch.cuda.current_stream()
     key = (stream.device_index, stream.cuda_stream)
-    h = _handles.get(key)
+    h = _handles.by_stream.get(key)
     if h is None:
-        hp = ctypes.c_void_p()
-        rc = lib.hps_create(ctypes.c_void_p(stream.cuda_stream), ctypes.byref(hp))
+        h = _Handle()
+        rc = lib.hps_create(ctypes.c_void_p(stream.cuda_stream), ctypes.byref(h))
         if rc != HPS_OK:
             raise HPSLibraryError("hps_create failed")
-        h = hp
-        _handles[key] = h
+        _handles.by_stream[key] = h
     return h
 
 

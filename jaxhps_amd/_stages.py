@@ -314,12 +314,13 @@ def merge_level(T_in, h_in, tables: MergeTables, keep_factors=False, want_T=True
     dissect = getattr(tables, "dissect", HPS_DISSECT_NONE)
     if kind == HPS_KIND_DTN and not getattr(tables, "reordered", False):
         final_of_internal = None  # the internal order is the final one
-    if not pivot:
-        check(lib.hps_set_merge_pivoting(hd, 0), hd, "hps_set_merge_pivoting")
-        if dissect:
-            by_child, pos = tables.by_child_device(dev)
-            check(lib.hps_set_merge_dissection(hd, dissect, ptr(by_child), ptr(pos)), hd, "hps_set_merge_dissection")
     try:
+        if not pivot:
+            check(lib.hps_set_merge_pivoting(hd, 0), hd, "hps_set_merge_pivoting")
+            if dissect:
+                by_child, pos = tables.by_child_device(dev)
+                check(lib.hps_set_merge_dissection(hd, dissect, ptr(by_child), ptr(pos)), hd,
+                      "hps_set_merge_dissection")
         rc = _merge_level_call(lib, hd, dt, kind, nm, nc, nec, ni, ne, nsrc, T_in, h_in, rows, cols, ext, cols_final,
                                final_of_internal, upd, d12, d21, S, T, ho, gt, F_lu, perm, dinv, info, D12, D21, B,
                                Finv, ws)

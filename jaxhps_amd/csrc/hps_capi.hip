@@ -477,7 +477,8 @@ static int leaf_t(hps_handle_t h, int kind, int nl, int n, int nb, int nq, int n
   // 3. factor and solve
   T* Afac = kind == HPS_KIND_DTN ? lu + nb : lu;
   T* sol = X;
-  if (kind == HPS_KIND_DTN && h->leaf_nopiv) {
+  const bool natural = h->leaf_nopiv;
+  if (kind == HPS_KIND_DTN && natural) {
     // natural order by blocks, the right-hand sides solved in place (X is
     // scratch), LEAF_CHUNK leaves at a time
     const int m = nl < LEAF_CHUNK ? nl : LEAF_CHUNK;
@@ -498,9 +499,9 @@ static int leaf_t(hps_handle_t h, int kind, int nl, int n, int nb, int nq, int n
     }
     sol = R;
   } else {
-    HPS_CHECK_HIP(h, getrf_ws<T>(nrows, Afac, ld_lu, s_lu, perm, dinv, scratch, info, nl, s, h->leaf_nopiv));
+    HPS_CHECK_HIP(h, getrf_ws<T>(nrows, Afac, ld_lu, s_lu, perm, dinv, scratch, info, nl, s, natural));
   }
-  if (kind == HPS_KIND_DTN && !h->leaf_nopiv) {
+  if (kind == HPS_KIND_DTN && !natural) {
     HPS_CHECK_HIP(h, getrs_perm<T>(nrows, w, Afac, ld_lu, s_lu, perm, dinv, R, w, (long)nrows * w, X, w,
                                    (long)nrows * w, nl, s));
   } else if (kind == HPS_KIND_ITI) {

@@ -108,6 +108,49 @@ def test_block_elimination_matches_pivoted(gpu, kind, m, nm, dtype):
     assert float((ho - piv.h).abs().max() / piv.h.abs().max()) < bound
 
 
+def test_merges_from_several_threads(gpu):
+    """Merges with different eliminations (dissected 2D and 3D, dense ItI,
+    pivoted) from four threads on one stream: each thread's factorisation
+    switches are its own, so every result is the one it has alone."""
+    import threading
+
+    from jaxhps_amd._stages import merge_level
+    from jaxhps_amd._tables import oct_merge_tables, quad_merge_tables
+
+    print("merges from several threads", flush=True)
+    jobs = []
+    for tb, nm, pivot in ((quad_merge_tables(60, "dtn"), 3, False), (oct_merge_tables(49), 1, False),
+                          (quad_merge_tables(20, "iti"), 8, False), (quad_merge_tables(60, "dtn"), 3, True)):
+        g = torch.Generator(device=gpu).manual_seed(tb.nec)
+        T = 0.1 * torch.randn(tb.nc * nm, tb.nec, tb.nec, generator=g, device=gpu, dtype=torch.float64) / tb.nec**0.5
+        if tb.kind == "iti":
+            T = T.to(torch.complex128)
+        else:
+            T = T + 2.0 * torch.eye(tb.nec, device=gpu, dtype=T.dtype)
+        jobs.append((T.contiguous(), tb, pivot))
+    alone = [merge_level(T, None, tb, pivot=pivot) for T, tb, pivot in jobs]
+    torch.cuda.synchronize()
+    wrong, start = [], threading.Barrier(len(jobs), timeout=60)
+
+    def work(i):
+        T, tb, pivot = jobs[i]
+        start.wait()
+        try:
+            for _ in range(20):
+                r = merge_level(T, None, tb, pivot=pivot)
+                if not (torch.equal(r.S, alone[i].S) and torch.equal(r.T, alone[i].T)):
+                    wrong.append(i)
+        except Exception as e:  # reported by the assertion below
+            wrong.append((i, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong
+
+
 def _iti_leaves(gpu, p, L, k2, imag=0.0):
     """An ItI problem with smooth coefficients on 4^L leaves, and its leaf
     matrices B = [G; A_int] (complex128, numpy) for chosen leaves."""

@@ -235,6 +235,49 @@ def test_library_argument_errors_without_gpu():
     assert lib.hps_destroy(h) == 0
 
 
+def test_each_thread_has_its_own_handle(monkeypatch):
+    """A handle carries pivoting and dissection from the set call to the stage
+    call, so two threads on one stream must not share it; a thread's handles
+    are given back when it ends."""
+    import threading
+
+    import torch
+
+    from jaxhps_amd import _lib
+
+    lib = _lib.load_library()
+    destroyed = []
+
+    class Counting:
+        hps_create = lib.hps_create
+
+        @staticmethod
+        def hps_destroy(h):
+            destroyed.append(h.value)
+            return lib.hps_destroy(h)
+
+    stream = type("Stream", (), {"device_index": 0, "cuda_stream": 0})()
+    monkeypatch.setattr(_lib, "_require_gpu", lambda: None)
+    monkeypatch.setattr(_lib, "_lib", Counting)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: stream)
+    seen = {}
+
+    def work(name):
+        h = _lib.handle()
+        seen[name] = h.value
+        assert _lib.handle() is h
+        barrier.wait()  # both are alive at once
+
+    barrier = threading.Barrier(2, timeout=60)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(seen) == 2 and seen[0] != seen[1]
+    assert sorted(destroyed) == sorted(seen.values())
+
+
 def test_block_inverse_sizes_and_argument_errors():
     """hps_block_inverses: eligible sizes (n > 256, a multiple of 32) hold two
     256 x 256 inverses per diagonal block (the last one padded), others none;
