@@ -674,11 +674,17 @@ __global__ __launch_bounds__(256) void scatter_kernel(const T* src, long ss, T* 
 template <typename T>
 static hipError_t scatter_rows(hipStream_t s, const T* src, long ss, T* dst, long sd, const int* map, const int* cmap,
                                int rows, int cols, int nm) {
-  if ((long)rows * cols >= (1L << 31)) return hipErrorInvalidValue;  // 32-bit indices in one matrix
   static const std::string nms = std::string("row_scatter<") + tname<T>() + ">";
   prof::Scope ps(s, nms.c_str(), 0.0, 2.0 * sizeof(T) * (double)rows * cols * nm);
-  hipLaunchKernelGGL((scatter_kernel<T>), grid_for((long)rows * cols, nm), dim3(256), 0, s, src, ss, dst, sd, map,
-                     cmap, rows, cols, nm);
+  // 32-bit indices in one launch: the rows whose elements stay below 2^31 (a
+  // 3D root of 2731 unknowns an interface has more)
+  const long most = ((1L << 31) - 1) / cols;
+  const int per = most < rows ? (int)most : rows;
+  for (int r0 = 0; r0 < rows; r0 += per) {
+    const int nr = rows - r0 < per ? rows - r0 : per;
+    hipLaunchKernelGGL((scatter_kernel<T>), grid_for((long)nr * cols, nm), dim3(256), 0, s, src + (long)r0 * cols, ss,
+                       map ? dst : dst + (long)r0 * cols, sd, map ? map + r0 : nullptr, cmap, nr, cols, nm);
+  }
   return hipGetLastError();
 }
 

@@ -108,6 +108,36 @@ def test_block_elimination_matches_pivoted(gpu, kind, m, nm, dtype):
     assert float((ho - piv.h).abs().max() / piv.h.abs().max()) < bound
 
 
+def test_merge_beyond_32_bit_indices(gpu):
+    """A 3D merge whose S has more than 2^31 elements (32784 x 65568).  Columns
+    of S put back into the children: the outgoing data of the two sides of
+    every interface cancel, to n eps of the terms' sum."""
+    from jaxhps_amd._stages import merge_level
+    from jaxhps_amd._tables import oct_merge_tables
+
+    if torch.cuda.mem_get_info(gpu)[0] < 64 << 30:
+        pytest.skip("needs 64 GB of device memory")
+    print("merge beyond 32-bit indices", flush=True)
+    tb = oct_merge_tables(2732)
+    assert tb.ni * tb.ne > 2**31
+    g = torch.Generator(device=gpu).manual_seed(1)
+    T = torch.randn(8, tb.nec, tb.nec, generator=g, device=gpu, dtype=torch.float32).mul_(0.1 / tb.nec**0.5)
+    T.diagonal(dim1=1, dim2=2).add_(2.0)
+    out = merge_level(T, None, tb, want_T=False, pivot=False)
+    assert int(out.info[0]) == 0
+    cols = torch.tensor([0, tb.ne // 2, tb.ne - 1], device=gpu)
+    S = out.S[0][:, cols].double()
+    del out
+    src = torch.as_tensor(tb.child_src, device=gpu).long().reshape(-1)
+    data = torch.where((src >= 0)[:, None], (src[:, None] == cols[None]).double(), S[(-src - 1).clamp(min=0)])
+    data = data.reshape(8, tb.nec, -1)
+    flux = torch.stack([T[c].double() @ data[c] for c in range(8)])
+    size = torch.stack([T[c].double().abs() @ data[c].abs() for c in range(8)])
+    c0, l0, c1, l1 = torch.as_tensor(tb.int_rows, device=gpu).long().T
+    res = (flux[c0, l0] + flux[c1, l1]).abs() / (size[c0, l0] + size[c1, l1])
+    assert float(res.max()) < tb.ni * EPS[torch.float32]
+
+
 def test_merges_from_several_threads(gpu):
     """Merges with different eliminations (dissected 2D and 3D, dense ItI,
     pivoted) from four threads on one stream: each thread's factorisation
