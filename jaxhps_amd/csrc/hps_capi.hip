@@ -873,7 +873,7 @@ static int merge_t(hps_handle_t h, int kind, int nm, int nc, int nec, int ni, in
 
   // ---- solves: X = -D^{-1} [C | h_int] -------------------------------------
   // one pass for the C columns (width ne) and one for h (width nsrc); natural
-  // order solves in place (its scratch is the output), pivoting out of place
+  // order solves in place, pivoting out of place
   for (int pass = 0; pass < 2; ++pass) {
     const int w = pass == 0 ? ne : nsrc;
     if (w <= 0) continue;
@@ -881,8 +881,12 @@ static int merge_t(hps_handle_t h, int kind, int nm, int nc, int nec, int ni, in
     T* Zp = pass == 0 ? Z : Zh;
     T* out = (T*)(pass == 0 ? S_out : gt_out);
     const long sY = (long)ni * w;
-    // DtN with pivoting: right-hand sides in the output, solutions in Yp
-    T* rhs = iti || natural ? Yp : out;
+    // DtN: the solution lies in the right-hand sides' buffer (natural order) or
+    // in the other one (pivoting); without a row map that buffer is the output,
+    // with one the solution is scattered there
+    const bool direct = !iti && !final_of_internal;
+    T* rhs = iti || natural != direct ? Yp : out;
+    T* other = rhs == Yp ? out : Yp;
     if (pass == 0) {
       HPS_CHECK_HIP(h, gather_launch<T>(s, "C", Tin, nc, nec, rows, ni, by_child ? (const int4*)h->ext_child : ex, ne,
                                         -1.0, 0, rhs, ne, sY, nm));
@@ -895,11 +899,12 @@ static int merge_t(hps_handle_t h, int kind, int nm, int nc, int nec, int ni, in
     }
     if (!iti) {
       if (natural)
-        HPS_CHECK_HIP(h, lu_blocks_solve<T>(plan, Fl, ni, sNF2, linv, Yp, w, sY, out, w, sY, w, pass == 0, nm, s));
+        HPS_CHECK_HIP(h, lu_blocks_solve<T>(plan, Fl, ni, sNF2, linv, rhs, w, sY, other, w, sY, w, pass == 0, nm, s));
       else
-        HPS_CHECK_HIP(h, getrs_perm<T>(ni, w, Fl, ni, sNF2, perm, dinv, rhs, w, sY, Yp, w, sY, nm, s));
-      HPS_CHECK_HIP(h, scatter_rows<T>(s, Yp, sY, out, sY, final_of_internal,
-                                       by_child && pass == 0 ? h->ext_pos : nullptr, ni, w, nm));
+        HPS_CHECK_HIP(h, getrs_perm<T>(ni, w, Fl, ni, sNF2, perm, dinv, rhs, w, sY, other, w, sY, nm, s));
+      if (!direct)
+        HPS_CHECK_HIP(h, scatter_rows<T>(s, Yp, sY, out, sY, final_of_internal,
+                                         by_child && pass == 0 ? h->ext_pos : nullptr, ni, w, nm));
     } else {
       const long sZ = (long)nF * w;
       // Z = Y_F - D12 Y_G

@@ -108,6 +108,36 @@ def test_block_elimination_matches_pivoted(gpu, kind, m, nm, dtype):
     assert float((ho - piv.h).abs().max() / piv.h.abs().max()) < bound
 
 
+@pytest.mark.parametrize("pivot", [True, False])
+def test_merge_without_row_map(gpu, pivot):
+    """DtN merges whose internal order is the final one (adaptive trees): the
+    rows of S and g_tilde come in internal order, T and h are the mapped
+    merge's, and the solution goes straight to the output."""
+    import copy
+
+    from jaxhps_amd import profiling
+    from jaxhps_amd._stages import merge_level
+    from jaxhps_amd._tables import quad_merge_tables
+
+    print(f"merge without row map pivot={pivot}", flush=True)
+    tb = quad_merge_tables(37, "dtn")
+    plain = copy.copy(tb)
+    plain.cols_final, plain.upd = tb.int_cols, np.zeros((0, 4), dtype=np.int32)
+    plain.reordered, plain.dissect, plain._dev = False, 0, {}
+    T = _children(37, 3, torch.float64, gpu, 5)
+    h = torch.randn(12, tb.nec, 2, device=gpu, dtype=torch.float64)
+    mapped = merge_level(T, h, tb, pivot=pivot)
+    out, kernels, _ = profiling.instrumented(lambda: merge_level(T, h, plain, pivot=pivot))
+    names = [r["name"] for r in kernels]
+    assert names and not any("row_scatter" in nm for nm in names), names
+    fin = torch.as_tensor(tb.final_of_internal, device=gpu).long()
+    bound = 4 * tb.ni * EPS[torch.float64]
+    for nm in ("S", "gt", "T", "h"):
+        a, b = getattr(out, nm), getattr(mapped, nm)
+        b = b[:, fin] if nm in ("S", "gt") else b
+        assert float((a - b).abs().max() / b.abs().max()) < bound, nm
+
+
 def test_merge_beyond_32_bit_indices(gpu):
     """A 3D merge whose S has more than 2^31 elements (32784 x 65568).  Columns
     of S put back into the children: the outgoing data of the two sides of
