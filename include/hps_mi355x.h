@@ -170,8 +170,9 @@ int hps_leaf_condensed(hps_handle_t h, int dtype, int nl, int n, int nb, int nq,
  * stably in their natural order (pivot growth ~1, multipliers below 4 on the
  * Helmholtz and variable-coefficient workloads), while pivoted panels are
  * latency-bound.  With 0, the panel kernels check each matrix and set
- * info = -1 when a multiplier exceeds 64, a pivot is zero or a value is not
- * finite; the caller refactors with pivoting then.  The reference factors
+ * info = -1 when a multiplier exceeds 64 or a pivot is not usable (zero, not
+ * finite, or without a normal reciprocal); the caller refactors with pivoting
+ * then.  The reference factors
  * with LAPACK's pivoted LU inside jnp.linalg.inv
  * (merge/_schur_complement.py:107,146). */
 int hps_set_merge_pivoting(hps_handle_t h, int partial_pivoting);

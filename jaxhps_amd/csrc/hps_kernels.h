@@ -231,8 +231,8 @@ size_t lub_scratch_bytes(const LuPlan& p, int batch);
 // A = L U in natural order, in place (batch matrices, row stride lda, batch
 // stride sA); perm becomes the identity, dinv as getrf_ws's, inv the inverses
 // of every block's L and U (lub_inv_elems), tmp lub_tmp_elems elements.
-// info[b] = -1 where a multiplier exceeds 64, a pivot is zero or a value is not
-// finite (the matrix then needs pivoting), else 0.
+// info[b] = -1 where a multiplier exceeds 64 or a pivot is zero, not finite or
+// without a normal reciprocal (the matrix then needs pivoting), else 0.
 template <typename T>
 hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* perm, T* dinv, T* inv, T* tmp,
                             int* scratch, int* info, int batch, hipStream_t s);

@@ -45,6 +45,15 @@ constexpr int LU_NB = 32;
 // largest multiplier an unpivoted register panel accepts (the leaf and merge
 // matrices of the HPS tree stay below 2)
 constexpr double LU_NOPIV_BOUND = 64.0;
+
+// a pivot that an unpivoted panel accepts, by its magnitude: finite, and with a
+// reciprocal that is a normal number (a zero, infinite, NaN or subnormal pivot
+// is none, nor one within four of the largest value)
+template <typename R>
+__device__ __forceinline__ bool pivot_usable(R mag) {
+  constexpr R lo = 4 * std::numeric_limits<R>::min();
+  return mag >= lo && mag <= R(1) / lo;
+}
 constexpr size_t LU_PANEL_LDS_MAX = 150 * 1024;
 constexpr int SWTAB = 1 + 4 * LU_NB;  // count, then up to 2*NB (row, src) int pairs
 template <typename T> __device__ __forceinline__ T make_conj(T x) { return x; }
@@ -775,7 +784,9 @@ __global__ __launch_bounds__(THREADS) void getrf_panel_rows_kernel(int n, T* A, 
 #pragma unroll
     for (int c = 0; c < LU_NB; ++c) x[r][c] = (live[r] && c < nb) ? P[(long)pos[r] * lda + c] : s_zero<T>();
   }
+  bool usable = true;  // every pivot, in natural order
   auto on_pivot = [&](int J, int pq, R fv, unsigned) {
+    if constexpr (NOPIV) usable = usable && pivot_usable(fv);
     if (t == 0) record_pivot(k, J, pq, fv == R(0), ipivb, info, 0);
   };
   R lmax = R(0);
@@ -783,8 +794,9 @@ __global__ __launch_bounds__(THREADS) void getrf_panel_rows_kernel(int n, T* A, 
                                             lmax);
   if constexpr (NOPIV) {
     // stability check of the natural-order elimination: a multiplier above
-    // LU_NOPIV_BOUND (or not finite) marks the matrix with info = -1, and the
-    // caller refactors with partial pivoting
+    // LU_NOPIV_BOUND (or not finite) or a pivot that is not usable (the last
+    // one has no multipliers) marks the matrix with info = -1, and the caller
+    // refactors with partial pivoting
     __shared__ R wmax[THREADS / 64];
     R v = lmax;
 #pragma unroll
@@ -799,7 +811,7 @@ __global__ __launch_bounds__(THREADS) void getrf_panel_rows_kernel(int n, T* A, 
       for (int w = 1; w < THREADS / 64; ++w) mx = (wmax[w] > mx || wmax[w] != wmax[w]) ? wmax[w] : mx;
       // a zero pivot in the natural order (info > 0) is no verdict on the
       // matrix either: pivoting decides
-      if (!(mx <= R(LU_NOPIV_BOUND)) || info[0] > 0) info[0] = -1;
+      if (!(mx <= R(LU_NOPIV_BOUND)) || !usable || info[0] > 0) info[0] = -1;
     }
   }
   // net row permutation of the panel: every row whose position changed
@@ -1141,8 +1153,8 @@ static int rows_panel_max() {
 // (dinv) and the identity pivots.  The rows are independent: grid
 // (ceil((n - k - nb) / NOPIV_ROWS) + U12 chunks, batch).
 //
-// A matrix with a multiplier above LU_NOPIV_BOUND, a zero pivot or a value
-// that is not finite gets info = -1 (the caller refactors with pivoting).
+// A matrix with a multiplier above LU_NOPIV_BOUND or a pivot that is not usable
+// (pivot_usable) gets info = -1 (the caller refactors with pivoting).
 //
 // Bound by the serial chain of 32 steps (publish, barrier, read, reciprocal,
 // update: about 0.4 us each in float64).  One wave with its rows in registers
@@ -1152,8 +1164,7 @@ static int rows_panel_max() {
 // also leaves no separate inversion and no check of the factors afterwards, 24 / 17 / 19 us.
 // ---------------------------------------------------------------------------
 // 1 / a from the hardware's reciprocal estimate and Newton steps (to the last
-// bit or the one before; zero, infinite and subnormal a give no usable value,
-// which the panel's check reports).  Complex a is first scaled by the power of
+// bit or the one before, for the a that pivot_usable accepts).  Complex a is first scaled by the power of
 // two that brings its larger part to [0.5, 1), so |a|^2 neither overflows nor
 // vanishes.  The reciprocal is on the panel's serial chain: half of a division.
 __device__ __forceinline__ double s_inv_fast(double a) {
@@ -1314,8 +1325,7 @@ __global__ __launch_bounds__(256) void getrf_panel_nopiv_kernel(int n, T* A, lon
 #pragma unroll
         for (int i = 1; i <= jq; ++i) s = s_fma(y[i], pc[i], s);
         s = oct_sum(s);
-        const R ap = s_abs1(piv);
-        ok = ok && ap > R(0) && ap <= std::numeric_limits<R>::max();
+        ok = ok && pivot_usable(s_abs1(piv));
         if (r > j) {
           const T l = s_mul(xr, inv);
           ok = ok && s_mod2(l) <= BOUND2;
