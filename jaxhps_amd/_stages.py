@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import ctypes
 from dataclasses import dataclass
-from typing import List, Optional
+from typing import List, Optional, Tuple
 
 import numpy as np
 import torch
@@ -58,8 +58,8 @@ def complex_dtype(dt):
 
 @dataclass
 class LeafResult:
-    Y: torch.Tensor
-    T: torch.Tensor
+    Y: Optional[torch.Tensor]
+    T: Optional[torch.Tensor]
     v: Optional[torch.Tensor]
     h: Optional[torch.Tensor]
     lu: torch.Tensor
@@ -84,6 +84,8 @@ class Condensed:
     dinv: torch.Tensor
     X: torch.Tensor     # (nl, ni, nb + 2 nsrc) real: A_ii^{-1} [A_ib | f_i]
     Gi: torch.Tensor    # (nb, ni) real: interior columns of G
+    # leaves that rejected the condensation, and their factorisation of B
+    redone: Optional[Tuple[torch.Tensor, LeafResult]] = None
 
 
 def iti_row_scale(pde, coeffs, clist, device):
@@ -138,14 +140,7 @@ def leaf_solve(pde, kind: int, dtype, device, source=None, nsrc_zero=False, leaf
     sizes with operators built for half side 1 -- each coefficient of a
     k-th order term is scaled by half^-k and T, h by 1/half (the operators
     are homogeneous in the half side)."""
-    lib = load_library()
-    h = _lib.handle()
-    dom = pde.domain
-    nl = dom.n_leaves
-    n = dom.p**2 if dom.bool_2D else dom.p**3
     ops = pde.device_ops(device, dtype)
-    P, Q = ops["P"], ops["Q"]
-    nb, nq = P.shape
     names = pde.operator_names()
     clist = pde.coefficient_list()
     if not clist:
@@ -162,7 +157,7 @@ def leaf_solve(pde, kind: int, dtype, device, source=None, nsrc_zero=False, leaf
             nsrc = source.shape[-1]
             src = source
     if kind == HPS_KIND_ITI and not is_complex_input(*[a for _, a in clist]):
-        res = _leaf_condensed(pde, dtype, device, clist, coef_ops, src, nsrc)
+        res = _leaf_condensed(pde, ops, dtype, device, clist, coef_ops, src, nsrc)
         if res is not None:
             return res
     coeffs = torch.stack([to_device(a, device, dtype) for _, a in clist]).contiguous()
@@ -174,6 +169,22 @@ def leaf_solve(pde, kind: int, dtype, device, source=None, nsrc_zero=False, leaf
             order = 0 if nm == "I" else len(nm) - 2
             if order:
                 scale_batched(coeffs[k], inv if order == 1 else inv2)
+    res = _leaf_direct(pde, ops, kind, dtype, device, clist, coef_ops, coeffs, src, nsrc)
+    if leaf_half_sides is not None:
+        scale_batched(res.T, inv)
+        if res.h is not None:
+            scale_batched(res.h, inv)
+    return res
+
+
+def _leaf_direct(pde, ops, kind, dtype, device, clist, coef_ops, coeffs, src, nsrc) -> LeafResult:
+    """Leaf stage by the factorisation of the whole leaf matrix, over the
+    leaves of coeffs (ncoef, nl, n) and src (nl, n, nsrc)."""
+    lib = load_library()
+    h = _lib.handle()
+    nl, n = coeffs.shape[1:]
+    P, Q = ops["P"], ops["Q"]
+    nb, nq = P.shape
     nrows = n - nb if kind == HPS_KIND_DTN else n
     Y = torch.empty((nl, n, nq), dtype=dtype, device=device)
     T = torch.empty((nl, nq, nq), dtype=dtype, device=device)
@@ -211,16 +222,24 @@ def leaf_solve(pde, kind: int, dtype, device, source=None, nsrc_zero=False, leaf
         lib.hps_set_leaf_pivoting(h, 1)
     if bool((info < 0).any()):
         run()
-    if leaf_half_sides is not None:
-        scale_batched(T, inv)
-        if hv is not None:
-            scale_batched(hv, inv)
     return LeafResult(Y, T, v, hv, lu, perm, dinv, info, kind, row_scale, nb)
 
 
-def _leaf_condensed(pde, dtype, device, clist, coef_ops, src, nsrc) -> Optional[LeafResult]:
-    """ItI leaf stage with real coefficients by static condensation; None
-    where a leaf rejects it (its interior problem is close to singular)."""
+# A leaf whose interior problem is close to singular rejects the condensation
+# (a few in a hundred of the wavenumbers past the leaf's first Dirichlet
+# eigenvalue do).  With at least this many leaves, one a CU, the rejected ones
+# alone are factored directly (p = 16, L = 7 at k h = 6, 510 of 16384 leaves
+# rejected: build 137 ms, with every leaf factored directly after them 191);
+# fewer leaves take as long as one, and one kind of factors is then half the
+# launches of every later solve.
+LEAF_REDO_MIN = 256
+
+
+def _leaf_condensed(pde, full_ops, dtype, device, clist, coef_ops, src, nsrc) -> Optional[LeafResult]:
+    """ItI leaf stage with real coefficients by static condensation, the leaves
+    that reject it by the factorisation of B.  None where all leaves are to be
+    factored that way: G's interior columns are not real, most leaves reject, or
+    some of less than LEAF_REDO_MIN."""
     ops = pde.condensed_ops(device, dtype)
     if ops is None:
         return None
@@ -251,10 +270,20 @@ def _leaf_condensed(pde, dtype, device, clist, coef_ops, src, nsrc) -> Optional[
         ws.numel(),
     )
     check(rc, h, "hps_leaf_condensed")
+    res = LeafResult(Y, T, v, hv, slu, sperm, sdinv, info, HPS_KIND_ITI, None, nb,
+                     Condensed(alu, aperm, adinv, X, ops["GQ"][:nb]))
     if bool((info < 0).any()):
-        return None
-    return LeafResult(Y, T, v, hv, slu, sperm, sdinv, info, HPS_KIND_ITI, None, nb,
-                      Condensed(alu, aperm, adinv, X, ops["GQ"][:nb]))
+        idx = (info < 0).nonzero().flatten()
+        if nl < LEAF_REDO_MIN or 2 * idx.numel() > nl:
+            return None
+        sub = _leaf_direct(pde, full_ops, HPS_KIND_ITI, dtype, device, clist, coef_ops, coeffs[:, idx].to(dtype).contiguous(),
+                           None if src is None else src[idx], nsrc)
+        for dst, part in ((Y, sub.Y), (T, sub.T), (v, sub.v), (hv, sub.h), (info, sub.info)):
+            if dst is not None:
+                dst[idx] = part
+        sub.Y = sub.T = sub.v = sub.h = None
+        res.condensed.redone = (idx, sub)
+    return res
 
 
 @dataclass
@@ -507,6 +536,9 @@ def _apply_inverse_condensed(leaf: LeafResult, rhs):
     check(rc, hd, "hps_getrs_batched")
     gemm_at(rdt, ni, w2, nb, -1.0, ptr(c.X), wr, ni * wr, at(out), w2, n * w2, 1.0, at(out, nb * w), w2, n * w2,
             at(out, nb * w), w2, n * w2, nl)
+    if c.redone is not None:
+        idx, sub = c.redone
+        out[idx] = leaf_apply_inverse(sub, rhs[idx])
     return out
 
 

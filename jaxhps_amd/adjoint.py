@@ -74,6 +74,7 @@ def _condensed_inverse_conjt(leaf, v):
     """B^{-H} v through the condensed leaf factors (hps_leaf_condensed):
     x_b = S^{-H}(v_b - X_b^T v_i), x_i = A_ii^{-T}(v_i - G_i^T x_b)."""
     c = leaf.condensed
+    v = v.contiguous()
     nl, n, w = v.shape
     nb, ni = c.Gi.shape
     rdt = c.alu.dtype
@@ -86,7 +87,28 @@ def _condensed_inverse_conjt(leaf, v):
     gemm_at(rdt, ni, w2, nb, -1.0, ptr(c.Gi), ni, 0, at(xb), w2, nb * w2, 1.0, at(v, nb * w), w2, n * w2, at(y), w2,
             ni * w2, nl, conjt=True)
     xi = getrs_conjt(ni, c.alu, nb, n, ni * n, c.perm, c.dinv, y)
-    return torch.cat([xb, torch.view_as_complex(xi.view(nl, ni, w, 2))], dim=1)
+    out = torch.cat([xb, torch.view_as_complex(xi.view(nl, ni, w, 2))], dim=1)
+    if c.redone is not None:
+        idx, sub = c.redone
+        out[idx] = _leaf_inverse_conjt(sub, v[idx])
+    return out
+
+
+def _leaf_inverse_conjt(leaf, v):
+    """(leaf operator)^{-H} v for v (n_leaves, n, w); zero on a DtN leaf's boundary."""
+    if leaf.condensed is not None:
+        return _condensed_inverse_conjt(leaf, v)
+    _, nrows, n = leaf.lu.shape
+    if leaf.kind == HPS_KIND_ITI:
+        # the factors are of B' = diag(s, 1) B, so B^{-H} = diag(s, 1) B'^{-H}
+        lam = getrs_conjt(n, leaf.lu, 0, n, n * n, leaf.perm, leaf.dinv, v)
+        if leaf.row_scale is not None:
+            lam[:, : leaf.nb, :] *= leaf.row_scale.to(lam.real.dtype)
+        return lam
+    nb = n - nrows
+    lam = torch.zeros_like(v)
+    lam[:, nb:, :] = getrs_conjt(nrows, leaf.lu, nb, n, nrows * n, leaf.perm, leaf.dinv, v[:, nb:, :].contiguous())
+    return lam
 
 
 def _adjoint_down_level(gbar_children, S, tables):
@@ -157,19 +179,7 @@ def adjoint_lambda(pde_problem, G):
     # 4. vbar = G + Q^H hbar_leaf ; lambda = (leaf operator)^{-H} vbar
     Q = pde_problem.device_ops(dev, dt)["Q"]
     vbar = _gemm_conjt(Q, n, 0, n, nq, hbar.contiguous(), w, nq * w, w, nl, C=Gd, beta=1.0)
-    _, nrows, _ = leaf.lu.shape
-    if leaf.condensed is not None:
-        lam = _condensed_inverse_conjt(leaf, vbar)
-    elif leaf.kind == HPS_KIND_ITI:
-        # the factors are of B' = diag(s, 1) B, so B^{-H} = diag(s, 1) B'^{-H}
-        lam = getrs_conjt(n, leaf.lu, 0, n, n * n, leaf.perm, leaf.dinv, vbar)
-        if leaf.row_scale is not None:
-            lam[:, : leaf.nb, :] *= leaf.row_scale.to(lam.real.dtype)
-    else:
-        nb = n - nrows
-        lam = torch.zeros_like(vbar)
-        lam[:, nb:, :] = getrs_conjt(nrows, leaf.lu, nb, n, nrows * n, leaf.perm, leaf.dinv,
-                                     vbar[:, nb:, :].contiguous())
+    lam = _leaf_inverse_conjt(leaf, vbar)
     return lam[..., 0] if squeeze else lam
 
 

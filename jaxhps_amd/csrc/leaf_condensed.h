@@ -19,7 +19,7 @@
 // values into the leaf and is of size 1 otherwise, then grows without bound.
 // A leaf with an entry of X_b above LEAF_EXT_BOUND (or not finite, or with a
 // rejected factorisation) gets info = -1, and the caller takes the
-// factorisation of B.
+// factorisation of B for it.
 //
 // Measured: leaf stage at p = 16, L = 7 (16384 leaves, complex128) 57 ms by the
 // LU of B, 33 ms condensed; Helmholtz build + solve there 159 / 135 ms, its

@@ -327,6 +327,102 @@ def test_condensed_leaves_give_way(gpu):
         assert err <= 64 * 2.0**-53 * np.linalg.cond(B), err
 
 
+def _resonant_leaf(gpu, p, L):
+    """_iti_leaves with the zeroth-order coefficient for which leaf 0's interior
+    problem is singular."""
+    pde, nb, matrix = _iti_leaves(gpu, p, L, 0.0)
+    x = pde.domain.interior_points[0, nb:]
+    A, W = matrix(0)[nb:, nb:].real, 1.0 + 0.3 * np.cos(x[:, 0] + x[:, 1])
+    w = np.linalg.eigvals(-A / W[:, None])
+    return _iti_leaves(gpu, p, L, float(w[np.abs(w.imag) < 1e-9].real.min()))
+
+
+@pytest.mark.parametrize("nsrc,dtype", [(0, torch.complex128), (2, torch.complex128), (1, torch.complex64)])
+def test_rejected_leaves_alone_are_redone(gpu, nsrc, dtype):
+    """Among 256 leaves the few that reject the condensation are factored
+    directly and the others stay condensed; Y, T, v, h, B^{-1} and B^{-H} of
+    both kinds against numpy solves with B (16, the extension's bound, times
+    the bound of test_condensed_leaves)."""
+    from jaxhps_amd._stages import HPS_KIND_ITI, leaf_apply_inverse, leaf_solve
+    from jaxhps_amd.adjoint import _leaf_inverse_conjt
+
+    print(f"rejected leaves redone nsrc={nsrc} {dtype}", flush=True)
+    pde, nb, matrix = _resonant_leaf(gpu, 8, 4)
+    nl, n = 256, 64
+    g = torch.Generator(device=gpu).manual_seed(3)
+    f = torch.randn(nl, n, max(nsrc, 1), generator=g, device=gpu, dtype=dtype)
+    res = leaf_solve(pde, HPS_KIND_ITI, dtype, gpu, source=f if nsrc else None, nsrc_zero=nsrc == 0)
+    assert res.condensed is not None and res.condensed.redone is not None
+    redone = res.condensed.redone[0].cpu().tolist()
+    assert 0 in redone and len(redone) <= nl // 4 and (res.info == 0).all()
+    inv, invh = leaf_apply_inverse(res, f), _leaf_inverse_conjt(res, f)
+    assert bool(torch.isfinite(inv.abs()).all()) and bool(torch.isfinite(invh.abs()).all())
+    P, QH = np.asarray(pde.P), np.asarray(pde.QH)
+    kept = [leaf for leaf in range(nl) if leaf not in redone]
+    for leaf in {0, redone[-1], kept[0], kept[-1]}:
+        B = matrix(leaf)
+        scale = np.ones(n)
+        scale[:nb] = np.abs(B[nb:]).max() / np.abs(B[:nb]).max()
+        bound = 16 * n * EPS[dtype] * np.linalg.cond(scale[:, None] * B)
+        fl = f[leaf].cpu().numpy().astype(complex)
+        fi = fl.copy()
+        fi[:nb] = 0.0
+        rhs = np.zeros((n, P.shape[1]), dtype=complex)
+        rhs[:nb] = P
+        ref = {"Y": np.linalg.solve(B, rhs), "inv": np.linalg.solve(B, fl), "invh": np.linalg.solve(B.conj().T, fl)}
+        got = {"Y": res.Y, "inv": inv, "invh": invh}
+        size = {nm: np.abs(r).max() for nm, r in ref.items()}
+        pairs = [("T", "Y", res.T)]
+        if nsrc:
+            ref["v"], got["v"] = np.linalg.solve(B, fi), res.v
+            size["v"] = np.abs(ref["v"]).max()
+            pairs.append(("h", "v", res.h))
+        for nm, of, t in pairs:  # the error of Y and v through QH
+            ref[nm], got[nm], size[nm] = QH @ ref[of], t, np.abs(QH).sum(1).max() * size[of]
+        for nm, r in ref.items():
+            err = np.abs(got[nm][leaf].cpu().numpy() - r).max() / size[nm]
+            assert err <= bound, (nm, leaf, err, bound)
+
+
+def test_solves_with_rejected_leaves(gpu):
+    """Build + solve, a new source and a gradient where some leaves reject the
+    condensation, against the same problem with its coefficients given as complex
+    numbers (every leaf factored directly).  Both solve one system whose
+    condition is below 1e6."""
+    import jaxhps_amd as jh
+    from jaxhps_amd.adjoint import differentiable_solve
+
+    print("solves with rejected leaves", flush=True)
+    pde, _, _ = _resonant_leaf(gpu, 8, 4)
+    dom = pde.domain
+    cf = {f"{nm}_coefficients": torch.as_tensor(a, device=gpu) for nm, a in pde.coefficient_list()}
+    g = torch.Generator(device=gpu).manual_seed(4)
+    src, src2 = (torch.randn(256, 64, generator=g, device=gpu, dtype=torch.complex128) for _ in range(2))
+    bd = torch.randn(dom.boundary_points.shape[0], generator=g, device=gpu, dtype=torch.complex128)
+    got = []
+    for cast in (lambda t: t, lambda t: t.to(torch.complex128)):
+        p1 = jh.PDEProblem(dom, source=src, use_ItI=True, eta=3.0, **{k: cast(a) for k, a in cf.items()})
+        jh.build_solver(p1)
+        c = p1._factors["leaf"].condensed
+        assert (c is not None and c.redone is not None) == (len(got) == 0)
+        out = [jh.solve(p1, bd)]
+        p2 = jh.PDEProblem(dom, use_ItI=True, eta=3.0, **{k: cast(a) for k, a in cf.items()})
+        jh.build_solver(p2)
+        out.append(jh.solve(p2, bd, source=src2))
+        if not got:
+            field = cf["I_coefficients"].clone().requires_grad_(True)
+            u = differentiable_solve(p1, bd, I=field)
+            (grad,) = torch.autograd.grad((u.abs() ** 2).sum(), field)
+        else:
+            from jaxhps_amd.adjoint import adjoint_lambda, coefficient_gradients
+
+            lam = adjoint_lambda(p1, 2.0 * out[0])
+            grad = coefficient_gradients(p1, out[0], lam)["I"]
+        got.append(out + [grad])
+    for nm, a, b in zip(("solve", "source", "gradient"), *got):
+        assert float((a - b).abs().max() / b.abs().max()) < 1e6 * 64 * 2.0**-53, nm
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("batch,M,N,K", [(1, 1, 1, 1), (3, 17, 2, 63), (2, 64, 1, 64), (2, 65, 2, 257), (1, 300, 1, 5),
                                          (5, 33, 1, 1000)])
