@@ -48,6 +48,22 @@ def check_input_shapes(source, use_ItI, expected_shape, **coeffs) -> None:
             )
 
 
+class _DeviceOps(dict):
+    """Host operators (arrays, or lists of arrays to be stacked) on the device
+    in one dtype, each converted and uploaded when it is first read: a stage
+    that reads some of them does not pay for the others."""
+
+    def __init__(self, host, device, dtype):
+        super().__init__()
+        self.host, self.device, self.dtype = host, device, dtype
+
+    def __missing__(self, name):
+        x = self.host[name]
+        x = np.ascontiguousarray(np.stack(x) if isinstance(x, list) else x)
+        self[name] = t = torch.as_tensor(x).to(device=self.device, dtype=self.dtype)
+        return t
+
+
 class PDEProblem:
     """Elliptic problem L u = f on a uniform HPS Domain.
 
@@ -225,22 +241,16 @@ class PDEProblem:
         return [n for n in (COEFF_NAMES_2D if self.domain.bool_2D else COEFF_NAMES_3D) if n != "I"]
 
     def device_ops(self, device, dtype):
-        """Stacked diff operators and P/Q (or P/QH/G) on the device in `dtype`."""
+        """Stacked diff operators and P/Q (or P/QH/G) on the device in `dtype`,
+        each uploaded when it is first read."""
         key = (str(device), dtype)
         if key not in self._dev_cache:
-            names = self.operator_names()
-            ops = np.stack([getattr(self, n) for n in names])
-
-            def dev(x):
-                return torch.as_tensor(np.ascontiguousarray(x)).to(device=device, dtype=dtype)
-
-            d = {"diffops": dev(ops), "P": dev(self.P)}
+            host = {"diffops": [getattr(self, n) for n in self.operator_names()], "P": self.P}
             if self.use_ItI:
-                d["Q"] = dev(self.QH)
-                d["G"] = dev(self.G)
+                host.update(Q=self.QH, G=self.G)
             else:
-                d["Q"] = dev(self.Q)
-            self._dev_cache[key] = d
+                host["Q"] = self.Q
+            self._dev_cache[key] = _DeviceOps(host, device, dtype)
         return self._dev_cache[key]
 
     def condensed_ops(self, device, dtype):
@@ -262,8 +272,7 @@ class PDEProblem:
                     return torch.as_tensor(np.ascontiguousarray(x)).to(device=device, dtype=dt)
 
                 self._dev_cache[key] = {
-                    "diffops": dev(np.stack([getattr(self, n) for n in self.operator_names()]), real),
+                    "diffops": self.device_ops(device, real)["diffops"], "P": self.device_ops(device, dtype)["P"],
                     "GQ": dev(GQ.real, real), "Gb": dev(G[:, :nb], dtype), "Qb": dev(QH[:, :nb], dtype),
-                    "P": dev(self.P, dtype),
                 }
         return self._dev_cache[key]

@@ -196,12 +196,11 @@ def _leaf_direct(pde, ops, kind, dtype, device, clist, coef_ops, coeffs, src, ns
     info = torch.empty((nl,), dtype=torch.int32, device=device)
     ws = workspace(lib.hps_leaf_workspace(dtype_code(dtype), kind, nl, n, nb, nq, nsrc), device)
     cop = coef_ops.ctypes.data_as(ctypes.c_void_p)
-    G = ops.get("G")
-    row_scale = None
+    G = row_scale = None
     if kind == HPS_KIND_ITI:
         row_scale = iti_row_scale(pde, coeffs, clist, device)
         rs = row_scale.to(real_dtype(dtype))
-        G = (G * rs).contiguous()
+        G = (ops["G"] * rs).contiguous()
         P = (P * rs).contiguous()
 
     def run():

@@ -303,6 +303,19 @@ def test_condensed_leaves(gpu, p, L, nsrc, dtype):
             assert err <= bound, (nm, leaf, err, bound)
 
 
+def test_condensed_build_leaves_the_complex_operators_alone(gpu):
+    """A build whose leaves are condensed uploads the real differentiation
+    operators, not a complex set beside them (a problem object per coefficient
+    field pays for each)."""
+    import jaxhps_amd as jh
+
+    print("condensed build's operators", flush=True)
+    pde, _, _ = _iti_leaves(gpu, 8, 2, 4.0)
+    jh.build_solver(pde)
+    assert pde._factors["leaf"].condensed is not None
+    assert not {"diffops", "G"} & set(pde.device_ops(gpu, torch.complex128))
+
+
 def test_condensed_leaves_give_way(gpu):
     """Complex coefficients, and a leaf at an eigenvalue of its Dirichlet
     problem, take the factorisation of B; the results stay right."""

@@ -235,6 +235,25 @@ def test_library_argument_errors_without_gpu():
     assert lib.hps_destroy(h) == 0
 
 
+def test_device_operators_are_uploaded_when_read():
+    """A stage that reads one operator does not convert and upload the others."""
+    import torch
+
+    import jaxhps_amd as jh
+
+    dom = jh.Domain(p=6, q=4, root=jh.DiscretizationNode2D(-1.0, 1.0, -1.0, 1.0), L=1)
+    one = np.ones(dom.interior_points.shape[:2])
+    pde = jh.PDEProblem(dom, D_xx_coefficients=one, I_coefficients=one, use_ItI=True, eta=2.0)
+    ops = pde.device_ops("cpu", torch.complex128)
+    assert set(ops) == set()
+    np.testing.assert_array_equal(ops["Q"].numpy(), pde.QH)
+    assert set(ops) == {"Q"} and pde.device_ops("cpu", torch.complex128)["Q"] is ops["Q"]
+    con = pde.condensed_ops("cpu", torch.complex128)
+    assert set(ops) == {"P", "Q"} and con["diffops"].dtype == torch.float64
+    np.testing.assert_array_equal(ops["diffops"].numpy(), np.stack([getattr(pde, n) for n in pde.operator_names()]))
+    np.testing.assert_array_equal(ops["G"].numpy(), pde.G)
+
+
 def test_each_thread_has_its_own_handle(monkeypatch):
     """A handle carries pivoting and dissection from the set call to the stage
     call, so two threads on one stream must not share it; a thread's handles
