@@ -235,6 +235,22 @@ def test_library_argument_errors_without_gpu():
     assert lib.hps_destroy(h) == 0
 
 
+def test_inputs_hold_their_values_in_memory():
+    """Autograd hands over conjugated views (a loss with u.conj()); kernels read
+    memory, so the inputs are written out first."""
+    import torch
+
+    from jaxhps_amd._stages import to_device
+
+    x = torch.randn(3, 4, dtype=torch.complex128)
+    for view in (x.conj(), x.mH, x.conj().imag):
+        t = to_device(view, "cpu", view.dtype)
+        raw = np.ctypeslib.as_array((ctypes.c_double * (t.numel() * (2 if t.is_complex() else 1)))
+                                    .from_address(t.data_ptr())).copy()
+        ref = view.resolve_conj().resolve_neg().contiguous()
+        np.testing.assert_array_equal(raw, (torch.view_as_real(ref) if ref.is_complex() else ref).numpy().reshape(-1))
+
+
 def test_device_operators_are_uploaded_when_read():
     """A stage that reads one operator does not convert and upload the others."""
     import torch
