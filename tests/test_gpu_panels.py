@@ -92,6 +92,66 @@ def test_last_pivot_is_checked(gpu, dtype, nm):
         assert info[2] == -1 and (np.delete(info, 2) == 0).all(), (value, info)
 
 
+def _natural_lu(A):
+    """L and U of A without row exchanges (numpy)."""
+    A = A.copy()
+    for k in range(len(A) - 1):
+        A[k + 1:, k] /= A[k, k]
+        A[k + 1:, k + 1:] -= np.outer(A[k + 1:, k], A[k, k + 1:])
+    return np.tril(A, -1), np.triu(A)
+
+
+def _entries(tb, i, j):
+    """The children's entries (child, row, column) that make D[i, j]."""
+    r, c = tb.int_rows[i], tb.int_cols[j]
+    return [(int(r[a]), int(r[a + 1]), int(c[b + 1])) for a in (0, 2) for b in (0, 2) if r[a] == c[b]]
+
+
+# D[row, col] gets the large multiplier, outside every diagonal block
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.complex128])
+@pytest.mark.parametrize("kind,m,nm,row,col", [
+    ("quad", 40, 3, 150, 3),      # dense, 32 + 128 unknowns: the panel copied back
+    ("quad", 25, 1024, 99, 2),    # many matrices, 36 + 64: in place, panel_check_kernel
+    ("quad", 50, 3, 101, 60),     # dissected, one 50-wide block a group: later rows of group 1, in place
+    ("quad", 70, 3, 279, 75),     # 70-wide blocks: later rows of group 1, copied back
+    ("quad", 150, 2, 299, 155),   # 22 + 128 a group: rows of group 1 itself
+    ("oct", 50, 2, 520, 160),     # group 3 of the x-interfaces, rows of a z-interface
+    ("oct", 70, 1, 459, 430),     # the second slab's y-interfaces (12 + 128)
+])
+def test_multipliers_outside_the_diagonal_blocks_are_checked(gpu, dtype, kind, m, nm, row, col):
+    """A multiplier above 64 in L21 alone marks its matrix, and no other, with
+    info = -1: every diagonal block of the bad matrix factors well."""
+    from jaxhps_amd._stages import merge_level
+    from jaxhps_amd._tables import oct_merge_tables, quad_merge_tables
+
+    print(f"multipliers outside {kind} m={m} nm={nm} D[{row}, {col}] {dtype}", flush=True)
+    tb = oct_merge_tables(m) if kind == "oct" else quad_merge_tables(m, "dtn")
+    g = torch.Generator(device=gpu).manual_seed(m)
+    T = torch.randn(tb.nc * nm, tb.nec, tb.nec, generator=g, device=gpu, dtype=torch.float64).to(dtype)
+    T = 0.1 * T / tb.nec**0.5 + 2.0 * torch.eye(tb.nec, device=gpu, dtype=dtype)
+    bad = nm - 1
+    assert (merge_level(T, None, tb, pivot=False).info == 0).all()
+    # row `col` of D keeps its diagonal entry alone, so that eliminating it spreads nothing
+    for j in range(tb.ni):
+        for c, lr, lc in _entries(tb, col, j):
+            if j != col:
+                T[tb.nc * bad + c, lr, lc] = 0.0
+    c, lr, lc = _entries(tb, row, col)[0]
+    T[tb.nc * bad + c, lr, lc] = 1000.0
+    # the oracle: of all multipliers that one alone passes the bound
+    Tb = T[tb.nc * bad:].cpu().numpy().astype(complex)
+    D = np.zeros((tb.ni, tb.ni), dtype=complex)
+    for i in range(tb.ni):
+        for a in (0, 2):
+            for b in (0, 2):
+                hit = tb.int_cols[:, b] == tb.int_rows[i, a]
+                D[i, hit] += Tb[tb.int_rows[i, a], tb.int_rows[i, a + 1], tb.int_cols[hit, b + 1]]
+    L, _ = _natural_lu(D)
+    assert [tuple(x) for x in np.argwhere(np.abs(L) > 32)] == [(row, col)]
+    info = merge_level(T, None, tb, pivot=False).info.cpu().numpy()
+    assert info[bad] == -1 and (np.delete(info, bad) == 0).all(), info
+
+
 @pytest.mark.parametrize("kind,m,nm,dtype", [
     ("quad", 47, 2, torch.float64), ("quad", 48, 3, torch.float32), ("quad", 65, 2, torch.complex128),
     ("quad", 129, 1, torch.float64), ("quad", 20, 40, torch.complex64), ("oct", 47, 1, torch.float64),
