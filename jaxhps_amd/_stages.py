@@ -33,8 +33,9 @@ def to_device(x, device, dtype):
         t = torch.as_tensor(np.asarray(x))
     if not t.is_complex() and dtype.is_complex:
         t = t.to(torch.float64)
+    t = t.to(device=device, dtype=dtype).contiguous()
     # the kernels read the memory: a view that is conjugated or negated on read is written out
-    return t.to(device=device, dtype=dtype).contiguous().resolve_conj().resolve_neg()
+    return t.resolve_conj().resolve_neg() if t.is_conj() or t.is_neg() else t
 
 
 def is_complex_input(*arrs) -> bool:

@@ -612,8 +612,11 @@ static bool merge_block_inverses(int dtype, int nfac, int nm) {
 
 // The elimination's structure of a merge: HPS_DISSECT_* (DtN) or dense.  Below
 // MERGE_DISSECT_MIN unknowns an interface the stages' extra launches cost more
-// than the zeros they leave out: the p = 8, L = 3 Poisson tree (6 .. 24 an
-// interface) took 1.08 ms with stages everywhere, 0.87 ms without.
+// than the zeros they leave out, in 2D and in 3D.  One level in float64, in
+// stages / densely: 16 2D merges with interfaces of 24 285 / 209 us, of 40 395 /
+// 359, of 48 422 / 424, of 64 498 / 532; 8 3D merges with 25 1166 / 1040, with 36
+// 1555 / 1425, with 48 1860 / 1875, with 64 2377 / 2615.  (float32 and 1 to 256
+// merges cross at the same place.)
 constexpr int MERGE_DISSECT_MIN = 48;
 static LuPlan merge_plan(int dissect, int nfac, int ne, int nm) {
   if (dissect == HPS_DISSECT_QUAD && nfac / 4 >= MERGE_DISSECT_MIN) return lu_plan_quad(nfac / 4);

@@ -197,7 +197,10 @@ inline LuPlan lu_plan_oct(int m) {
 // products of every step are whole tiles; the first block takes the remainder
 // (with 64-wide blocks one of up to 16 joins the first whole block: 196 unknowns
 // are 68 + 64 + 64, where 64 + 64 + 64 + 4 left 132 and 68 unknowns to nine and
-// four 64 x 64 tiles).
+// four 64 x 64 tiles).  A level of 1024 float64 merges of 68, 72, 80 unknowns,
+// joined / in a block of its own: 920 / 990, 960 / 1026, 1090 / 1145 us; 132 and
+// 144 unknowns 3062 / 3174, 3344 / 3425.  From 84 to 96 unknowns (20 to 32 over)
+// joining would still gain 3 to 4 %.
 inline int lub_first(const LuPlan& p, int size) {
   if (size <= p.nbmax) return size;
   const int r = size % p.nbmax;

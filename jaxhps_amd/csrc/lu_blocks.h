@@ -26,7 +26,14 @@
 
 namespace hps {
 
-// parts up to which the unpivoted panel kernel takes the diagonal blocks
+// Parts up to which the unpivoted panel kernel takes the diagonal blocks (its
+// workgroups repeat the diagonal block, up to five of them a part), above it one
+// workgroup a part with its rows in registers: the repeated work has to stay
+// small beside the GPU's 256 CUs.  A level of merges with 112 unknowns each
+// (float64 DtN; complex128 ItI), spread / one workgroup: 16 merges 246 / 318; 437
+// / 528 us, 96 merges 339 / 404; 821 / 898, 256 merges 631 / 683; 1705 / 1728, 512
+// merges 1129 / 1158; 3160 / 3088: the two meet between 256 and 512 parts, so
+// levels of 97 to 256 give up 1 to 14 %.
 constexpr int LUB_SPREAD_PARTS = 96;
 
 // widest block whose products with its inverses run in place: the GEMM's tile
@@ -267,9 +274,7 @@ static hipError_t diag_block_lu(int nb, Parts<T> A, T* db, int* arrivals, int* s
   for (int k = 0; k < nb; k += LU_NB) {
     const int kb = nb - k < LU_NB ? nb - k : LU_NB, m = nb - k;
     const double pf = flop_mult<T>() * parts * ((double)m * kb * kb - (double)kb * kb * kb / 3.0);
-    // few matrices: the unpivoted panel (its workgroups repeat the diagonal
-    // block, up to five of them a matrix); many: one workgroup per matrix with
-    // its rows in registers.  The line is where the repeated work fills the GPU.
+    // few parts: the unpivoted panel; many: one workgroup a part
     if (parts <= LUB_SPREAD_PARTS) {
       static const std::string nm_np = std::string("getrf_panel_nopiv<") + tname<T>() + ">";
       prof::Scope ps(s, nm_np.c_str(), pf, 2.0 * sizeof(T) * (double)m * kb * parts);
