@@ -115,8 +115,8 @@ int hps_leaf_solve(hps_handle_t h, int dtype, int kind, int nl, int n, int nb, i
  *   with aperm, adinv;  X (nl, n-nb, nb + 2 nsrc): e, A_ii^{-1} [A_ib | f_i]
  *   (the sources' columns as (re, im) pairs);  slu (nl, nb, nb) = LU(S) with
  *   sperm, sdinv;  info[l] = -1 where the condensation is not to be used (a
- *   rejected factorisation, or an entry of X_b above 16: A_ii close to a
- *   Dirichlet eigenvalue), and the caller takes hps_leaf_solve for that leaf.
+ *   multiplier above 4 in A_ii's or above 10 in S's elimination, or an entry of
+ *   X_b above 2: A_ii is not definite, or S close to singular), and the caller takes hps_leaf_solve for that leaf.
  * Replaces local_solve_stage_uniform_2D_ItI + get_ItI
  *   (local_solve/_uniform_2D_ItI.py:10-193), which inverts B. */
 size_t hps_leaf_condensed_workspace(int dtype, int nl, int n, int nb, int nq, int nsrc);

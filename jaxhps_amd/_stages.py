@@ -226,21 +226,38 @@ def _leaf_direct(pde, ops, kind, dtype, device, clist, coef_ops, coeffs, src, ns
     return LeafResult(Y, T, v, hv, lu, perm, dinv, info, kind, row_scale, nb)
 
 
-# A leaf whose interior problem is close to singular rejects the condensation
-# (a few in a hundred of the wavenumbers past the leaf's first Dirichlet
-# eigenvalue do).  With at least this many leaves, one a CU, the rejected ones
-# alone are factored directly (p = 16, L = 7 at k h = 6, 510 of 16384 leaves
-# rejected: build 137 ms, with every leaf factored directly after them 191);
-# fewer leaves take as long as one, and one kind of factors is then half the
-# launches of every later solve.
+# A leaf whose interior problem is not safely definite is factored directly: one
+# whose I / (D_xx + D_yy) exceeds this part of the first Dirichlet eigenvalue
+# (pi / h)^2 somewhere, or one that the condensed stage rejects.
+LEAF_DEFINITE = 0.9
+# With at least this many leaves, one a CU, and at most this share of such ones,
+# they alone are factored directly: fewer leaves take as long as one, and one
+# kind of factors is then half the launches of every later solve; and the
+# condensed stage of all leaves plus a larger share costs more than factoring
+# every leaf directly (p = 16, L = 7: 33 ms and 57 ms).
 LEAF_REDO_MIN = 256
+LEAF_REDO_SHARE = 0.4
+
+
+def _too_many(count, nl):
+    return count > 0 and (nl < LEAF_REDO_MIN or count > LEAF_REDO_SHARE * nl)
+
+
+def _indefinite_leaves(pde, coeffs, clist) -> np.ndarray:
+    """Which leaves' interior problems may not be definite (LEAF_DEFINITE), from
+    the coefficients alone; one that is not finite counts as such."""
+    c = {nm: t for (nm, _), t in zip(clist, coeffs)}
+    second = [c[nm] for nm in ("D_xx", "D_yy") if nm in c]
+    if "I" not in c or not second:
+        return np.zeros(coeffs.shape[1], dtype=bool)  # the condensed stage's own checks decide
+    ratio = (c["I"] / (second[0] + second[1] if len(second) == 2 else second[0])).amax(dim=1)
+    return ~(ratio.cpu().numpy() * (2 * pde.half_side_len / np.pi) ** 2 <= LEAF_DEFINITE)
 
 
 def _leaf_condensed(pde, full_ops, dtype, device, clist, coef_ops, src, nsrc) -> Optional[LeafResult]:
     """ItI leaf stage with real coefficients by static condensation, the leaves
-    that reject it by the factorisation of B.  None where all leaves are to be
-    factored that way: G's interior columns are not real, most leaves reject, or
-    some of less than LEAF_REDO_MIN."""
+    whose interior problem is not definite by the factorisation of B.  None where
+    all leaves are to be factored that way."""
     ops = pde.condensed_ops(device, dtype)
     if ops is None:
         return None
@@ -252,6 +269,9 @@ def _leaf_condensed(pde, full_ops, dtype, device, clist, coef_ops, src, nsrc) ->
     ni = n - nb
     rdt = real_dtype(dtype)
     coeffs = torch.stack([to_device(a, device, rdt) for _, a in clist]).contiguous()
+    indefinite = _indefinite_leaves(pde, coeffs, clist)
+    if _too_many(np.count_nonzero(indefinite), nl):
+        return None
 
     def empty(*shape, dt=dtype):
         return torch.empty(shape, dtype=dt, device=device)
@@ -273,9 +293,11 @@ def _leaf_condensed(pde, full_ops, dtype, device, clist, coef_ops, src, nsrc) ->
     check(rc, h, "hps_leaf_condensed")
     res = LeafResult(Y, T, v, hv, slu, sperm, sdinv, info, HPS_KIND_ITI, None, nb,
                      Condensed(alu, aperm, adinv, X, ops["GQ"][:nb]))
+    if indefinite.any():
+        info.masked_fill_(torch.as_tensor(indefinite).to(device), -1)
     if bool((info < 0).any()):
         idx = (info < 0).nonzero().flatten()
-        if nl < LEAF_REDO_MIN or 2 * idx.numel() > nl:
+        if _too_many(idx.numel(), nl):
             return None
         sub = _leaf_direct(pde, full_ops, HPS_KIND_ITI, dtype, device, clist, coef_ops, coeffs[:, idx].to(dtype).contiguous(),
                            None if src is None else src[idx], nsrc)

@@ -125,8 +125,12 @@ struct LuStage {
   int c0 = 0, nc = 0, c_step = 0;
   LuGroup g[LUB_MAX_CNT];
 };
+// largest multiplier that an elimination without row exchanges accepts (the
+// leaf and merge matrices of the HPS tree stay below 4)
+constexpr double LU_NOPIV_BOUND = 64.0;
 struct LuPlan {
   int n = 0, nstage = 0;
+  double bound = LU_NOPIV_BOUND;  // largest multiplier
   int nbmax = LUB_NB;  // widest block
   LuStage st[LUB_MAX_STAGES];
 };
@@ -234,7 +238,7 @@ size_t lub_scratch_bytes(const LuPlan& p, int batch);
 // A = L U in natural order, in place (batch matrices, row stride lda, batch
 // stride sA); perm becomes the identity, dinv as getrf_ws's, inv the inverses
 // of every block's L and U (lub_inv_elems), tmp lub_tmp_elems elements.
-// info[b] = -1 where a multiplier exceeds 64 or a pivot is zero, not finite or
+// info[b] = -1 where a multiplier exceeds the plan's bound or a pivot is zero, not finite or
 // without a normal reciprocal (the matrix then needs pivoting), else 0.
 template <typename T>
 hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* perm, T* dinv, T* inv, T* tmp,

@@ -15,11 +15,16 @@
 // interleaved array read as real, without a copy.
 //
 // A_ii is the leaf's Dirichlet problem, singular where k^2 is one of its
-// eigenvalues (leaf side h with k h >= sqrt(2) pi): X_b, which extends boundary
-// values into the leaf and is of size 1 otherwise, then grows without bound.
-// A leaf with an entry of X_b above LEAF_EXT_BOUND (or not finite, or with a
-// rejected factorisation) gets info = -1, and the caller takes the
-// factorisation of B for it.
+// eigenvalues (leaf side h with k h >= sqrt(2) pi) and indefinite above the
+// first.  While it is definite, its multipliers stay below 2.2, those of S
+// mostly below 3 and the entries of X_b, which extend boundary values into the
+// leaf, below 1.2, and T is as exact as through the factorisation of B:
+// error ratio 0.4 to 1.1 at p = 8, 11 and 16 up to k h = 4.2.  Past the first
+// eigenvalue elimination without row exchanges loses up to two digits, often
+// with X_b still of size 1 (p = 16: ratio 100 at k h = 4.5, multipliers of 20).  A
+// leaf that passes one of the bounds below (or is not finite) gets info = -1, and
+// the caller takes the factorisation of B for it: with them the ratio stays below
+// 1.5 also for strong advection and small eta, where S is hard to eliminate.
 //
 // Measured: leaf stage at p = 16, L = 7 (16384 leaves, complex128) 57 ms by the
 // LU of B, 33 ms condensed; Helmholtz build + solve there 159 / 135 ms, its
@@ -29,7 +34,9 @@
 
 namespace hps {
 
-constexpr double LEAF_EXT_BOUND = 16.0;
+constexpr double LEAF_EXT_BOUND = 2.0;     // entries of X_b
+constexpr double LEAF_INNER_BOUND = 4.0;   // multipliers of A_ii
+constexpr double LEAF_BORDER_BOUND = 10.0;  // multipliers of S
 
 // S = G_b - R[:nb, :nb], RB = [P | -R[:nb, nb:]], Z = Q_b - R[nb:, :nb],
 // h = R[nb:, nb:]; R (nb + nq, nb + 2 nsrc) real, the sources' columns (re, im)
@@ -125,7 +132,9 @@ static int leaf_condensed_t(hps_handle_t h, int nl_all, int n, int nb, int nq, i
   const int ni = n - nb, wr = nb + 2 * nsrc, wb = nq + nsrc;
   const CondensedWs o = condensed_ws(sizeof(R), nl_all, n, nb, nq, nsrc);
   const int m = nl_all < LEAF_CHUNK ? nl_all : LEAF_CHUNK;  // every chunk takes the first one's plan
-  const LuPlan pa = lu_plan_dense(ni, wr, m), ps = lu_plan_dense(nb, wb, m);
+  LuPlan pa = lu_plan_dense(ni, wr, m), ps = lu_plan_dense(nb, wb, m);
+  pa.bound = LEAF_INNER_BOUND;
+  ps.bound = LEAF_BORDER_BOUND;
   CoefOps co;
   for (int i = 0; i < 16; ++i) co.op[i] = i < ncoef ? coef_ops[i] : 0;
   {

@@ -42,10 +42,6 @@ namespace hps {
 #endif
 
 constexpr int LU_NB = 32;
-// largest multiplier an unpivoted register panel accepts (the leaf and merge
-// matrices of the HPS tree stay below 2)
-constexpr double LU_NOPIV_BOUND = 64.0;
-
 // a pivot that an unpivoted panel accepts, by its magnitude: finite, and with a
 // reciprocal that is a normal number (a zero, infinite, NaN or subnormal pivot
 // is none, nor one within four of the largest value)
@@ -764,7 +760,8 @@ __device__ __forceinline__ void panel_steps(std::integer_sequence<int, J...>, T 
 template <typename T, int RPT, int THREADS, bool NOPIV = false>
 __global__ __launch_bounds__(THREADS) void getrf_panel_rows_kernel(int n, T* A, long lda, long sA, int k, int nb,
                                                                    int* ipiv, int* info, T* dinv, int* swtab,
-                                                                   int nin, long sA2) {
+                                                                   int nin, long sA2,
+                                                                   typename real_of<T>::type bound) {
   using R = typename real_of<T>::type;
   __shared__ PanelLDS<T, THREADS / 64> sh;
   __shared__ T Dblk[LU_NB][LU_NB + 1];
@@ -794,7 +791,7 @@ __global__ __launch_bounds__(THREADS) void getrf_panel_rows_kernel(int n, T* A, 
                                             lmax);
   if constexpr (NOPIV) {
     // stability check of the natural-order elimination: a multiplier above
-    // LU_NOPIV_BOUND (or not finite) or a pivot that is not usable (the last
+    // `bound` (or not finite) or a pivot that is not usable (the last
     // one has no multipliers) marks the matrix with info = -1, and the caller
     // refactors with partial pivoting
     __shared__ R wmax[THREADS / 64];
@@ -811,7 +808,7 @@ __global__ __launch_bounds__(THREADS) void getrf_panel_rows_kernel(int n, T* A, 
       for (int w = 1; w < THREADS / 64; ++w) mx = (wmax[w] > mx || wmax[w] != wmax[w]) ? wmax[w] : mx;
       // a zero pivot in the natural order (info > 0) is no verdict on the
       // matrix either: pivoting decides
-      if (!(mx <= R(LU_NOPIV_BOUND)) || !usable || info[0] > 0) info[0] = -1;
+      if (!(mx <= bound) || !usable || info[0] > 0) info[0] = -1;
     }
   }
   // net row permutation of the panel: every row whose position changed
@@ -1153,7 +1150,7 @@ static int rows_panel_max() {
 // (dinv) and the identity pivots.  The rows are independent: grid
 // (ceil((n - k - nb) / NOPIV_ROWS) + U12 chunks, batch).
 //
-// A matrix with a multiplier above LU_NOPIV_BOUND or a pivot that is not usable
+// A matrix with a multiplier above `bound` or a pivot that is not usable
 // (pivot_usable) gets info = -1 (the caller refactors with pivoting).
 //
 // Bound by the serial chain of 32 steps (publish, barrier, read, reciprocal,
@@ -1231,11 +1228,12 @@ __device__ __forceinline__ void mma_step(T a, T b, typename Mfma<typename real_o
 template <typename T>
 __global__ __launch_bounds__(256) void getrf_panel_nopiv_kernel(int n, T* A, long lda, long sA, int k, int nb,
                                                                 int* ipiv, T* dinv, int* arrivals, int* info,
-                                                                int row_wgs, int u12_end, int nin, long sA2) {
+                                                                int row_wgs, int u12_end, int nin, long sA2,
+                                                                typename real_of<T>::type bound) {
   using R = typename real_of<T>::type;
   using M = Mfma<R>;
   using acc_t = typename M::acc_t;
-  constexpr R BOUND2 = R(LU_NOPIV_BOUND * LU_NOPIV_BOUND);
+  const R bound2 = bound * bound;
   __shared__ T D[LU_NB][LU_NB + 1];
   __shared__ T P[LU_NB][LU_NB + 1];  // packed inverse
   __shared__ T prow[2][LU_NB], pcol[2][LU_NB];
@@ -1328,7 +1326,7 @@ __global__ __launch_bounds__(256) void getrf_panel_nopiv_kernel(int n, T* A, lon
         ok = ok && pivot_usable(s_abs1(piv));
         if (r > j) {
           const T l = s_mul(xr, inv);
-          ok = ok && s_mod2(l) <= BOUND2;
+          ok = ok && s_mod2(l) <= bound2;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             if (i < jq) z[i] = s_fnms(z[i], l, pr[i]);
@@ -1389,7 +1387,7 @@ __global__ __launch_bounds__(256) void getrf_panel_nopiv_kernel(int n, T* A, lon
         const int r = m0 + M::out_row(lk, i), c = 16 * t + li;
         if (r < n && c < nb) {
           const T v = make_val<T>(re[t][i], is_cplx<T>::value ? im[t][i] : R(0));
-          ok = ok && s_mod2(v) <= BOUND2;
+          ok = ok && s_mod2(v) <= bound2;
           Ab[(long)r * lda + k + c] = v;
         }
       }
@@ -1416,6 +1414,7 @@ static hipError_t launch_panel(int n, T* A, long lda, long sA, int k, int nb, in
                                int* swtab, int* cand, int batch, hipStream_t s, bool* swapped,
                                bool unpivoted = false) {
   const int m = n - k;
+  const auto bound = typename real_of<T>::type(LU_NOPIV_BOUND);
   const double pf = flop_mult<T>() * batch * ((double)m * nb * nb - (double)nb * nb * nb / 3.0);
   *swapped = m <= rows_panel_max<T>();
   if (unpivoted && m <= rows_panel_max<T>()) {
@@ -1424,16 +1423,16 @@ static hipError_t launch_panel(int n, T* A, long lda, long sA, int k, int nb, in
     prof::Scope ps(s, nm_rows.c_str(), pf, 2.0 * sizeof(T) * (double)m * nb * batch);
     if (m <= 128)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 128, true>), dim3(batch), dim3(128), 0, s, n, A, lda, sA, k,
-                         nb, ipiv, info, dinv, swtab, 1, 0L);
+                         nb, ipiv, info, dinv, swtab, 1, 0L, bound);
     else if (m <= 256)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 256, true>), dim3(batch), dim3(256), 0, s, n, A, lda, sA, k,
-                         nb, ipiv, info, dinv, swtab, 1, 0L);
+                         nb, ipiv, info, dinv, swtab, 1, 0L, bound);
     else if (m <= 512)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 512, true>), dim3(batch), dim3(512), 0, s, n, A, lda, sA, k,
-                         nb, ipiv, info, dinv, swtab, 1, 0L);
+                         nb, ipiv, info, dinv, swtab, 1, 0L, bound);
     else if constexpr (sizeof(T) < 16)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 1024, true>), dim3(batch), dim3(1024), 0, s, n, A, lda, sA,
-                         k, nb, ipiv, info, dinv, swtab, 1, 0L);
+                         k, nb, ipiv, info, dinv, swtab, 1, 0L, bound);
     else
       return hipErrorInvalidValue;  // not reached: rows_panel_max<c128>() is 512
     return hipGetLastError();
@@ -1444,16 +1443,16 @@ static hipError_t launch_panel(int n, T* A, long lda, long sA, int k, int nb, in
     // short panels in smaller workgroups: more of them share a CU
     if (m <= 128)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 128>), dim3(batch), dim3(128), 0, s, n, A, lda, sA, k, nb,
-                         ipiv, info, dinv, swtab, 1, 0L);
+                         ipiv, info, dinv, swtab, 1, 0L, bound);
     else if (m <= 256)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 256>), dim3(batch), dim3(256), 0, s, n, A, lda, sA, k, nb,
-                         ipiv, info, dinv, swtab, 1, 0L);
+                         ipiv, info, dinv, swtab, 1, 0L, bound);
     else if (m <= 512)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 512>), dim3(batch), dim3(512), 0, s, n, A, lda, sA, k, nb,
-                         ipiv, info, dinv, swtab, 1, 0L);
+                         ipiv, info, dinv, swtab, 1, 0L, bound);
     else if constexpr (sizeof(T) < 16)
       hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 1024>), dim3(batch), dim3(1024), 0, s, n, A, lda, sA, k, nb,
-                         ipiv, info, dinv, swtab, 1, 0L);
+                         ipiv, info, dinv, swtab, 1, 0L, bound);
     else
       return hipErrorInvalidValue;  // not reached: rows_panel_max<c128>() is 512
     return hipGetLastError();

@@ -165,9 +165,9 @@ static __global__ __launch_bounds__(256) void lu_blocks_init_kernel(int n, int b
 // are multipliers
 template <typename T, bool CHECK>
 __global__ __launch_bounds__(256) void panel_back_kernel(int rows, int cols, const T* tmp, long ldt, long sT, T* A,
-                                                         long lda, long sA, int nin, long sA2, int* info,
-                                                         int batch) {
-  constexpr auto BOUND2 = typename real_of<T>::type(LU_NOPIV_BOUND * LU_NOPIV_BOUND);
+                                                         long lda, long sA, int nin, long sA2,
+                                                         typename real_of<T>::type bound, int* info, int batch) {
+  const auto bound2 = bound * bound;
   const int total = rows * cols;
   for (int b = blockIdx.y; b < batch; b += gridDim.y) {
     const T* t = tmp + (long)b * sT;
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void panel_back_kernel(int rows, int cols, con
       const int r = idx / cols, c = idx - r * cols;
       const T v = t[(long)r * ldt + c];
       a[(long)r * lda + c] = v;
-      if (CHECK) ok = ok && s_mod2(v) <= BOUND2;
+      if (CHECK) ok = ok && s_mod2(v) <= bound2;
     }
     if (!ok) info[b / nin] = -1;
   }
@@ -186,15 +186,16 @@ __global__ __launch_bounds__(256) void panel_back_kernel(int rows, int cols, con
 // info of the matrices whose multipliers (rows x cols at A) pass the bound
 template <typename T>
 __global__ __launch_bounds__(256) void panel_check_kernel(int rows, int cols, const T* A, long lda, long sA, int nin,
-                                                          long sA2, int* info, int batch) {
-  constexpr auto BOUND2 = typename real_of<T>::type(LU_NOPIV_BOUND * LU_NOPIV_BOUND);
+                                                          long sA2, typename real_of<T>::type bound, int* info,
+                                                          int batch) {
+  const auto bound2 = bound * bound;
   const int total = rows * cols;
   for (int b = blockIdx.y; b < batch; b += gridDim.y) {
     const T* a = A + batch_offset(b, nin, sA, sA2);
     bool ok = true;
     for (int idx = blockIdx.x * 256 + threadIdx.x; idx < total; idx += gridDim.x * 256) {
       const int r = idx / cols, c = idx - r * cols;
-      ok = ok && s_mod2(a[(long)r * lda + c]) <= BOUND2;
+      ok = ok && s_mod2(a[(long)r * lda + c]) <= bound2;
     }
     if (!ok) info[b / nin] = -1;
   }
@@ -265,8 +266,8 @@ static hipError_t mul(int M, int N, int K, double alpha, Parts<T> A, Parts<T> B,
 // LU of the nb x nb diagonal blocks (nb <= 128) of nin parts of batch matrices;
 // db receives the packed 32 x 32 inverses, part by part.
 template <typename T>
-static hipError_t diag_block_lu(int nb, Parts<T> A, T* db, int* arrivals, int* scratch, int* info, int nin, int batch,
-                                hipStream_t s) {
+static hipError_t diag_block_lu(int nb, Parts<T> A, T* db, int* arrivals, int* scratch, int* info,
+                                typename real_of<T>::type bound, int nin, int batch, hipStream_t s) {
   const int parts = nin * batch;
   int* ipiv = scratch;  // the panel kernels' pivots and swap tables, not used here
   int* swtab = ipiv + (long)parts * nb;
@@ -281,14 +282,14 @@ static hipError_t diag_block_lu(int nb, Parts<T> A, T* db, int* arrivals, int* s
       const int row_wgs = m - kb > 0 ? ceil_div(m - kb, NOPIV_ROWS) : 1;
       const int u12_wgs = ceil_div(m - kb, LU_NB);
       hipLaunchKernelGGL((getrf_panel_nopiv_kernel<T>), dim3(row_wgs + u12_wgs, parts), dim3(256), 0, s, nb, a, A.ld,
-                         A.s, k, kb, ipiv, db, arrivals, info, row_wgs, nb, nin, A.s2);
+                         A.s, k, kb, ipiv, db, arrivals, info, row_wgs, nb, nin, A.s2, bound);
       HPS_LU_CHECK(hipGetLastError());
     } else {
       {
         static const std::string nm_rows = std::string("getrf_panel_rows_nopiv<") + tname<T>() + ">";
         prof::Scope ps(s, nm_rows.c_str(), pf, 2.0 * sizeof(T) * (double)m * kb * parts);
         hipLaunchKernelGGL((getrf_panel_rows_kernel<T, 1, 128, true>), dim3(parts), dim3(128), 0, s, nb, a, A.ld, A.s,
-                           k, kb, ipiv, info, db, swtab, nin, A.s2);
+                           k, kb, ipiv, info, db, swtab, nin, A.s2, bound);
         HPS_LU_CHECK(hipGetLastError());
       }
       if (m - kb > 0) {
@@ -308,6 +309,7 @@ template <typename T>
 hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* perm, T* dinv, T* inv, T* tmp,
                             int* scratch, int* info, int batch, hipStream_t s) {
   const int n = plan.n;
+  const auto bound = typename real_of<T>::type(plan.bound);
   if (n <= 0 || batch <= 0) return hipSuccess;
   int cnt = 1;
   for (int i = 0; i < plan.nstage; ++i) cnt = cnt > plan.st[i].cnt ? cnt : plan.st[i].cnt;
@@ -340,7 +342,7 @@ hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* pe
       T* akk = a0 + (long)k * (lda + 1);
       T* li = ginv + (long)blk * 2 * nb0 * nb0;
       const T* ui = li + nb0 * nb0;
-      HPS_LU_CHECK(diag_block_lu<T>(nb, {akk, lda, sA, gs}, db, arrivals, scratch, info, nin, batch, s));
+      HPS_LU_CHECK(diag_block_lu<T>(nb, {akk, lda, sA, gs}, db, arrivals, scratch, info, bound, nin, batch, s));
       {
         static const std::string nm = std::string("block_inverse<") + tname<T>() + ">";
         prof::Scope ps(s, nm.c_str(), flop_mult<T>() * parts * 2.0 / 3.0 * (double)nb * nb * nb,
@@ -379,7 +381,7 @@ hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* pe
           static const std::string nmk = std::string("panel_check<") + tname<T>() + ">";
           prof::Scope ps(s, nmk.c_str(), 0.0, sizeof(T) * (double)rows * nb * parts);
           hipLaunchKernelGGL((panel_check_kernel<T>), bgrid, dim3(256), 0, s, rows, nb,
-                             seg == 0 ? akk + (long)nb * lda : arc, lda, sA, nin, seg == 0 ? gs : gc, info, parts);
+                             seg == 0 ? akk + (long)nb * lda : arc, lda, sA, nin, seg == 0 ? gs : gc, bound, info, parts);
           HPS_LU_CHECK(hipGetLastError());
         }
       } else {
@@ -393,10 +395,10 @@ hipError_t lu_blocks_factor(const LuPlan& plan, T* A, long lda, long sA, int* pe
           prof::Scope ps(s, nmc.c_str(), 0.0, 2.0 * sizeof(T) * (double)count * nb * parts);
           if (rows)
             hipLaunchKernelGGL((panel_back_kernel<T, true>), bgrid, dim3(256), 0, s, count, nb,
-                               pan + (long)first_ * nb, (long)nb, sP, dst, lda, sA, nin, step, info, parts);
+                               pan + (long)first_ * nb, (long)nb, sP, dst, lda, sA, nin, step, bound, info, parts);
           else
             hipLaunchKernelGGL((panel_back_kernel<T, false>), bgrid, dim3(256), 0, s, nb, count, pan + first_, (long)m,
-                               sP, dst, lda, sA, nin, step, info, parts);
+                               sP, dst, lda, sA, nin, step, bound, info, parts);
           return hipGetLastError();
         };
         HPS_LU_CHECK(back(true, 0, nin == 1 ? m : below, akk + (long)nb * lda, gs));
