@@ -126,6 +126,14 @@ int hps_leaf_condensed(hps_handle_t h, int dtype, int nl, int n, int nb, int nq,
                        void* alu, int* aperm, void* adinv, void* X, void* slu, int* sperm, void* sdinv, int* info,
                        void* ws, size_t ws_bytes);
 
+/* info[l] = -1 for the leaves with zeroth / (xx + yy) above limit, or not a
+ * number, at one of their n points (zeroth, xx, yy (nl, n) real coefficient
+ * fields of the identity, D_xx and D_yy; yy NULL: xx alone); other entries stay.
+ * With limit a little below (pi / side)^2 these are the leaves whose interior
+ * problem may not be definite, for which hps_leaf_condensed is not exact. */
+int hps_mark_indefinite(hps_handle_t h, int dtype, int nl, int n, const void* zeroth, const void* xx, const void* yy,
+                        double limit, int* info);
+
 /* ---- merge stage (one tree level) ------------------------------------------
  * nm merges of nc children each (4 in 2D, 8 in 3D); children's maps
  * T_in (nm*nc, nec, nec) and data h_in (nm*nc, nec, nsrc).

@@ -51,6 +51,7 @@ SIGNATURES = {
     ),
     "hps_leaf_condensed_workspace": (_S, [_I] * 6),
     "hps_leaf_condensed": (_I, [_P] + [_I] * 7 + [_P] * 21 + [_S]),
+    "hps_mark_indefinite": (_I, [_P, _I, _I, _I, _P, _P, _P, _D, _P]),
     "hps_set_merge_pivoting": (_I, [_P, _I]),
     "hps_set_merge_dissection": (_I, [_P, _I, _P, _P]),
     "hps_set_leaf_pivoting": (_I, [_P, _I]),

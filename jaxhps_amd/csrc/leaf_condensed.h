@@ -84,6 +84,21 @@ __global__ __launch_bounds__(256) void extension_check_kernel(int ni, int nb, co
   if (!ok) info[l] = -1;
 }
 
+// info[l] = -1 where zeroth / (xx + yy) of the leaf's n points passes the limit
+// or is not a number (yy may be null)
+template <typename R>
+__global__ __launch_bounds__(256) void mark_indefinite_kernel(int n, const R* zeroth, const R* xx, const R* yy,
+                                                              R limit, int* info, int nl) {
+  for (int l = blockIdx.x; l < nl; l += gridDim.x) {
+    bool ok = true;
+    for (int i = threadIdx.x; i < n; i += 256) {
+      const long at = (long)l * n + i;
+      ok = ok && zeroth[at] / (yy ? xx[at] + yy[at] : xx[at]) <= limit;
+    }
+    if (!ok) info[l] = -1;  // every writer writes the same value
+  }
+}
+
 }  // namespace hps
 
 struct CondensedWs {
@@ -229,6 +244,23 @@ static int leaf_condensed_t(hps_handle_t h, int nl_all, int n, int nb, int nq, i
       HPS_CHECK_HIP(h, gemm_call<C>(s, nq, nsrc, nb, 1.0, Z, nb, (long)nq * nb, RB + nq, wb, sRB, 1.0, hh, nsrc,
                                     (long)nq * nsrc, hh, nsrc, (long)nq * nsrc, nl));
   }
+  return HPS_OK;
+}
+
+int hps_mark_indefinite(hps_handle_t h, int dtype, int nl, int n, const void* zeroth, const void* xx, const void* yy,
+                        double limit, int* info) {
+  if (!h) return HPS_ERR_ARG;
+  HPS_ARG(h, dtype == HPS_F64 || dtype == HPS_F32, "real coefficients required");
+  HPS_ARG(h, nl > 0 && n > 0, "bad leaf sizes");
+  HPS_ARG(h, zeroth && xx && info, "null pointer");
+  const dim3 grid(nl < 65535 ? nl : 65535);
+  if (dtype == HPS_F64)
+    hipLaunchKernelGGL((mark_indefinite_kernel<double>), grid, dim3(256), 0, h->stream, n, (const double*)zeroth,
+                       (const double*)xx, (const double*)yy, limit, info, nl);
+  else
+    hipLaunchKernelGGL((mark_indefinite_kernel<float>), grid, dim3(256), 0, h->stream, n, (const float*)zeroth,
+                       (const float*)xx, (const float*)yy, (float)limit, info, nl);
+  HPS_CHECK_HIP(h, hipGetLastError());
   return HPS_OK;
 }
 

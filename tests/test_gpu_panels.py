@@ -418,6 +418,23 @@ def test_condensed_leaves_lose_no_precision(gpu, monkeypatch, kh, found_by):
     assert err[0] <= 2.0**2 * err[1], np.sqrt(err / 16)
 
 
+def test_definiteness_is_read_before_or_after_alike(gpu, monkeypatch):
+    """The coefficients' estimate gives one result whether it is read before the
+    condensed stage (eta as large as the wavenumber) or after it."""
+    from jaxhps_amd import _stages
+    from jaxhps_amd._stages import HPS_KIND_ITI, leaf_solve
+
+    print("definiteness read before or after", flush=True)
+    for k2_extra in (False, True):
+        res = []
+        for first in (0.0, float("inf")):
+            monkeypatch.setattr(_stages, "LEAF_LOOK_FIRST", first)
+            pde = (_resonant_leaf if k2_extra else lambda *a: _iti_leaves(*a, 2000.0))(gpu, 8, 4)[0]
+            res.append(leaf_solve(pde, HPS_KIND_ITI, torch.complex128, gpu, nsrc_zero=True))
+        assert (res[0].condensed is None) == (res[1].condensed is None) == (not k2_extra)
+        assert torch.equal(res[0].Y, res[1].Y) and torch.equal(res[0].T, res[1].T)
+
+
 def test_condensed_build_leaves_the_complex_operators_alone(gpu):
     """A build whose leaves are condensed uploads the real differentiation
     operators, not a complex set beside them (a problem object per coefficient
@@ -429,6 +446,32 @@ def test_condensed_build_leaves_the_complex_operators_alone(gpu):
     jh.build_solver(pde)
     assert pde._factors["leaf"].condensed is not None
     assert not {"diffops", "G"} & set(pde.device_ops(gpu, torch.complex128))
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n,nl", [(9, 1), (256, 300), (400, 70000)])
+def test_mark_indefinite(gpu, dtype, n, nl):
+    """Leaves with a point above the limit, or a NaN, are marked, whichever
+    point it is; other entries of info stay, with one second-order field or two."""
+    from jaxhps_amd import _lib
+
+    print(f"mark indefinite {dtype} n={n} nl={nl}", flush=True)
+    lib, h = _lib.load_library(), _lib.handle()
+    g = torch.Generator(device=gpu).manual_seed(n)
+    z = 3.9 * torch.rand(nl, n, generator=g, device=gpu, dtype=dtype)
+    xx, yy = torch.full_like(z, 0.5), torch.full_like(z, 1.5)
+    want = torch.zeros(nl, dtype=torch.int32, device=gpu)
+    for leaf, point, value in ((0, n - 1, 4.5), (nl // 2, 0, float("nan")), (nl - 1, n // 2, float("inf"))):
+        z[leaf, point] = value
+        want[leaf] = -1
+    want[nl // 3] = 7 if want[nl // 3] == 0 else -1
+    for fields, limit in (((xx, yy), 2.0), ((2 * xx, None), 4.0)):
+        info = torch.zeros_like(want)
+        info[nl // 3] = 7
+        rc = lib.hps_mark_indefinite(h, _lib.dtype_code(dtype), nl, n, _lib.ptr(z), _lib.ptr(fields[0]),
+                                     _lib.ptr(fields[1]), limit, _lib.ptr(info))
+        _lib.check(rc, h, "hps_mark_indefinite")
+        assert torch.equal(info, want)
 
 
 def test_condensed_leaves_give_way(gpu):
