@@ -419,8 +419,9 @@ def merge_factors_stable(F_lu, bound=64.0):
     """Device bool: the natural-order (unpivoted) LU factors of a merge level
     are usable -- every entry finite, no zero pivot, every multiplier at most
     `bound` in magnitude (partial pivoting would guarantee 1; the merge
-    matrices of uniform trees give values below 4).  The panel kernels report
-    the same through info; this reads factors from anywhere."""
+    matrices of uniform trees give values below 4).  The stages themselves go
+    by the kernels' own checks (info); this is for factors in hand, whoever
+    formed them."""
     a = F_lu.abs()
     finite = torch.isfinite(a.amax(dim=(-2, -1)))
     mult = torch.tril(a, -1).amax(dim=(-2, -1))

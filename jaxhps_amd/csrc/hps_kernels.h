@@ -78,7 +78,7 @@ template <typename T>
 hipError_t getrs_inplace(int n, int nrhs, const T* LU, long lda, long sA, const T* dinv, T* X, long ldx, long sX,
                          int batch, hipStream_t s);
 
-// few-column block size and the wide column block of large pivoted matrices
+// smallest matrix that pivoted factorisations cut into column blocks of 512
 constexpr int LU_WIDE_MIN = 3072;
 
 // Few-column solves (at most 16 columns) of matrices too large for one

@@ -26,9 +26,9 @@
 // the caller takes the factorisation of B for it: with them the ratio stays below
 // 1.5 also for strong advection and small eta, where S is hard to eliminate.
 //
-// Measured: leaf stage at p = 16, L = 7 (16384 leaves, complex128) 57 ms by the
-// LU of B, 33 ms condensed; Helmholtz build + solve there 159 / 135 ms, its
-// gradient at L = 6 49 / 37 ms.  Bound by the real products (12.5 ms, tiles of
+// Measured, by the LU of B / condensed: leaf stage at p = 16, L = 7 (16384
+// leaves) 55 / 31 ms in complex128, 32 / 19 ms in complex64; Helmholtz build +
+// solve there 158 / 135 and, mixed, 107 / 88 ms; gradient at L = 6 43 / 37 ms.  Bound by the real products (12.5 ms, tiles of
 // 64 x 64 on 60 .. 196 rows) and the passes between them.
 #pragma once
 

@@ -1,4 +1,5 @@
-// Batched dense LU with partial pivoting and the matching solve, gfx950.
+// Batched dense LU with partial pivoting and the matching solve, gfx950
+// (natural-order LU by blocks: lu_blocks.h).
 //
 // Factor format: P A = L U stored LAPACK-style in A, plus
 //   perm[b][i]        row of A that became row i of P A,
@@ -1161,9 +1162,9 @@ static int rows_panel_max() {
 // also leaves no separate inversion and no check of the factors afterwards, 24 / 17 / 19 us.
 // ---------------------------------------------------------------------------
 // 1 / a from the hardware's reciprocal estimate and Newton steps (to the last
-// bit or the one before, for the a that pivot_usable accepts).  Complex a is first scaled by the power of
-// two that brings its larger part to [0.5, 1), so |a|^2 neither overflows nor
-// vanishes.  The reciprocal is on the panel's serial chain: half of a division.
+// bit or the one before, for the a that pivot_usable accepts).  Complex a is
+// first scaled by the power of two that brings its larger part to [0.5, 1), so
+// |a|^2 neither overflows nor vanishes.  The reciprocal is on the panel's serial chain: half of a division.
 __device__ __forceinline__ double s_inv_fast(double a) {
   double r = __builtin_amdgcn_rcp(a);
   r = fma(fma(-a, r, 1.0), r, r);

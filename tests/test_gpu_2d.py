@@ -327,7 +327,7 @@ def test_unpivoted_merge_falls_back_to_pivoting(gpu):
     from jaxhps_amd._tables import quad_merge_tables
 
     print("unpivoted merge fallback", flush=True)
-    m = 280  # 1120 interface unknowns: taller than the register panels, so unpivoted
+    m = 280  # 1120 interface unknowns: several diagonal blocks
     ne = 4 * m
     rng = np.random.default_rng(21)
     T = 2.0 * np.eye(ne) + rng.standard_normal((4, ne, ne)) / np.sqrt(ne)

@@ -185,9 +185,8 @@ def test_getrs_conjt_solves_adjoint_system(gpu, dtype, n, nrhs, batch):
                                              ("dtn", torch.float32, 768, 1)])
 def test_block_inverse_solves_match_fp64_merge(gpu, kind, dtype, m, nm):
     """A merge level whose factored matrix has 3072 unknowns in low precision
-    takes its many-column solve through the inverses of the 512 x 512
-    diagonal blocks; S, T, g_tilde and h agree with the same merge in double
-    precision (the standard blocked solve) to the low precision's accuracy."""
+    (with pivoting, in column blocks of 512): S, T, g_tilde and h agree with
+    the same merge in double precision to the low precision's accuracy."""
     from jaxhps_amd._stages import merge_level
     from jaxhps_amd._tables import quad_merge_tables
 
@@ -215,12 +214,11 @@ def test_block_inverse_solves_match_fp64_merge(gpu, kind, dtype, m, nm):
 
 
 def test_unpivoted_panels_of_many_matrices(gpu):
-    """96 complex64 interface matrices of 1200 unknowns: the leading panels
-    (taller than 1024 rows) unpivoted, the rest partially pivoted, with more
-    unpivoted-panel workgroups than the GPU holds at once, so the workgroups of
-    one matrix do not all run together.  S, T, g_tilde and h equal the
-    pivoted merge's (the factored diagonal block is written only after every
-    workgroup of its matrix has read the original)."""
+    """96 complex64 interface matrices of 1200 unknowns, the most whose diagonal
+    blocks take the unpivoted panel kernel together: several blocks, each with
+    workgroups for its rows and columns beside the one that writes the factors.
+    S, T, g_tilde and h equal the pivoted merge's (the factored diagonal block
+    is written only after every workgroup of its matrix has read the original)."""
     from jaxhps_amd._stages import merge_factors_stable, merge_level
     from jaxhps_amd._tables import quad_merge_tables
 
@@ -245,11 +243,10 @@ def test_unpivoted_panels_of_many_matrices(gpu):
 @pytest.mark.parametrize("kind,dtype", [("iti", torch.complex128), ("iti", torch.complex64),
                                         ("dtn", torch.float64), ("dtn", torch.float32)])
 def test_unpivoted_tall_merge_matches_pivoted(gpu, kind, dtype):
-    """A merge level whose interface matrix is tall enough for the unpivoted
-    panel kernel (1792 unknowns, children with 448 Gauss nodes per side) on
-    well-conditioned synthetic maps: the unpivoted factors pass the check
-    and S, T and g_tilde equal the partially pivoted merge's (a single
-    matrix: every panel unpivoted)."""
+    """A merge level with an interface matrix of 1792 unknowns (children with
+    448 Gauss nodes per side; a single matrix, eliminated by 128-wide blocks
+    in natural order) on well-conditioned synthetic maps: the unpivoted factors
+    pass the check and S, T and g_tilde equal the partially pivoted merge's."""
     from jaxhps_amd._stages import merge_factors_stable, merge_level
     from jaxhps_amd._tables import quad_merge_tables
 
