@@ -178,7 +178,7 @@ int hps_mark_indefinite(hps_handle_t h, int dtype, int nl, int n, const void* ze
  * stably in their natural order (pivot growth ~1, multipliers below 4 on the
  * Helmholtz and variable-coefficient workloads), while pivoted panels are
  * latency-bound.  With 0, the panel kernels check each matrix and set
- * info = -1 when a multiplier exceeds 64 or a pivot is not usable (zero, not
+ * info = -1 when a multiplier exceeds 16 (ItI: 64) or a pivot is not usable (zero, not
  * finite, or without a normal reciprocal); the caller refactors with pivoting
  * then.  The reference factors
  * with LAPACK's pivoted LU inside jnp.linalg.inv
@@ -200,7 +200,7 @@ enum { HPS_DISSECT_NONE = 0, HPS_DISSECT_QUAD = 1, HPS_DISSECT_OCT = 2 };
 int hps_set_merge_dissection(hps_handle_t h, int dissect, const int* ext_by_child, const int* ext_pos);
 /* Pivoting of hps_leaf_solve's factorisation on this handle: 1 (default) =
  * partial pivoting; 0 = natural order, every panel checked in the kernel:
- * a leaf whose largest multiplier exceeds 64 (or is not finite) gets
+ * a leaf whose largest multiplier exceeds 16 (ItI: 64) or is not finite gets
  * info[l] = -1, and the caller reruns the leaf stage with pivoting.  The
  * row-scaled ItI leaf matrices and the DtN interior blocks eliminate with
  * multipliers below 2 on the benchmark workloads.  The reference factors

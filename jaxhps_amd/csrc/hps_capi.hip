@@ -482,7 +482,8 @@ static int leaf_t(hps_handle_t h, int kind, int nl, int n, int nb, int nq, int n
     // natural order by blocks, the right-hand sides solved in place (X is
     // scratch), LEAF_CHUNK leaves at a time
     const int m = nl < LEAF_CHUNK ? nl : LEAF_CHUNK;
-    const LuPlan p = lu_plan_dense(nrows, w, m);
+    LuPlan p = lu_plan_dense(nrows, w, m);
+    p.bound = LU_DTN_BOUND;
     char* q = wp + align_up(getrf_scratch_bytes(nrows, nl));
     T* inv = (T*)q;
     q += align_up(lub_inv_elems(p, m) * es);
@@ -841,7 +842,8 @@ static int merge_t(hps_handle_t h, int kind, int nm, int nc, int nec, int ni, in
   // natural order: by blocks, with the handle's dissection for DtN
   const bool natural = h->merge_nopiv;
   const int dissect = !iti ? h->dissect : HPS_DISSECT_NONE;
-  const LuPlan plan = merge_plan(dissect, nfac, ne, nm);
+  LuPlan plan = merge_plan(dissect, nfac, ne, nm);
+  if (!iti) plan.bound = LU_DTN_BOUND;
   const bool by_child = natural && plan.nstage > 1;  // columns of C by child
   T* linv = natural ? (T*)take(lub_inv_elems(plan, nm) * es) : nullptr;
   T* ltmp = natural ? (T*)take(lub_tmp_elems(plan, nm) * es) : nullptr;

@@ -125,9 +125,16 @@ struct LuStage {
   int c0 = 0, nc = 0, c_step = 0;
   LuGroup g[LUB_MAX_CNT];
 };
-// largest multiplier that an elimination without row exchanges accepts (the
-// leaf and merge matrices of the HPS tree stay below 4)
+// Largest multiplier that an elimination without row exchanges accepts, and the
+// one for DtN matrices by blocks.  The matrices of definite problems stay below 8
+// (anisotropy 100, coefficient jumps of 1000, strong advection).  DtN Helmholtz
+// problems past the first eigenvalues reach any size, and the blocks' explicit
+// 64- and 128-wide inverses amplify growth: with multipliers up to 16 the
+// solution's error is up to 2.4 times that of pivoting everywhere (60 problems, p =
+// 6 .. 16), with 16 to 20 up to 6, with 44 to 55 up to 240 times.  ItI merges reach
+// 15 to 58 with eta below k / 20 and lose nothing (ratio 0.94 to 1.01, 40 problems).
 constexpr double LU_NOPIV_BOUND = 64.0;
+constexpr double LU_DTN_BOUND = 16.0;
 struct LuPlan {
   int n = 0, nstage = 0;
   double bound = LU_NOPIV_BOUND;  // largest multiplier

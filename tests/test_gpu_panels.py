@@ -295,6 +295,47 @@ def test_merges_from_several_threads(gpu):
     assert not wrong, wrong
 
 
+@pytest.mark.parametrize("p,L,k", [(12, 3, 20.0), (16, 3, 20.0), (8, 3, 12.0), (16, 2, 12.0)])
+def test_indefinite_dtn_problems_keep_their_precision(gpu, monkeypatch, p, L, k):
+    """DtN Helmholtz problems past the leaves' first eigenvalues, whose natural
+    order elimination grows: the solution's distance to the exact discrete one
+    is that of pivoting everywhere (5: twice the largest ratio that multipliers
+    up to the bound showed; 60 and 100 without it in the first two cases)."""
+    import config_oracle as co
+    import jaxhps_amd as jh
+    from jaxhps_amd import _build_solver, _lib
+    from jaxhps_amd.merge import _levels
+
+    print(f"indefinite DtN p={p} L={L} k={k}", flush=True)
+    dom = jh.Domain(p=p, q=p - 2, root=jh.DiscretizationNode2D(-1.0, 1.0, -1.0, 1.0), L=L)
+    x = dom.interior_points
+    rng = np.random.default_rng(3)
+    con = 0.2 * np.exp(-((x - np.array([0.2, -0.1])) ** 2).sum(-1) / 0.09)
+    one = np.ones(x.shape[:2])
+    kw = dict(D_xx_coefficients=one, D_yy_coefficients=one, I_coefficients=k * k * (1 - con),
+              source=rng.standard_normal(x.shape[:2]))
+    g = rng.standard_normal(dom.boundary_points.shape[0])
+    exact = co.exact_solution(dom, kw, g)
+
+    def error():
+        pde = jh.PDEProblem(dom, **kw)
+        jh.build_solver(pde)
+        return co.rel2(jh.solve(pde, g).cpu().numpy(), exact)
+
+    natural = error()
+    lib = _lib.load_library()
+
+    class Pivoting:
+        """The library with the leaves' switch left at partial pivoting."""
+
+        def __getattr__(self, name):
+            return (lambda h, v: 0) if name == "hps_set_leaf_pivoting" else getattr(lib, name)
+
+    monkeypatch.setattr(_lib, "_lib", Pivoting())
+    monkeypatch.setattr(_build_solver, "_levels", lambda *a, **kwargs: _levels(*a, **dict(kwargs, pivot=True)))
+    assert natural <= 5 * error()
+
+
 def _iti_leaves(gpu, p, L, k2, imag=0.0, extra=None):
     """An ItI problem with smooth coefficients on 4^L leaves (extra(x): a further
     zeroth-order term), and its leaf matrices B = [G; A_int] (complex128, numpy)
