@@ -130,9 +130,10 @@ struct LuStage {
 // (anisotropy 100, coefficient jumps of 1000, strong advection).  DtN Helmholtz
 // problems past the first eigenvalues reach any size, and the blocks' explicit
 // 64- and 128-wide inverses amplify growth: with multipliers up to 16 the
-// solution's error is up to 2.4 times that of pivoting everywhere (60 problems, p =
-// 6 .. 16), with 16 to 20 up to 6, with 44 to 55 up to 240 times.  ItI merges reach
-// 15 to 58 with eta below k / 20 and lose nothing (ratio 0.94 to 1.01, 40 problems).
+// solution's error is up to 3.3 times that of pivoting everywhere, with 17 to 64
+// mostly below 5, but up to 2300 times (120 problems, p = 6 .. 16; no norm of the
+// inverses tells the two apart).  ItI merges reach 15 to 58 with eta below k / 20
+// and lose nothing (ratio 0.94 to 1.01, 40 problems).
 constexpr double LU_NOPIV_BOUND = 64.0;
 constexpr double LU_DTN_BOUND = 16.0;
 struct LuPlan {

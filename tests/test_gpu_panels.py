@@ -299,8 +299,8 @@ def test_merges_from_several_threads(gpu):
 def test_indefinite_dtn_problems_keep_their_precision(gpu, monkeypatch, p, L, k):
     """DtN Helmholtz problems past the leaves' first eigenvalues, whose natural
     order elimination grows: the solution's distance to the exact discrete one
-    is that of pivoting everywhere (5: twice the largest ratio that multipliers
-    up to the bound showed; 60 and 100 without it in the first two cases)."""
+    is that of pivoting everywhere (5: the largest ratio that multipliers up to
+    the bound showed is 3.3; 60 and 100 without it in the first two cases)."""
     import config_oracle as co
     import jaxhps_amd as jh
     from jaxhps_amd import _build_solver, _lib
