@@ -169,6 +169,7 @@ def _nosource_build_solver(pde_problem, return_top_T, compute_device, dtype=None
         dtype = _compute_dtype(pde_problem, force_complex=(kind == HPS_KIND_ITI))
     with profiling.stage("leaf"):
         res = leaf_solve(pde_problem, kind, dtype, device, nsrc_zero=True)
+        pde_problem.device_ops(device, dtype)["Q"]  # uploaded here, not in the first solve for a source
     raise_on_info(res.info, "leaf stage")
     levels, _ = _merge_levels(pde_problem, res.T, None, return_top_T, dtypes)
     pde_problem.Y = cast(res.Y, store_dtype or res.Y.dtype)
